@@ -37,6 +37,7 @@
 #include "bn_core.h"
 #include "bn_internal.h"
 #include "bn_sites.h"
+#include "bn_tile.h"
 
 using namespace bn;
 
@@ -797,128 +798,438 @@ __global__ __launch_bounds__(kT) void k_st_marginals(StDims dm, const double* __
 }
 
 // ---------------------------------------------------------------------------
+// k_st_transitions: A(dt_t), Q(dt_t) of every (step, run), 2 KT^2 values each, so that the
+// recursions read them as uniform values instead of evaluating them on one lane per step.
+// ---------------------------------------------------------------------------
+template <int KT>
+__global__ __launch_bounds__(kT) void k_st_transitions(StDims dm, StHyp hy, const double* __restrict__ dt,
+                                                       double* __restrict__ aq) {
+  const int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (e >= (int64_t)dm.K * dm.T) return;
+  const int64_t k = e / dm.T;
+  double A[KT * KT], Q[KT * KT];
+  temporal_AQ<KT>(hy.ls_t[k * hy.stride], hy.var_t[k * hy.stride], dt[e], A, Q);
+  double* o = aq + e * 2 * KT * KT;
+  for (int i = 0; i < KT * KT; ++i) { o[i] = A[i]; o[KT * KT + i] = Q[i]; }
+}
+
+// ---------------------------------------------------------------------------
 // k_st_filter: one workgroup per run, sequential over T (ops.py:154-180 in whitened form).
-// Per step outputs for the smoother: U0 = P-[:, :M] (D x M), Y (M x M), w (M), H m- (M).
+// Per step, with U = P-[:, :M] L and the Cholesky factor Lm Lm' = Mm = I + L' U[:M]:
+//   W = U Lm^-T,  e = Lm^-1 (z - L' H m-),  m = m- + W e,  P = P- - W W',
+//   log N = -1/2 (e' e + M log 2pi + log det Mm - 2 ldl).
+//
+// Bound by the latency of one workgroup's chain of steps.  At M = 64, D = 128 a step has 23 k
+// cycles of FP64 matrix instructions a SIMD (64 cycles each) and four pivot chains of 3.5 k
+// cycles; it takes 61 k cycles = 25 us, against 126 us for products from L2 through LDS panels
+// with a 64-pivot sweep inverse (one run of 1000 steps: 125.6 -> 25 ms).
+// The covariance stays in registers for the whole walk: a wavefront holds the 16 x 16 tiles
+// (i, j), i <= j, of all KT x KT blocks, so the predict step, which mixes blocks elementwise,
+// touches no memory, and the tiles below the diagonal are transposes of held ones.  Predict
+// and W W' round alike for an entry and its mirror image, so the diagonal tiles stay
+// symmetric to the last bit.  [Mm; U; q'] is eliminated together, 16 columns at a
+// time: one wavefront factors the diagonal block (chol16_inverse), every wavefront multiplies
+// its row tiles by the block's inverse, then updates its remaining columns and its part of P
+// while the next diagonal block is factored.  M is padded to 16 MB with zero rows of L, which
+// leave Mm's padding the identity.
 // ---------------------------------------------------------------------------
 struct StFilterIO {
-  const double* dt;   // [K,T], dt[0] = 0
+  const double* aq;   // [K,T,2 KT^2] transitions
   const double* Lw;   // [K,T,M,M]
   const double* zw;   // [K,T,M]
-  const double* ldl;  // [K,T]
-  double* P;          // per-run scratch [K,D,D]
-  double* U;          // per-run scratch [K,D,M]
-  double* V;          // per-run scratch [K,D,M]
   double* fmean;      // [K,T,D] filtered means
   double* fcov;       // [K,T,D(D+1)/2] filtered covariances, packed upper triangle by rows
-  double* ell;        // [K,T] per-step log-likelihood terms
+  double* ell;        // [K,T] per-step log-likelihood terms: e' e, until k_st_ell completes them
+  double* det;        // [K,T,2] mantissa and exponent of 1 / sqrt(det Mm)
 };
+
+// ell = -1/2 (e' e + M log 2pi + log det Mm - 2 ldl), one step a thread: the logarithms stay
+// out of the recursion.
+__global__ __launch_bounds__(kT) void k_st_ell(StDims dm, const double* __restrict__ det,
+                                               const double* __restrict__ ldl, double* __restrict__ ell) {
+  const int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (e >= (int64_t)dm.K * dm.T) return;
+  const double ld = -2.0 * (log(det[2 * e]) + det[2 * e + 1] * 0.69314718055994530942);
+  ell[e] = -0.5 * (ell[e] + dm.M * kLog2Pi + ld - 2.0 * ldl[e]);
+}
 
 // packed upper-triangle index of (i, j), i <= j, in an n x n matrix
 __device__ inline int64_t pidx(int i, int j, int n) { return (int64_t)i * n - (int64_t)i * (i - 1) / 2 + (j - i); }
 
-template <int KT>
-__global__ __launch_bounds__(kT) void k_st_filter(StDims dm, StHyp hy, StFilterIO io) {
-  extern __shared__ double smem[];
-  const int M = dm.M, D = dm.D, tid = threadIdx.x;
-  const int k = blockIdx.x;
-  double* pan = smem;                        // 2*kPK*kPS
-  double* sL = pan + 2 * kPK * kPS;          // M*M
-  double* sM = sL + kMaxM * kMaxM;           // M*M
-  double* row = sM + kMaxM * kMaxM;          // 2 M (pivot rows)
-  double* vm = row + 2 * kMaxM;              // D mean
-  double* vq = vm + kMaxD;                   // M
-  double* red = vq + kMaxM;                  // 4
-  __shared__ double sA[KT * KT], sQ[KT * KT];
-  double* P = io.P + (int64_t)k * D * D;
-  double* U = io.U + (int64_t)k * D * M;
-  double* V = io.V + (int64_t)k * D * M;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  // P0 = Pinf (x) I, m0 = 0
-  {
-    double Ai[KT * KT], Pinf[KT * KT];
-    (void)Ai;
-    Model<KT, 0> mdl;
-    mdl.init(ls, var, 1.0, 1.0);
-    for (int i = 0; i < KT; ++i)
-      for (int j = 0; j < KT; ++j) Pinf[i * KT + j] = mdl.Pinf[i][j];
-    for (int64_t e = tid; e < (int64_t)D * D; e += kT) {
-      const int i = (int)(e / D), j = (int)(e % D);
-      P[e] = (i % M == j % M) ? Pinf[(i / M) * KT + (j / M)] : 0.0;
+// LDS of k_st_filter in doubles
+constexpr int filter_smem(int KT, int MB) {
+  const int MP = 16 * MB, LD = MP + 2;
+  return (KT + 2) * MP * LD + (MB + 1) * 16 * kDiagLd + 2 * MP + KT * MP + 2 * KT * KT;
+}
+
+// Row tile I of the lower triangle of Mm = I + L' U[:M] (column tiles <= I; L' is upper
+// triangular, so inner tiles >= I).
+template <int MB, int I>
+__device__ inline void filter_mm_row(const double* LT, const double* X, int ld, tile4 (&V)[MB], int l) {
+#pragma unroll
+  for (int j = 0; j <= I; ++j) V[j] = tile_zero();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) V[I][q] = (l >> 4) + 4 * q == (l & 15) ? 1.0 : 0.0;
+#pragma unroll
+  for (int kk = I; kk < MB; ++kk) {
+#pragma unroll
+    for (int c = 0; c < 16; c += 4) {
+      const double a = frag(LT, ld, 16 * I, 16 * kk + c, l);
+#pragma unroll
+      for (int j = 0; j <= I; ++j) V[j] = mfma16(a, frag_t(X, ld, 16 * kk + c, 16 * j, l), V[j]);
     }
-    for (int e = tid; e < D; e += kT) vm[e] = 0.0;
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __syncthreads();
-  for (int t = 0; t < dm.T; ++t) {
-    const int64_t kt = (int64_t)k * dm.T + t;
-    if (tid == 0) temporal_AQ<KT>(ls, var, io.dt[kt], sA, sQ);
-    __syncthreads();
-    // predict: P- = (A (x) I) P (A (x) I)' + Q (x) I, m- = (A (x) I) m
-    for (int e = tid; e < M * M; e += kT) {
-      const int a = e / M, c = e % M;
-      double blk[KT][KT], out[KT][KT];
-      for (int i = 0; i < KT; ++i)
-        for (int j = 0; j < KT; ++j) blk[i][j] = P[(int64_t)(i * M + a) * D + j * M + c];
-      for (int i = 0; i < KT; ++i)
-        for (int j = 0; j < KT; ++j) {
-          double s = (a == c) ? sQ[i * KT + j] : 0.0;
-          for (int p = 0; p < KT; ++p)
-            for (int q = 0; q < KT; ++q) s = fma(sA[i * KT + p] * blk[p][q], sA[j * KT + q], s);
-          out[i][j] = s;
-        }
-      for (int i = 0; i < KT; ++i)
-        for (int j = 0; j < KT; ++j) P[(int64_t)(i * M + a) * D + j * M + c] = out[i][j];
-    }
-    if (tid < M) {
-      double x[KT];
-      for (int i = 0; i < KT; ++i) x[i] = vm[i * M + tid];
-      for (int i = 0; i < KT; ++i) {
-        double s = 0.0;
-        for (int p = 0; p < KT; ++p) s = fma(sA[i * KT + p], x[p], s);
-        vm[i * M + tid] = s;
+}
+
+template <int KT, int MB>
+__global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, StFilterIO io) {
+  constexpr int MP = 16 * MB, LD = MP + 2, NW = 2 * MB, NT = 64 * NW;
+  constexpr int NR = KT * MB;                       // row tiles of U
+  constexpr int NPOS = MB * (MB + 1) / 2;           // tile positions (i, j), i <= j, of P
+  constexpr int NP = (NPOS + NW - 1) / NW;          // positions per wavefront, at most
+  constexpr bool kAllR = NR == NW;
+  constexpr int NL = (MP * MP + NT - 1) / NT;       // elements of L per thread
+  constexpr int NAQ = 2 * KT * KT;
+  extern __shared__ double smem[];
+  double* X = smem;                    // KT*MP x LD: P-[:, :M], then U, then W
+  double* LT = X + KT * MP * LD;       // MP x LD: L'
+  double* Lm = LT + MP * LD;           // MP x LD: Lm below the diagonal blocks
+  double* sI = Lm + MP * LD;           // MB of 16 x kDiagLd: diagonal blocks, then their inverse factors
+  double* sG = sI + MB * 16 * kDiagLd; // 16 x kDiagLd: row tile of q'
+  double* sq = sG + 16 * kDiagLd;      // MP: z, then q
+  double* se = sq + MP;                // MP: e
+  double* vm = se + MP;                // KT*MP: mean
+  double* saq = vm + KT * MP;          // NAQ: the step's A, Q
+  const int M = dm.M, D = dm.D, tid0 = threadIdx.x;
+  int tid = tid0, l = tid & 63;
+  const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int w = w0;
+  const int k = blockIdx.x;
+  // position n of a wavefront: w, then (four tiles a side only, 10 positions) 8 on wavefront 0 and
+  // 9 on wavefront 6, whose SIMDs are not the ones that factor the second and the last block
+  auto position = [&](int n, int& i, int& j) {
+    int p = n == 0 ? w : (w == 0 ? 8 : w == 6 ? 9 : NPOS);
+    const bool on = p < NPOS;
+    i = 0;
+#pragma unroll
+    for (int r = 0; r < MB - 1; ++r)
+      if (i == r && p >= MB - r) { p -= MB - r; i = r + 1; }
+    j = i + p;
+    return on;
+  };
+  tile4 P[NP][KT][KT];
+  {  // P0 = Pinf (x) I, m0 = 0
+    Model<KT, 0> mdl;
+    mdl.init(hy.ls_t[k * hy.stride], hy.var_t[k * hy.stride], 1.0, 1.0);
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      const bool held = position(n, i, j);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+        const bool on = gi == gj && gi < M && held;
+#pragma unroll
+        for (int a = 0; a < KT; ++a)
+#pragma unroll
+          for (int b = 0; b < KT; ++b) P[n][a][b][q] = on ? mdl.Pinf[a][b] : 0.0;
       }
     }
+  }
+  for (int e = tid; e < KT * MP; e += NT) vm[e] = 0.0;
+  for (int e = tid; e < 16 * kDiagLd; e += NT) sG[e] = 0.0;
+  const int64_t k0 = (int64_t)k * dm.T;
+  // the next step's L, z and transition are loaded a whole step ahead, before this step's
+  // stores: vector memory operations complete in order, so a load behind the packed
+  // covariance's stores would wait for them
+  double lreg[NL], zreg = 0.0, aqreg = 0.0;
+  auto fetch = [&](int64_t kt) {
     const double* L = io.Lw + kt * M * M;
-    for (int e = tid; e < M * M; e += kT) sL[e] = L[e];
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      const int e = tid + n * NT, r = e / MP, c = e % MP;
+      const bool on = r < M && c < M;
+      const double v = L[on ? r * M + c : 0];
+      lreg[n] = on ? v : 0.0;
+    }
+    if (tid < M) zreg = io.zw[kt * M + tid];
+    if (tid < NAQ) aqreg = io.aq[kt * NAQ + tid];
+  };
+  auto place = [&]() {
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      const int e = tid + n * NT, r = e / MP, c = e % MP;
+      if (NL * NT == MP * MP || e < MP * MP) LT[c * LD + r] = lreg[n];
+    }
+    if (tid < MP) sq[tid] = zreg;
+    if (tid < NAQ) saq[tid] = aqreg;
+  };
+  auto update_P = [&](int b) {  // P -= W_b W_b'
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!position(n, i, j)) continue;
+#pragma unroll
+      for (int c = 0; c < 16; c += 4) {
+        double ra[KT], rb[KT];
+#pragma unroll
+        for (int a = 0; a < KT; ++a) {
+          ra[a] = -frag(X, LD, (a * MB + i) * 16, 16 * b + c, l);
+          rb[a] = frag(X, LD, (a * MB + j) * 16, 16 * b + c, l);
+        }
+#pragma unroll
+        for (int a = 0; a < KT; ++a)
+#pragma unroll
+          for (int d = 0; d < KT; ++d) P[n][a][d] = mfma16(ra[a], rb[d], P[n][a][d]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto phase = [&]() { w = fresh_s(w0); tid = fresh_v(tid0); l = tid & 63; };
+  fetch(k0);
+  place();
+  __syncthreads();
+#pragma unroll 1
+  for (int t = 0; t < dm.T; ++t) {
+    phase();
+    const int64_t kt = k0 + t;
+    double A[KT][KT], Q[KT][KT];
+#pragma unroll
+    for (int a = 0; a < KT; ++a)
+#pragma unroll
+      for (int b = 0; b < KT; ++b) {
+        A[a][b] = saq[a * KT + b];
+        Q[a][b] = saq[KT * KT + a * KT + b];
+      }
+    // P- = (A (x) I) P (A (x) I)' + Q (x) I; the mixed products are added first, so that
+    // (i, j) and (j, i) round alike
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!position(n, i, j)) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+        const double on = gi == gj && gi < M ? 1.0 : 0.0;
+        if (KT == 1) {
+          P[n][0][0][q] = fma(A[0][0] * A[0][0], P[n][0][0][q], on * Q[0][0]);
+        } else {
+          constexpr int o = KT - 1;
+          const double a = P[n][0][0][q], b = P[n][0][o][q], c = P[n][o][0][q], d = P[n][o][o][q];
+          const double s = b + c;
+          P[n][0][0][q] = fma(A[0][0] * A[0][0], a, fma(A[0][0] * A[0][o], s, fma(A[0][o] * A[0][o], d, on * Q[0][0])));
+          P[n][o][o][q] = fma(A[o][0] * A[o][0], a, fma(A[o][0] * A[o][o], s, fma(A[o][o] * A[o][o], d, on * Q[o][o])));
+          const double u = fma(A[0][0] * A[o][0], a, fma(A[0][o] * A[o][o], d, on * Q[0][o]));
+          const double x = A[0][0] * A[o][o], y = A[0][o] * A[o][0];
+          P[n][0][o][q] = fma(y, c, fma(x, b, u));
+          P[n][o][0][q] = fma(y, b, fma(x, c, u));
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < KT; ++a) {
+        tile_store(X, LD, (a * MB + i) * 16, 16 * j, P[n][a][0], l);
+        if (i != j) tile_store_t(X, LD, (a * MB + j) * 16, 16 * i, P[n][0][a], l);
+      }
+    }
+    if (tid < MP) {
+      double x[KT];
+#pragma unroll
+      for (int a = 0; a < KT; ++a) x[a] = vm[a * MP + tid];
+#pragma unroll
+      for (int a = 0; a < KT; ++a) {
+        double v = 0.0;
+#pragma unroll
+        for (int b = 0; b < KT; ++b) v = fma(A[a][b], x[b], v);
+        vm[a * MP + tid] = v;
+      }
+    }
     __syncthreads();
-    // U = P-[:, :M] L ;  Mm = I + L' Sh L = I + L' U[:M] ;  q = z - L' H m-
-    wg_gemm(D, M, M, 1.0, MatRef{P, D, 1}, MatRef{sL, M, 1}, 0.0, U, M, pan);
-    wg_gemm(M, M, M, 1.0, MatRef{sL, 1, M}, MatRef{U, M, 1}, 0.0, sM, M, pan);
-    for (int e = tid; e < M; e += kT) sM[e * M + e] += 1.0;
-    if (tid < M) {
-      double u = io.zw[kt * M + tid];
-      for (int a = tid; a < M; ++a) u = fma(-sL[a * M + tid], vm[a], u);
-      vq[tid] = u;
+    phase();
+    if (t + 1 < dm.T) fetch(kt + 1);
+    // U (row tile w) = P-[:, :M] L: L is lower triangular, column tile j needs inner tiles >= j
+    tile4 U[MB];
+#pragma unroll
+    for (int j = 0; j < MB; ++j) U[j] = tile_zero();
+    if (kAllR || w < NR) {
+#pragma unroll
+      for (int kk = 0; kk < MB; ++kk) {
+#pragma unroll
+        for (int c = 0; c < 16; c += 4) {
+          const double a = frag(X, LD, 16 * w, 16 * kk + c, l);
+#pragma unroll
+          for (int j = 0; j <= kk; ++j) U[j] = mfma16(a, frag(LT, LD, 16 * j, 16 * kk + c, l), U[j]);
+        }
+      }
+      wave_sync();
+#pragma unroll
+      for (int j = 0; j < MB; ++j) tile_store(X, LD, 16 * w, 16 * j, U[j], l);
     }
-    const double ldM = wg_sweep_inv<kMaxM / 16, true>(sM, M, M, row);  // sM = -Mm^-1 (ldM: thread 0)
-    // log N = -1/2 (q' Mm^-1 q + M log 2pi + log det Mm - 2 ldl)
-    double qq = 0.0;
-    if (tid < M) {
-      double u = 0.0;
-      for (int c = 0; c < M; ++c) u = fma(sM[tid * M + c], vq[c], u);
-      qq = -vq[tid] * u;
+    if (w >= MB) {  // q = z - L' H m-, 16 rows a wavefront
+      const int r0 = 16 * (w - MB);
+      double v = 0.0;
+#pragma unroll
+      for (int c = 0; c < MP; c += 4) v = fma(frag(LT, LD, r0, c, l), vm[c + (l >> 4)], v);
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (l < 16) sq[r0 + l] -= v;
     }
-    const double quad = wg_sum(qq, red);
-    if (tid == 0) io.ell[kt] = -0.5 * (quad + M * kLog2Pi + ldM - 2.0 * io.ldl[kt]);
-    // V = U Mm^-1 ; m = m- + V q ; P = P- - V U'
-    wg_gemm(D, M, M, -1.0, MatRef{U, M, 1}, MatRef{sM, M, 1}, 0.0, V, M, pan);
-    for (int i = tid; i < D; i += kT) {
-      double s2 = vm[i];
-      for (int c = 0; c < M; ++c) s2 = fma(V[(int64_t)i * M + c], vq[c], s2);
-      vm[i] = s2;
+    __syncthreads();
+    phase();
+    // the wavefront's second row tile V: row tile w of Mm (w < MB), or q' (the last wavefront)
+    tile4 V[MB];
+    double quad = 0.0;  // lanes 0-15 of the last wavefront: e' e
+    if (w == 0) {
+      filter_mm_row<MB, 0>(LT, X, LD, V, l);
+      tile_store(sI, kDiagLd, 0, 0, V[0], l);
+      wave_sync();
+      chol16_inverse(sI, l);
+    } else if (MB > 1 && w == 1) {
+      filter_mm_row<MB, (MB > 1 ? 1 : 0)>(LT, X, LD, V, l);
+    } else if (MB > 2 && w == 2) {
+      filter_mm_row<MB, (MB > 2 ? 2 : 0)>(LT, X, LD, V, l);
+    } else if (MB > 3 && w == 3) {
+      filter_mm_row<MB, (MB > 3 ? 3 : 0)>(LT, X, LD, V, l);
+    } else if (w == NW - 1) {
+#pragma unroll
+      for (int j = 0; j < MB; ++j) {
+        V[j] = tile_zero();
+        V[j][0] = l < 16 ? sq[16 * j + l] : 0.0;
+      }
     }
-    wg_gemm(D, D, M, -1.0, MatRef{V, M, 1}, MatRef{U, 1, M}, 1.0, P, D, pan);
-    for (int i = tid; i < D; i += kT) io.fmean[kt * D + i] = vm[i];
-    // P - V U' is symmetric only to rounding, and the asymmetry compounds through the next
-    // steps' Mm (whose inverse assumes symmetry): P := (P + P')/2, each pair (i < j) by the
-    // one lane that also writes its packed entry
+    // one copy of the block's code (the unrolled loop would not fit the instruction cache): U and
+    // V are shifted by one tile after each block, so that tile 0 is always the current one
+#pragma unroll 1
+    for (int b = 0; b < MB; ++b) {
+      const double* Ib = sI + b * 16 * kDiagLd;
+      __syncthreads();  // inverse factor of diagonal block b
+      phase();
+      // row tiles times the inverse factor's transpose: column block b of W, Lm and e
+      if (w > b && w < MB) {
+        tile_store(Lm, LD, 16 * w, 16 * b, V[0], l);
+        wave_sync();
+        const tile4 v = tile_mul_t(Lm, LD, 16 * w, Ib, kDiagLd, 0, 16 * b, 0, tile_zero(), l);
+        wave_sync();
+        tile_store(Lm, LD, 16 * w, 16 * b, v, l);
+      } else if (w == NW - 1) {
+        tile_store(sG, kDiagLd, 0, 0, V[0], l);
+        wave_sync();
+        const tile4 v = tile_mul_t(sG, kDiagLd, 0, Ib, kDiagLd, 0, 0, 0, tile_zero(), l);
+        wave_sync();
+        tile_store(sG, kDiagLd, 0, 0, v, l);
+        if (l < 16) {
+          se[16 * b + l] = v[0];
+          quad = fma(v[0], v[0], quad);
+        }
+      }
+      if (kAllR || w < NR) {
+        if (b > 0) {
+          tile_store(X, LD, 16 * w, 16 * b, U[0], l);
+          wave_sync();
+        }
+        const tile4 v = tile_mul_t(X, LD, 16 * w, Ib, kDiagLd, 0, 16 * b, 0, tile_zero(), l);
+        wave_sync();
+        tile_store(X, LD, 16 * w, 16 * b, v, l);
+      }
+      if (MB > 1 && w == b + 1 && w < MB) {
+        // the next diagonal block first: its factorisation is the critical path
+#pragma unroll
+        for (int c = 0; c < 16; c += 4) {
+          const double a = frag(Lm, LD, 16 * w, 16 * b + c, l);
+          V[MB > 1 ? 1 : 0] = mfma16(-a, a, V[MB > 1 ? 1 : 0]);
+        }
+        tile_store(sI + (b + 1) * 16 * kDiagLd, kDiagLd, 0, 0, V[MB > 1 ? 1 : 0], l);
+      }
+      __syncthreads();  // column block b of W and Lm
+      phase();
+      // remaining columns of the row tiles
+      if (b + 1 < MB) {
+        if (w == b + 1) chol16_inverse(sI + (b + 1) * 16 * kDiagLd, l);
+        double a[4];
+        if ((w > b + 1 && w < MB) || w == NW - 1) {
+          const double* S = w == NW - 1 ? sG : Lm + 16 * w * LD + 16 * b;
+          const int ld = w == NW - 1 ? kDiagLd : LD;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) a[c] = -frag(S, ld, 0, 4 * c, l);
+#pragma unroll
+          for (int j = 1; j < MB; ++j)
+            if (b + j < MB) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) V[j] = mfma16(a[c], frag(Lm, LD, 16 * (b + j), 16 * b + 4 * c, l), V[j]);
+            }
+        }
+        if (kAllR || w < NR) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) a[c] = -frag(X, LD, 16 * w, 16 * b + 4 * c, l);
+#pragma unroll
+          for (int j = 1; j < MB; ++j)
+            if (b + j < MB) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) U[j] = mfma16(a[c], frag(Lm, LD, 16 * (b + j), 16 * b + 4 * c, l), U[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j + 1 < MB; ++j) { U[j] = U[j + 1]; V[j] = V[j + 1]; }
+      }
+      // (a wavefront on the SIMD that factors the next block leaves its part to the last one)
+      const int late = (w & 3) > 0 && (w & 3) < MB ? (w & 3) - 1 : -1;
+      const int n = b == late ? 0 : b == MB - 1 && late >= 0 ? 2 : 1;
+#pragma unroll 1
+      for (int u = 0; u < n; ++u) update_P(u == 0 ? b : late);
+    }
+    phase();
+    if (t + 1 < dm.T) place();  // LT, sq and saq are not read again in this step
+    // m = m- + W e, rows 16 w .. (each wavefront its own)
+    if (kAllR || w < NR) {
+      double v = 0.0;
+#pragma unroll
+      for (int c = 0; c < MP; c += 4) v = fma(frag(X, LD, 16 * w, c, l), se[c + (l >> 4)], v);
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      if (l < 16) {
+        const double m = vm[16 * w + l] + v;
+        vm[16 * w + l] = m;
+        const int a = w / MB, i = 16 * (w % MB) + l;
+        if (i < M) io.fmean[kt * D + a * M + i] = m;
+      }
+    }
+    if (w == NW - 1) {
+      // 1 / sqrt(det Mm): the product of the inverse factors' diagonals
+      double m = 1.0;
+      int x = 0;
+      if (l < MP) m = frexp(sI[(l >> 4) * 16 * kDiagLd + (l & 15) * (kDiagLd + 1)], &x);
+      quad = l < 16 ? quad : 0.0;
+      for (int o = 32; o > 0; o >>= 1) {
+        m *= __shfl_xor(m, o, 64);
+        x += __shfl_xor(x, o, 64);
+        quad += __shfl_xor(quad, o, 64);
+      }
+      if (l == 0) {
+        io.ell[kt] = quad;
+        io.det[2 * kt] = m;
+        io.det[2 * kt + 1] = x;
+      }
+    }
     double* fc = io.fcov + kt * ((int64_t)D * (D + 1) / 2);
-    for (int i = tid >> 6; i < D; i += kT / 64) {  // one wave per row
-      const int64_t o = pidx(i, i, D) - i;
-      for (int j = i + (tid & 63); j < D; j += 64) {
-        const double v = 0.5 * (P[(int64_t)i * D + j] + P[(int64_t)j * D + i]);
-        P[(int64_t)i * D + j] = v;
-        P[(int64_t)j * D + i] = v;
-        fc[o + j] = v;
+    phase();
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!position(n, i, j)) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+        if (gi < M && gj < M) {
+#pragma unroll
+          for (int a = 0; a < KT; ++a) {
+            const int r = a * M + gi;
+            double* o = fc + r * D - r * (r - 1) / 2 - r + gj;
+#pragma unroll
+            for (int d = a; d < KT; ++d)
+              if (d > a || gi <= gj) o[d * M] = P[n][a][d][q];
+          }
+          if (KT > 1 && i != j) fc[gj * D - gj * (gj - 1) / 2 - gj + M + gi] = P[n][KT - 1][0][q];
+        }
       }
     }
     __syncthreads();
@@ -1908,7 +2219,6 @@ __global__ __launch_bounds__(kT) void k_st_predict(StDims dm, StHyp hy, StPredIO
   }
 }
 
-constexpr size_t kFilterSmem = sizeof(double) * (2 * kPK * kPS + 2 * kMaxM * kMaxM + 2 * kMaxM + kMaxD + kMaxM + 4);
 constexpr size_t kSmootherSmem = sizeof(double) * (2 * kPK * kPS + kMaxD * kMaxD + 6 * kMaxD);
 constexpr size_t kGainsSmem = sizeof(double) * (2 * kPK * kPS + kMaxD * kMaxD + 2 * kMaxD);
 constexpr size_t kSmootherSeqSmem = sizeof(double) * (2 * kPK * kPS + 4 * kMaxD);
@@ -1941,10 +2251,18 @@ StHyp make_hyp(const bn_st_hypers* h) { return StHyp{h->ls_t, h->var_t, h->var_s
 int set_smem_limits() {
   static int done = 0;
   if (done) return BN_OK;
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_filter<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kFilterSmem));
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_filter<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kFilterSmem));
+#define ST_FILTER_ATTR(KT, MB)                                                                                  \
+  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_filter<KT, MB>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                   (int)sizeof(double) * filter_smem(KT, MB)))
+  ST_FILTER_ATTR(1, 1);
+  ST_FILTER_ATTR(1, 2);
+  ST_FILTER_ATTR(1, 3);
+  ST_FILTER_ATTR(1, 4);
+  ST_FILTER_ATTR(2, 1);
+  ST_FILTER_ATTR(2, 2);
+  ST_FILTER_ATTR(2, 3);
+  ST_FILTER_ATTR(2, 4);
+#undef ST_FILTER_ATTR
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_gains<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kGainsSmem));
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_gains<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1982,6 +2300,31 @@ int set_smem_limits() {
                                    (int)kCavitySmem));
   done = 1;
   return BN_OK;
+}
+
+// k_st_filter for the 16-wide tiles that M needs.
+template <int KT>
+void launch_st_filter(hipStream_t st, StDims dm, StHyp hy, StFilterIO io) {
+  switch ((dm.M + 15) / 16) {
+    case 1:
+      hipLaunchKernelGGL((k_st_filter<KT, 1>), dim3(dm.K), dim3(128), sizeof(double) * filter_smem(KT, 1), st, dm, hy, io);
+      break;
+    case 2:
+      hipLaunchKernelGGL((k_st_filter<KT, 2>), dim3(dm.K), dim3(256), sizeof(double) * filter_smem(KT, 2), st, dm, hy, io);
+      break;
+    case 3:
+      hipLaunchKernelGGL((k_st_filter<KT, 3>), dim3(dm.K), dim3(384), sizeof(double) * filter_smem(KT, 3), st, dm, hy, io);
+      break;
+    default:
+      hipLaunchKernelGGL((k_st_filter<KT, 4>), dim3(dm.K), dim3(512), sizeof(double) * filter_smem(KT, 4), st, dm, hy, io);
+      break;
+  }
+}
+
+template <int KT>
+void launch_st_transitions(hipStream_t st, StDims dm, StHyp hy, const double* dt, double* aq) {
+  const unsigned nb = (unsigned)(((int64_t)dm.K * dm.T + kT - 1) / kT);
+  hipLaunchKernelGGL(k_st_transitions<KT>, dim3(nb), dim3(kT), 0, st, dm, hy, dt, aq);
 }
 
 // k_st_sites<MT, MD> for the likelihood kind L.kind (checked by check_lik).
@@ -2114,10 +2457,12 @@ int bn_st_ep_sites(const bn_st_dims* dims, const bn_lik_desc* lik, int32_t mode,
 int64_t bn_st_workspace_bytes(const bn_st_dims* dims) {
   StDims dm;
   if (check_dims(dims, dm) != BN_OK) return -1;
-  // per run: filter P (D x D) and V (D x M); smoother Ps, Dl, GT (3 x D x D) and m_s (D),
-  // then the smoother's block of gains and unpacked covariances (gain_block_steps)
+  // filter: the transitions (2 KT^2) and the determinant (2) of every step.  Smoother, per run: Ps, Dl, GT (3 x D x D) and
+  // m_s (D), then the block of gains and unpacked covariances (gain_block_steps)
   const int64_t D = dm.D;
-  return (int64_t)dm.K * (5 * D * D + 2 * D * D * gain_block_steps(dm)) * (int64_t)sizeof(double) + 4096;
+  const int64_t smoother = 5 * D * D + 2 * D * D * gain_block_steps(dm);
+  const int64_t filter = 2 * ((int64_t)dm.KT * dm.KT + 1) * dm.T;
+  return (int64_t)dm.K * (smoother > filter ? smoother : filter) * (int64_t)sizeof(double) + 4096;
 }
 
 int bn_st_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, const double* dt, const double* Lw,
@@ -2128,17 +2473,21 @@ int bn_st_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, const double* 
   if (!hyp || !dt || !Lw || !zw || !ldl || !filter_mean || !filter_cov || !ell_steps || !loglik || !workspace)
     return st_fail(BN_EINVAL, "NULL argument to bn_st_filter");
   double* ws = (double*)workspace;
-  const int64_t D = dm.D;
   if (int rc = set_smem_limits()) return rc;
-  StFilterIO io{dt, Lw, zw, ldl, ws, ws + dm.K * D * D, ws + dm.K * (D * D + D * dm.M), filter_mean, filter_cov,
-                ell_steps};
+  StFilterIO io{ws, Lw, zw, filter_mean, filter_cov, ell_steps, ws + (int64_t)dm.K * dm.T * 2 * dm.KT * dm.KT};
   hipStream_t st = (hipStream_t)stream;
+  const StHyp hy = make_hyp(hyp);
   {
     BN_TIMED(KID_ST_FILTER, st);
-    if (dm.KT == 1)
-      hipLaunchKernelGGL(k_st_filter<1>, dim3(dm.K), dim3(kT), kFilterSmem, st, dm, make_hyp(hyp), io);
-    else
-      hipLaunchKernelGGL(k_st_filter<2>, dim3(dm.K), dim3(kT), kFilterSmem, st, dm, make_hyp(hyp), io);
+    if (dm.KT == 1) {
+      launch_st_transitions<1>(st, dm, hy, dt, ws);
+      launch_st_filter<1>(st, dm, hy, io);
+    } else {
+      launch_st_transitions<2>(st, dm, hy, dt, ws);
+      launch_st_filter<2>(st, dm, hy, io);
+    }
+    hipLaunchKernelGGL(k_st_ell, dim3((unsigned)(((int64_t)dm.K * dm.T + kT - 1) / kT)), dim3(kT), 0, st, dm, io.det,
+                       ldl, ell_steps);
   }
   ST_HIP_CHECK(hipGetLastError());
   {

@@ -1,0 +1,62 @@
+"""The space-time kernels at the edges of their 16-wide tiles: numbers of inducing points
+around multiples of 16, both temporal state sizes, the shortest runs, against the FP64 oracle.
+
+Tolerance 1e-6 of the field's scale: FP64 throughout on both sides, and the oracle's explicit
+inverse of B' diag(nat2) B (condition up to about 1e7 on these grids) limits the agreement to
+about 1e7 * 2e-16 with two orders of headroom.
+"""
+import numpy as np
+import pytest
+
+from oracle import kernels as OK, likelihoods as OL, models as OM
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+
+
+def _case(M, kt, T, seed=11):
+    from bayesnewton_amd import kernels as K, likelihoods as L, models as GM
+    g = np.linspace(0.0, 1.0, 8)
+    a, b = np.meshgrid(g, g)
+    z = np.stack([a.ravel(), b.ravel()], 1)[:M]
+    rng = np.random.default_rng(seed)
+    nr = 4 * M + 3
+    t = np.cumsum(rng.integers(1, 4, T)).astype(np.float64)
+    r = rng.uniform(size=(T, nr, 2)).astype(np.float32).astype(np.float64)
+    f = np.sin(0.3 * t)[:, None] + np.cos(3.0 * r[..., 0]) * np.sin(2.0 * r[..., 1])
+    y = rng.poisson(2.0 * np.exp(f)).astype(np.float64)
+    gt, ot = ((K.Matern12, OK.Matern12), (K.Matern32, OK.Matern32))[kt - 1]
+    gk = K.SpatioTemporalKernel(gt(variance=1.2, lengthscale=6.0), K.Matern32(variance=0.9, lengthscale=0.25), z=z)
+    ok = OK.SpatioTemporalKernel(ot(1.2, 6.0), OK.Matern32(0.9, 0.25), z, sparse=True, conditional="Full")
+    gm = GM.MarkovVariationalGP(gk, L.Poisson(binsize=2.0), t, y, R=r)
+    om = OM.MarkovGP(ok, OL.Poisson(2.0), t[:, None], y, R=r, inference="VI")
+    return gm, om
+
+
+def _close(got, want):
+    got, want = got.cpu().numpy(), np.asarray(want)
+    assert got.shape == want.shape
+    assert np.max(np.abs(got - want)) <= TOL * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("kt", [1, 2])
+@pytest.mark.parametrize("M", [1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64])
+def test_inducing_points_around_tiles(M, kt):
+    gm, om = _case(M, kt, 6)
+    for _ in range(2):
+        gm.inference(lr=0.2)
+        om.inference(lr=0.2)
+    _close(gm.posterior_mean, om.posterior_mean)
+    _close(gm.posterior_variance, om.posterior_variance)
+    assert abs(float(gm.energy()) - om.energy()) <= TOL * abs(om.energy())
+
+
+@pytest.mark.parametrize("T", [1, 2, 3])
+def test_shortest_runs(T):
+    gm, om = _case(20, 2, T)
+    gm.inference(lr=0.2)
+    om.inference(lr=0.2)
+    _close(gm.posterior_mean, om.posterior_mean)
+    _close(gm.posterior_variance, om.posterior_variance)
+    assert abs(float(gm.compute_log_lik()) - om.compute_log_lik()) <= TOL * abs(om.compute_log_lik())
