@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
       filter_mm_row<MB, 0>(LT, X, LD, V, l);
       tile_store(sI, kDiagLd, 0, 0, V[0], l);
       wave_sync();
-      chol16_inverse(sI, l);
+      chol16_inverse(sI, kDiagLd, l);
     } else if (MB > 1 && w == 1) {
       filter_mm_row<MB, (MB > 1 ? 1 : 0)>(LT, X, LD, V, l);
     } else if (MB > 2 && w == 2) {
@@ -1144,7 +1144,7 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
       phase();
       // remaining columns of the row tiles
       if (b + 1 < MB) {
-        if (w == b + 1) chol16_inverse(sI + (b + 1) * 16 * kDiagLd, l);
+        if (w == b + 1) chol16_inverse(sI + (b + 1) * 16 * kDiagLd, kDiagLd, l);
         double a[4];
         if ((w > b + 1 && w < MB) || w == NW - 1) {
           const double* S = w == NW - 1 ? sG : Lm + 16 * w * LD + 16 * b;
@@ -1237,207 +1237,517 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
 }
 
 // ---------------------------------------------------------------------------
-// RTS backward pass (ops.py:288-311) in two kernels.  The gain of step t,
-//   G_t' = (P-_{t+1})^-1 A P_t,  P-_{t+1} = A P_t A' + Q  (A, Q of dt[t+1], basemodels.py:700),
-// depends on the filtered covariances only, so k_st_gains computes the gains of a block
-// of steps for every run at once, one workgroup per (step, run) (sweep inverse of P- in
-// LDS, one D^3 product); k_st_smoother then walks the block backwards, one workgroup per
-// run, with the two D^3 products left on the recursion:
-//   m_s = m + G (m_s' - A m),  P_s = P + G (P_s' - P-) G'.
-// Outputs H m_s and H P_s H' (the first M states), and with return_full the state, its
-// covariance and the neighbours' cross covariance G_t P_s,t+1.
-// Blocks of steps run from the end of the series; a block's gains and unpacked filtered
-// covariances sit in a workspace buffer of gain_block_steps() steps per run.
+// RTS backward pass (ops.py:288-311).  The step from t + 1 to t is the affine map
+//   m_s = c_t + G_t m_s',  P_s = R_t + G_t P_s' G_t',
+//   G_t = P_t A' (P-)^-1,  c_t = m_t - G_t m-,  R_t = P_t - G_t P- G_t'  (P-, m-, A of t + 1),
+// whose coefficients depend on the filter only:
+//   k_st_gains     the maps of a block of steps of every run, one workgroup per (step, run):
+//                  P- = Lc Lc', W = P_t A' Lc^-T, R = P_t - W W', G = W Lc^-1
+//   k_st_chain     with few runs, the product of the G_t of a chunk of steps, and
+//   k_st_smoother  in COMPOSE mode the chunk's c and R, which make the chunk one map; in JOIN
+//                  mode the chunks' maps applied one after the other to the state at the
+//                  block's end; in WALK mode every chunk's steps from its right end, with the
+//                  outputs H m_s, H P_s H' (the first M states) and, for prediction, the state,
+//                  its covariance and the neighbours' cross covariance G_t P_s,t+1.
+// One workgroup walks a chunk, so a block of n steps costs n / chunks (compose) + chunks (join)
+// + n / chunks (walk) steps instead of n; smoother_chunks() picks the number.
+// State layout of these kernels: each of the KT components padded to MP = 16 MB entries, as
+// NR = KT MB tiles a side; symmetric matrices as the NR (NR + 1) / 2 tiles (r, j <= r).
 // ---------------------------------------------------------------------------
-struct StSmootherIO {
-  const double* dt;
-  const double* fmean;  // [K,T,D]
-  const double* fcov;   // [K,T,D(D+1)/2]
-  double* Ps;           // per-run scratch [K,D,D] each: P_s of the step after the current one
-  double* Dl;           //   P_s' - P-
-  double* GT;           //   G (P_s' - P-)
-  double* ms;           // per-run [K,D]: m_s of the step after the current one
-  double* buf;          // [K, tb, 2, D, D]: unpacked P_t and G_t' of the block's steps
-  int tb;               // steps per block in buf
-  double* pm;           // [K,T,M]
-  double* pP;           // [K,T,M,M]
-  double* smean;        // optional [K,T,D] smoothed state (return_full)
-  double* scov;         // optional [K,T,D,D]
-  double* scross;       // optional [K,T,D,D]: G_t P_s,t+1 = Cov(x_t, x_t+1 | y); Pinf at the last step
+template <int KT, int MB>
+struct StTiles {
+  static constexpr int MP = 16 * MB, NR = KT * MB, DP = 16 * NR, LD = DP + 2, NF = DP / 4;
+  static constexpr int SYM = NR * (NR + 1) / 2 * 256;   // symmetric matrix
+  static constexpr int STATE = SYM + DP;                // covariance, mean
+  static constexpr int REC = DP * DP + SYM + DP;        // map: G (fragments by row tile), R, c
+  static constexpr int SMEM = DP * LD + DP * kDiagLd + 2 * DP;
+  // row tile of a wavefront: with eight, wavefronts w and w + 4 share a SIMD, and rows w and 7 - w
+  // together have the same number of tiles of a symmetric matrix for every w
+  static __device__ int row(int w) { return NR == 8 && w >= 4 ? 11 - w : w; }
+  static __device__ int sym(int r, int j) { return (r * (r + 1) / 2 + j) * 256; }
 };
 
-// bytes of the gain block buffer: 1953 steps of one d = 128 run, 9 steps each of 200 runs
+struct StGainIO {
+  const double* aq;     // [K,T,2 KT^2]
+  const double* fmean;  // [K,T,D]
+  const double* fcov;   // [K,T,D(D+1)/2]
+  double* rec;          // [K, tb] maps
+  int t0, tb;
+};
+
+// Per workgroup: 36 + 64 tiles in registers, Lc in LDS.  Bound by the eight pivot chains
+// (chol16_inverse) and, behind them, by the matrix instructions of the elimination and of the
+// back substitution.  M = 64, D = 128: 999 steps in 293 us (617 us with the sweep inverse of P-
+// in LDS and a product through panels).
+template <int KT, int MB>
+__global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainIO io) {
+  using S = StTiles<KT, MB>;
+  constexpr int MP = S::MP, NR = S::NR, DP = S::DP, LD = S::LD, NW = NR;
+  extern __shared__ double smem[];
+  double* X = smem;              // DP x LD: P_t, then Lc (inverse factors on the diagonal tiles)
+  double* sW = X + DP * LD;      // DP x kDiagLd: column block b of W; 16 rows of it a wavefront's staging
+  double* vp = sW + DP * kDiagLd;  // DP: m-
+  const int M = dm.M, D = dm.D, tid = threadIdx.x;
+  int l = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = S::row(w);
+  const int k = blockIdx.y, t = io.t0 + blockIdx.x;
+  const int64_t kt = (int64_t)k * dm.T + t;
+  const double* aq = io.aq + (kt + 1) * 2 * KT * KT;
+  double A[KT][KT], Q[KT][KT];
+#pragma unroll
+  for (int a = 0; a < KT; ++a)
+#pragma unroll
+    for (int b = 0; b < KT; ++b) {
+      A[a][b] = aq[a * KT + b];
+      Q[a][b] = aq[KT * KT + a * KT + b];
+    }
+  {  // P_t into LDS, both triangles, zero padding
+    const double* pk = io.fcov + kt * ((int64_t)D * (D + 1) / 2);
+#pragma unroll 4
+    for (int pr = w; pr < DP; pr += NW) {
+      const int a = pr / MP, i = pr % MP, u = a * M + i;
+      const double* row = pk + u * D - u * (u - 1) / 2 - u;
+#pragma unroll
+      for (int n = 0; n < (DP + 63) / 64; ++n) {
+        const int pc = l + 64 * n, b = pc / MP, j = pc % MP;
+        if (pc >= pr && pc < DP) {
+          const bool on = i < M && j < M;
+          const double v = on ? row[b * M + j] : 0.0;
+          X[pr * LD + pc] = v;
+          X[pc * LD + pr] = v;
+        }
+      }
+    }
+    for (int e = tid; e < DP; e += 64 * NW) {
+      const int a = e / MP, i = e % MP;
+      double v = 0.0;
+      if (i < M) {
+#pragma unroll
+        for (int b = 0; b < KT; ++b) v = fma(aq[a * KT + b], io.fmean[kt * D + b * M + i], v);
+      }
+      vp[e] = v;
+    }
+  }
+  __syncthreads();
+  // row tile r of P- (tiles <= r; identity padding), of P_t A' and of P_t
+  tile4 Sm[NR], U[NR], R[NR];
+  {
+    const int ra = r / MB, ri = r % MB;
+    double Ar[KT], Qr[KT];
+#pragma unroll
+    for (int b = 0; b < KT; ++b) {
+      Ar[b] = ra == 0 ? A[0][b] : A[KT - 1][b];
+      Qr[b] = ra == 0 ? Q[0][b] : Q[KT - 1][b];
+    }
+#pragma unroll
+    for (int jj = 0; jj < MB; ++jj)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * ri + (l >> 4) + 4 * q, gj = 16 * jj + (l & 15);
+        double own[KT], ap[KT];
+#pragma unroll
+        for (int b = 0; b < KT; ++b) {
+          double p[KT];
+#pragma unroll
+          for (int a = 0; a < KT; ++a) p[a] = X[(a * MP + gi) * LD + b * MP + gj];
+          own[b] = ra == 0 ? p[0] : p[KT - 1];
+          ap[b] = 0.0;
+#pragma unroll
+          for (int a = 0; a < KT; ++a) ap[b] = fma(Ar[a], p[a], ap[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < KT; ++b) {
+          double s = gi != gj ? 0.0 : gi < M ? Qr[b] : ra == b ? 1.0 : 0.0, u = 0.0;
+#pragma unroll
+          for (int a = 0; a < KT; ++a) {
+            s = fma(ap[a], A[b][a], s);
+            u = fma(own[a], A[b][a], u);
+          }
+          Sm[b * MB + jj][q] = s;
+          U[b * MB + jj][q] = u;
+          R[b * MB + jj][q] = own[b];
+        }
+      }
+  }
+  __syncthreads();  // X becomes Lc
+  double* st = sW + r * 16 * kDiagLd;
+  if (r == 0) {
+    tile_store(X, LD, 0, 0, Sm[0], l);
+    wave_sync();
+    chol16_inverse(X, LD, l);
+  }
+#pragma unroll
+  for (int b = 0; b < NR; ++b) {
+    const double* Ib = X + 16 * b * LD + 16 * b;
+    __syncthreads();  // inverse factor of diagonal block b
+    l = fresh_v(l);
+    if (r > b) {
+      tile_store(st, kDiagLd, 0, 0, Sm[b], l);
+      wave_sync();
+      const tile4 v = tile_mul_t(st, kDiagLd, 0, Ib, LD, 0, 0, 0, tile_zero(), l);
+      tile_store(X, LD, 16 * r, 16 * b, v, l);
+      wave_sync();
+    }
+    tile_store(st, kDiagLd, 0, 0, U[b], l);
+    wave_sync();
+    U[b] = tile_mul_t(st, kDiagLd, 0, Ib, LD, 0, 0, 0, tile_zero(), l);
+    wave_sync();
+    tile_store(st, kDiagLd, 0, 0, U[b], l);
+    if (b + 1 < NR && r == b + 1) {  // the next diagonal block first
+      double a[4];
+      frag4(a, X, LD, 16 * r, 16 * b, 1.0, l);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) Sm[b + 1] = mfma16(-a[c], a[c], Sm[b + 1]);
+      tile_store(X, LD, 16 * r, 16 * r, Sm[b + 1], l);
+    }
+    __syncthreads();  // column block b of Lc and W
+    l = fresh_v(l);
+    double a[4];
+    if (b + 1 < NR) {
+      if (r == b + 1) {
+        chol16_inverse(X + 16 * r * LD + 16 * r, LD, l);
+      } else if (r > b + 1) {
+        frag4(a, X, LD, 16 * r, 16 * b, -1.0, l);
+#pragma unroll
+        for (int j = b + 1; j < NR; ++j)
+          if (j <= r) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) Sm[j] = mfma16(a[c], frag(X, LD, 16 * j, 16 * b + 4 * c, l), Sm[j]);
+          }
+      }
+    }
+    frag4(a, st, kDiagLd, 0, 0, -1.0, l);
+#pragma unroll
+    for (int j = b + 1; j < NR; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) U[j] = mfma16(a[c], frag(X, LD, 16 * j, 16 * b + 4 * c, l), U[j]);
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) R[j] = mfma16(a[c], frag(sW, kDiagLd, 16 * j, 4 * c, l), R[j]);
+      }
+  }
+  double* rec = io.rec + ((int64_t)k * io.tb + blockIdx.x) * S::REC;
+#pragma unroll
+  for (int j = 0; j < NR; ++j)
+    if (j <= r) tile_put(rec + DP * DP + S::sym(r, j), R[j], l);
+  __syncthreads();  // every wavefront has read the last column block of W
+  // G = W Lc^-1, columns from the last; the rows are the wavefront's own
+  double cv = 0.0;
+  double* g = rec + r * 16 * DP;
+#pragma unroll
+  for (int b = NR - 1; b >= 0; --b) {
+    l = fresh_v(l);
+    double a[4];
+    tile_store(st, kDiagLd, 0, 0, U[b], l);
+    wave_sync();
+    frag4(a, st, kDiagLd, 0, 0, 1.0, l);
+    tile4 v = tile_zero();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v = mfma16(a[c], frag_t(X, LD, 16 * b + 4 * c, 16 * b, l), v);
+    wave_sync();
+    tile_store(st, kDiagLd, 0, 0, v, l);
+    wave_sync();
+    frag4(a, st, kDiagLd, 0, 0, 1.0, l);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      g[(4 * b + c) * 64 + l] = a[c];
+      cv = fma(a[c], vp[16 * b + 4 * c + (l >> 4)], cv);
+      a[c] = -a[c];
+    }
+#pragma unroll
+    for (int j = 0; j < b; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) U[j] = mfma16(a[c], frag_t(X, LD, 16 * b + 4 * c, 16 * j, l), U[j]);
+    wave_sync();
+  }
+  cv += __shfl_xor(cv, 16, 64);
+  cv += __shfl_xor(cv, 32, 64);
+  if (l < 16) {
+    const int i = 16 * (r % MB) + l;
+    rec[DP * DP + S::SYM + 16 * r + l] = i < M ? io.fmean[kt * D + (r / MB) * M + i] - cv : 0.0;
+  }
+}
+
+struct StSmootherIO {
+  double* rec;       // [K, tb] maps of the block's steps
+  double* comp;      // [K, nc] maps of its chunks
+  double* state;     // [K, slots] states: 0 / 1 the block's right end and its result, 2 + c the right
+                     // end of chunk c
+  int tb, nc, slots, in;  // in: slot of the right end (0 or 1)
+  int t0, nb;        // the block's first step, its number of steps
+  double* pm;        // [K,T,M]
+  double* pP;        // [K,T,M,M]
+  double* smean;     // optional [K,T,D] smoothed state (return_full)
+  double* scov;      // optional [K,T,D,D]
+  double* scross;    // optional [K,T,D,D]: G_t P_s,t+1 = Cov(x_t, x_t+1 | y); Pinf at the last step
+};
+
+// first step of chunk c of a block
+__device__ inline int chunk_start(const StSmootherIO& io, int c) { return (int)((int64_t)io.nb * c / io.nc); }
+
+// The last step: the smoothed state is the filtered one (ops.py:314-315).
+template <int KT, int MB>
+__global__ __launch_bounds__(kT) void k_st_terminal(StDims dm, StHyp hy, const double* __restrict__ fmean,
+                                                    const double* __restrict__ fcov, StSmootherIO io) {
+  using S = StTiles<KT, MB>;
+  const int M = dm.M, D = dm.D, tid = threadIdx.x, k = blockIdx.x;
+  const int64_t kt = (int64_t)k * dm.T + dm.T - 1, DD = (int64_t)D * D;
+  const double* pk = fcov + kt * ((int64_t)D * (D + 1) / 2);
+  double* st = io.state + (int64_t)k * io.slots * S::STATE;
+  for (int e = tid; e < S::SYM; e += kT) {
+    int tile = e >> 8, r = 0;
+    while (tile > r) tile -= ++r;
+    const int l = (e & 255) >> 2, q = e & 3;
+    const int pi = 16 * r + (l >> 4) + 4 * q, pj = 16 * tile + (l & 15);
+    const int i = pi % S::MP, j = pj % S::MP, u = pi / S::MP * M + i, v = pj / S::MP * M + j;
+    st[e] = (i < M && j < M) ? pk[u <= v ? pidx(u, v, D) : pidx(v, u, D)] : 0.0;
+  }
+  for (int e = tid; e < S::DP; e += kT) {
+    const int i = e % S::MP;
+    st[S::SYM + e] = i < M ? fmean[kt * D + e / S::MP * M + i] : 0.0;
+  }
+  for (int e = tid; e < M; e += kT) io.pm[kt * M + e] = fmean[kt * D + e];
+  for (int e = tid; e < M * M; e += kT) {
+    const int i = e / M, j = e % M;
+    io.pP[kt * M * M + e] = pk[i <= j ? pidx(i, j, D) : pidx(j, i, D)];
+  }
+  if (io.smean) {
+    Model<KT, 0> mdl;
+    mdl.init(hy.ls_t[k * hy.stride], hy.var_t[k * hy.stride], 1.0, 1.0);
+    for (int e = tid; e < D; e += kT) io.smean[kt * D + e] = fmean[kt * D + e];
+    for (int64_t e = tid; e < DD; e += kT) {
+      const int i = (int)(e / D), j = (int)(e % D);
+      io.scov[kt * DD + e] = pk[i <= j ? pidx(i, j, D) : pidx(j, i, D)];
+      io.scross[kt * DD + e] = (i % M == j % M) ? mdl.Pinf[i / M][j / M] : 0.0;
+    }
+  }
+}
+
+// Product of the G_t of chunk blockIdx.x + 1, block per (chunk, run): E = G_first ... G_last,
+// from the last factor, with E' in LDS.
+template <int KT, int MB>
+__global__ __launch_bounds__(64 * KT * MB, 2) void k_st_chain(StSmootherIO io) {
+  using S = StTiles<KT, MB>;
+  constexpr int NR = S::NR, DP = S::DP, LD = S::LD, NF = S::NF;
+  extern __shared__ double X[];  // DP x LD: E'
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = blockIdx.x + 1, k = blockIdx.y;
+  const int s0 = chunk_start(io, c), s1 = chunk_start(io, c + 1);
+  const double* src = io.rec + (int64_t)k * io.tb * S::REC + w * 16 * DP + l;
+  double g[NF];
+  auto fetch = [&](int s) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) g[f] = src[(int64_t)s * S::REC + f * 64];
+  };
+  fetch(s1 - 1);
+#pragma unroll
+  for (int f = 0; f < NF; ++f) X[(4 * f + (l >> 4)) * LD + 16 * w + (l & 15)] = g[f];
+#pragma unroll 1
+  for (int s = s1 - 2; s >= s0; --s) {
+    fetch(s);
+    __syncthreads();
+    tile4 E[NR];
+#pragma unroll
+    for (int j = 0; j < NR; ++j) E[j] = tile_zero();
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) E[j] = mfma16(g[f], frag(X, LD, 16 * j, 4 * f, l), E[j]);
+      if (f % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NR; ++j) tile_store_t(X, LD, 16 * j, 16 * w, E[j], l);
+  }
+  __syncthreads();
+  double* out = io.comp + ((int64_t)k * io.nc + c) * S::REC + w * 16 * DP + l;
+#pragma unroll
+  for (int f = 0; f < NF; ++f) out[f * 64] = frag_t(X, LD, 4 * f, 16 * w, l);
+}
+
+enum { ST_WALK = 0, ST_COMPOSE = 1, ST_JOIN = 2 };
+
+// Per step T = G P_s' (G's row tile from registers, P_s' in LDS, both triangles) and
+// P_s = R + T G' (tiles j <= r; G in LDS, T through a staging tile): 51 k cycles of FP64 matrix
+// instructions a SIMD at D = 128, which bound it; the next step's G is on its way meanwhile.
+// 28 us a step, 35 with the outputs (89 us with both products through LDS panels of 8 columns);
+// one run of 1000 steps in 45 chunks: 3.3 ms for the whole pass, 90 ms walked as one chain.
+template <int KT, int MB, int MODE>
+__global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSmootherIO io) {
+  using S = StTiles<KT, MB>;
+  constexpr int MP = S::MP, NR = S::NR, DP = S::DP, LD = S::LD, NF = S::NF, NT = 64 * NR;
+  extern __shared__ double smem[];
+  double* X = smem;                  // DP x LD: P_s', then G
+  double* sT = X + DP * LD;          // NR of 16 x kDiagLd: staging tiles
+  double* ms = sT + DP * kDiagLd;    // 2 x DP: means, alternating
+  const int M = dm.M, D = dm.D, tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = S::row(w);
+  int l = tid & 63;
+  const int k = blockIdx.y;
+  const int c = MODE == ST_COMPOSE ? blockIdx.x + 1 : blockIdx.x;
+  const int s0 = MODE == ST_JOIN ? 1 : chunk_start(io, c), s1 = MODE == ST_JOIN ? io.nc : chunk_start(io, c + 1);
+  const double* rec = MODE == ST_JOIN ? io.comp + (int64_t)k * io.nc * S::REC : io.rec + (int64_t)k * io.tb * S::REC;
+  double* states = io.state + (int64_t)k * io.slots * S::STATE;
+  double* st = sT + w * 16 * kDiagLd;
+  tile4 P[NR];
+  if (MODE == ST_COMPOSE) {
+#pragma unroll
+    for (int j = 0; j < NR; ++j) P[j] = tile_zero();
+    for (int e = tid; e < DP; e += NT) ms[e] = 0.0;
+  } else {
+    const double* in = states + (MODE == ST_WALK && c + 1 < io.nc ? 2 + c : io.in) * S::STATE;
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) P[j] = tile_get(in + S::sym(r, j), l);
+    for (int e = tid; e < DP; e += NT) ms[e] = in[S::SYM + e];
+  }
+  double g[NF];
+  auto fetch = [&](int s) {
+    const double* src = rec + (int64_t)s * S::REC + r * 16 * DP + l;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) g[f] = src[f * 64];
+  };
+  auto publish = [&]() {  // P_s into LDS, both triangles
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) {
+        tile_store(X, LD, 16 * r, 16 * j, P[j], l);
+        if (j != r) tile_store_t(X, LD, 16 * j, 16 * r, P[j], l);
+      }
+  };
+  auto emit = [&](int s, const double* mean) {  // outputs of step s from LDS
+    const int64_t kt = (int64_t)k * dm.T + io.t0 + s;
+    for (int e = tid; e < M; e += NT) io.pm[kt * M + e] = mean[e];
+    for (int e = tid; e < M * M; e += NT) io.pP[kt * M * M + e] = X[(e / M) * LD + e % M];
+    if (io.smean) {
+      for (int e = tid; e < D; e += NT) io.smean[kt * D + e] = mean[e / M * MP + e % M];
+      for (int e = tid; e < D * D; e += NT) {
+        const int i = e / D, j = e % D;
+        io.scov[kt * D * D + e] = X[(i / M * MP + i % M) * LD + j / M * MP + j % M];
+      }
+    }
+  };
+  if (s0 < s1) fetch(s1 - 1);
+  int cur = 0;
+#pragma unroll 1
+  for (int s = s1 - 1; s >= s0; --s) {
+    l = fresh_v(l);
+    publish();
+    __syncthreads();
+    if (MODE == ST_WALK && s + 1 < s1) emit(s + 1, ms + cur * DP);
+    const double* rs = rec + (int64_t)s * S::REC + DP * DP;
+    tile4 T[NR];
+    double v = 0.0;
+#pragma unroll
+    for (int j = 0; j < NR; ++j) T[j] = tile_zero();
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) T[j] = mfma16(g[f], frag(X, LD, 16 * j, 4 * f, l), T[j]);
+      v = fma(g[f], ms[cur * DP + 4 * f + (l >> 4)], v);
+      if (f % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    }
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    cur ^= 1;
+    if (l < 16) ms[cur * DP + 16 * r + l] = rs[S::SYM + 16 * r + l] + v;
+    if (MODE == ST_WALK && io.scross) {
+      const int64_t kt = (int64_t)k * dm.T + io.t0 + s;
+#pragma unroll
+      for (int j = 0; j < NR; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int gi = 16 * (r % MB) + (l >> 4) + 4 * q, gj = 16 * (j % MB) + (l & 15);
+          if (gi < M && gj < M) io.scross[kt * D * D + (int64_t)(r / MB * M + gi) * D + j / MB * M + gj] = T[j][q];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) P[j] = tile_get(rs + S::sym(r, j), l);
+    __syncthreads();  // P_s' is read
+#pragma unroll
+    for (int f = 0; f < NF; ++f) X[(16 * r + (l & 15)) * LD + 4 * f + (l >> 4)] = g[f];
+    __syncthreads();  // G
+    l = fresh_v(l);
+    if (s > s0) fetch(s - 1);
+#pragma unroll
+    for (int b = 0; b < NR; ++b) {
+      double a[4];
+      tile_store(st, kDiagLd, 0, 0, T[b], l);
+      wave_sync();
+      frag4(a, st, kDiagLd, 0, 0, 1.0, l);
+      wave_sync();
+#pragma unroll
+      for (int j = 0; j < NR; ++j)
+        if (j <= r) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) P[j] = mfma16(a[e], frag(X, LD, 16 * j, 16 * b + 4 * e, l), P[j]);
+        }
+    }
+    __syncthreads();  // G is read
+    if (MODE == ST_JOIN) {  // the right end of chunk s - 1
+      double* o = states + (2 + s - 1) * S::STATE;
+#pragma unroll
+      for (int j = 0; j < NR; ++j)
+        if (j <= r) tile_put(o + S::sym(r, j), P[j], l);
+      for (int e = tid; e < DP; e += NT) o[S::SYM + e] = ms[cur * DP + e];
+    }
+  }
+  if (MODE == ST_WALK) {
+    publish();
+    __syncthreads();
+    if (s0 < s1) emit(s0, ms + cur * DP);
+  }
+  if (MODE == ST_COMPOSE || (MODE == ST_WALK && c == 0)) {
+    double* o = MODE == ST_COMPOSE ? io.comp + ((int64_t)k * io.nc + c) * S::REC + DP * DP
+                                   : states + (1 - io.in) * S::STATE;
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) tile_put(o + S::sym(r, j), P[j], l);
+    for (int e = tid; e < DP; e += NT) o[S::SYM + e] = ms[cur * DP + e];
+  }
+}
+
+// bytes of the block of maps: 2500 steps of one d = 128 run, 12 steps each of 200 runs
 constexpr int64_t kGainBudget = int64_t(512) << 20;
+// Workgroups that run side by side: one a compute unit (k_st_smoother fills a unit's LDS).
+constexpr int kUnits = 256;
+
+// doubles of one map / one state of the smoother (StTiles::REC, STATE)
+int64_t map_doubles(const StDims& dm) {
+  const int64_t nr = dm.KT * ((dm.M + 15) / 16), dp = 16 * nr;
+  return dp * dp + nr * (nr + 1) / 2 * 256 + dp;
+}
+int64_t state_doubles(const StDims& dm) {
+  const int64_t nr = dm.KT * ((dm.M + 15) / 16);
+  return nr * (nr + 1) / 2 * 256 + 16 * nr;
+}
 
 int gain_block_steps(const StDims& dm) {
-  const int64_t per = (int64_t)dm.K * 2 * dm.D * dm.D * (int64_t)sizeof(double);
-  int64_t tb = kGainBudget / (per > 0 ? per : 1);
+  const int64_t per = (int64_t)dm.K * map_doubles(dm) * (int64_t)sizeof(double);
+  int64_t tb = kGainBudget / per;
   const int64_t need = dm.T > 1 ? dm.T - 1 : 1;
   if (tb > need) tb = need;
   if (tb < 1) tb = 1;
   return (int)tb;
 }
 
-template <int KT>
-__global__ __launch_bounds__(kT) void k_st_gains(StDims dm, StHyp hy, StSmootherIO io, int t0) {
-  extern __shared__ double smem[];
-  const int M = dm.M, D = dm.D, tid = threadIdx.x;
-  const int j = blockIdx.x, k = blockIdx.y, t = t0 + j;
-  if (t >= dm.T - 1) return;  // uniform over the workgroup
-  double* pan = smem;                        // 2*kPK*kPS
-  double* sL = pan + 2 * kPK * kPS;          // D*D
-  double* row = sL + kMaxD * kMaxD;          // 2 D (pivot rows)
-  __shared__ double sA[KT * KT], sQ[KT * KT];
-  const int64_t DD = (int64_t)D * D, NSD = (int64_t)D * (D + 1) / 2;
-  const int64_t kt = (int64_t)k * dm.T + t;
-  double* F = io.buf + ((int64_t)k * io.tb + j) * 2 * DD;
-  double* G = F + DD;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  {
-    const double* pk = io.fcov + kt * NSD;
-    for (int i = tid >> 6; i < D; i += kT / 64)
-      for (int c = tid & 63; c < D; c += 64) F[(int64_t)i * D + c] = pk[i <= c ? pidx(i, c, D) : pidx(c, i, D)];
+// Chunks per run of a block of nb steps: the number with the shortest chain, 2 ceil(nb / c) + c - 1
+// steps (compose, join, walk) against nb for one chunk, as long as the two workgroups a chunk
+// takes in the compose step run side by side for all runs.
+int smoother_chunks(const StDims& dm, int nb) {
+  int best = 1, cost = nb;
+  for (int c = 2; c <= nb && 2 * (int64_t)c * dm.K <= kUnits; ++c) {
+    const int n = 2 * ((nb + c - 1) / c) + c - 1;
+    if (n < cost) { best = c; cost = n; }
   }
-  if (tid == 0) temporal_AQ<KT>(ls, var, io.dt[kt + 1], sA, sQ);
-  __syncthreads();
-  // P- = (A (x) I) F (A (x) I)' + Q (x) I, block (a, c) of M x M position pairs at a time
-  for (int e = tid; e < M * M; e += kT) {
-    const int a = e / M, c = e % M;
-    double f[KT][KT], af[KT][KT];
-    for (int p = 0; p < KT; ++p)
-      for (int q = 0; q < KT; ++q) f[p][q] = F[(int64_t)(p * M + a) * D + q * M + c];
-    for (int i = 0; i < KT; ++i)
-      for (int q = 0; q < KT; ++q) {
-        double v = 0.0;
-        for (int p = 0; p < KT; ++p) v = fma(sA[i * KT + p], f[p][q], v);
-        af[i][q] = v;
-      }
-    for (int i = 0; i < KT; ++i)
-      for (int jj = 0; jj < KT; ++jj) {
-        double v = (a == c) ? sQ[i * KT + jj] : 0.0;
-        for (int q = 0; q < KT; ++q) v = fma(af[i][q], sA[jj * KT + q], v);
-        sL[(int64_t)(i * M + a) * D + jj * M + c] = v;
-      }
-  }
-  (void)wg_sweep_inv<kMaxD / 16, false>(sL, D, D, row);  // sL = -(P-)^-1
-  // X = sL (A (x) I): columns {p M + a} of a row mix by A' (in place, one (row, a) per thread)
-  for (int e = tid; e < D * M; e += kT) {
-    const int r = e / M, a = e % M;
-    double x[KT];
-    for (int p = 0; p < KT; ++p) x[p] = sL[(int64_t)r * D + p * M + a];
-    for (int i = 0; i < KT; ++i) {
-      double v = 0.0;
-      for (int p = 0; p < KT; ++p) v = fma(x[p], sA[p * KT + i], v);
-      sL[(int64_t)r * D + i * M + a] = v;
-    }
-  }
-  // G' = (P-)^-1 (A (x) I) F = -X F
-  wg_gemm(D, D, D, -1.0, MatRef{sL, D, 1}, MatRef{F, D, 1}, 0.0, G, D, pan);
+  return best;
 }
-
-template <int KT>
-__global__ __launch_bounds__(kT) void k_st_smoother(StDims dm, StHyp hy, StSmootherIO io, int t1, int t0,
-                                                    int terminal) {
-  extern __shared__ double smem[];
-  const int M = dm.M, D = dm.D, tid = threadIdx.x;
-  const int k = blockIdx.x;
-  double* pan = smem;                        // 2*kPK*kPS
-  double* mf = pan + 2 * kPK * kPS;          // D
-  double* mp = mf + kMaxD;                   // D
-  double* dv = mp + kMaxD;                   // D
-  double* ms = dv + kMaxD;                   // D
-  __shared__ double sA[KT * KT], sQ[KT * KT];
-  const int64_t DD = (int64_t)D * D, NSD = (int64_t)D * (D + 1) / 2;
-  double* Ps = io.Ps + k * DD;
-  double* Dl = io.Dl + k * DD;
-  double* GT = io.GT + k * DD;
-  double* msg = io.ms + (int64_t)k * D;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  auto emit = [&](int64_t kt) {
-    for (int e = tid; e < M; e += kT) io.pm[kt * M + e] = ms[e];
-    for (int e = tid; e < M * M; e += kT) io.pP[kt * M * M + e] = Ps[(int64_t)(e / M) * D + e % M];
-    if (io.smean) {
-      for (int e = tid; e < D; e += kT) io.smean[kt * D + e] = ms[e];
-      for (int64_t e = tid; e < DD; e += kT) io.scov[kt * DD + e] = Ps[e];
-    }
-  };
-  if (terminal) {
-    // the last step: the smoothed state is the filtered one (ops.py:314-315)
-    const int64_t kt = (int64_t)k * dm.T + dm.T - 1;
-    const double* pk = io.fcov + kt * NSD;
-    for (int i = tid >> 6; i < D; i += kT / 64)
-      for (int c = tid & 63; c < D; c += 64) Ps[(int64_t)i * D + c] = pk[i <= c ? pidx(i, c, D) : pidx(c, i, D)];
-    for (int e = tid; e < D; e += kT) ms[e] = io.fmean[kt * D + e];
-    __syncthreads();
-    emit(kt);
-    if (io.scross) {
-      Model<KT, 0> mdl;
-      mdl.init(ls, var, 1.0, 1.0);
-      for (int64_t e = tid; e < DD; e += kT) {
-        const int i = (int)(e / D), j = (int)(e % D);
-        io.scross[kt * DD + e] = (i % M == j % M) ? mdl.Pinf[i / M][j / M] : 0.0;
-      }
-    }
-  } else {
-    for (int e = tid; e < D; e += kT) ms[e] = msg[e];
-  }
-  __syncthreads();
-  for (int t = t1; t >= t0; --t) {
-    const int64_t kt = (int64_t)k * dm.T + t;
-    const double* F = io.buf + ((int64_t)k * io.tb + (t - t0)) * 2 * DD;
-    const double* G = F + DD;  // G_t' (row-major)
-    for (int e = tid; e < D; e += kT) mf[e] = io.fmean[kt * D + e];
-    if (tid == 0) temporal_AQ<KT>(ls, var, io.dt[kt + 1], sA, sQ);
-    __syncthreads();
-    // Dl = sym(P_s') - P-, P- = (A (x) I) F (A (x) I)' + Q (x) I
-    for (int e = tid; e < M * M; e += kT) {
-      const int a = e / M, c = e % M;
-      double f[KT][KT], af[KT][KT];
-      for (int p = 0; p < KT; ++p)
-        for (int q = 0; q < KT; ++q) f[p][q] = F[(int64_t)(p * M + a) * D + q * M + c];
-      for (int i = 0; i < KT; ++i)
-        for (int q = 0; q < KT; ++q) {
-          double v = 0.0;
-          for (int p = 0; p < KT; ++p) v = fma(sA[i * KT + p], f[p][q], v);
-          af[i][q] = v;
-        }
-      for (int i = 0; i < KT; ++i)
-        for (int jj = 0; jj < KT; ++jj) {
-          double v = (a == c) ? sQ[i * KT + jj] : 0.0;
-          for (int q = 0; q < KT; ++q) v = fma(af[i][q], sA[jj * KT + q], v);
-          const int64_t o = (int64_t)(i * M + a) * D + jj * M + c;
-          const int64_t ot = (int64_t)(jj * M + c) * D + i * M + a;
-          Dl[o] = 0.5 * (Ps[o] + Ps[ot]) - v;  // symmetric part of the next step's P_s
-        }
-    }
-    if (tid < M) {
-      double x[KT];
-      for (int i = 0; i < KT; ++i) x[i] = mf[i * M + tid];
-      for (int i = 0; i < KT; ++i) {
-        double v = 0.0;
-        for (int p = 0; p < KT; ++p) v = fma(sA[i * KT + p], x[p], v);
-        mp[i * M + tid] = v;
-      }
-    }
-    // scross = G P_s' ; GT = G (P_s' - P-) ; P_s = P + GT G'
-    if (io.scross) wg_gemm(D, D, D, 1.0, MatRef{G, 1, D}, MatRef{Ps, D, 1}, 0.0, io.scross + kt * DD, D, pan);
-    wg_gemm(D, D, D, 1.0, MatRef{G, 1, D}, MatRef{Dl, D, 1}, 0.0, GT, D, pan);
-    for (int e = tid; e < D; e += kT) dv[e] = ms[e] - mp[e];
-    wg_gemm_128(D, D, D, 1.0, MatRef{GT, D, 1}, MatRef{G, D, 1}, 1.0, F, D, Ps, D, pan);
-    {  // m_s = m + G dv, the two halves of the workgroup split q; mp is free again
-      const int i = tid & (kMaxD - 1), h = tid / kMaxD;
-      double v = 0.0;
-      if (i < D)
-        for (int q = h; q < D; q += 2) v = fma(G[(int64_t)q * D + i], dv[q], v);
-      if (h == 1 && i < D) mp[i] = v;
-      __syncthreads();
-      if (h == 0 && i < D) ms[i] = mf[i] + v + mp[i];
-    }
-    __syncthreads();
-    emit(kt);
-    __syncthreads();
-  }
-  for (int e = tid; e < D; e += kT) msg[e] = ms[e];
+int smoother_max_chunks(const StDims& dm) {
+  const int64_t c = kUnits / (2 * (int64_t)dm.K);
+  return c > 1 ? (int)c : 1;
 }
 
 // per-run sums of per-step partials: out[k] = sum_t a[k*T + t]
@@ -2220,8 +2530,6 @@ __global__ __launch_bounds__(kT) void k_st_predict(StDims dm, StHyp hy, StPredIO
 }
 
 constexpr size_t kSmootherSmem = sizeof(double) * (2 * kPK * kPS + kMaxD * kMaxD + 6 * kMaxD);
-constexpr size_t kGainsSmem = sizeof(double) * (2 * kPK * kPS + kMaxD * kMaxD + 2 * kMaxD);
-constexpr size_t kSmootherSeqSmem = sizeof(double) * (2 * kPK * kPS + 4 * kMaxD);
 constexpr size_t kPseudoSmem = sizeof(double) * (2 * kPK * kPS + kMaxM * kMaxM + 3 * kMaxM);
 constexpr size_t kTiedSmem = sizeof(double) * (2 * kPK * kPS + kMaxM * kMaxM);
 constexpr size_t kIhDareSmem = sizeof(double) * (2 * kPK * kPS + 2 * kMaxM * kMaxM + 2 * kMaxM);
@@ -2247,13 +2555,24 @@ int check_dims(const bn_st_dims* d, StDims& dm) {
 
 StHyp make_hyp(const bn_st_hypers* h) { return StHyp{h->ls_t, h->var_t, h->var_s, h->stride}; }
 
+template <int KT, int MB>
+int smoother_attr() {
+  const int n = (int)sizeof(double) * StTiles<KT, MB>::SMEM;
+  for (const void* f : {(const void*)k_st_gains<KT, MB>, (const void*)k_st_chain<KT, MB>,
+                        (const void*)k_st_smoother<KT, MB, ST_WALK>, (const void*)k_st_smoother<KT, MB, ST_COMPOSE>,
+                        (const void*)k_st_smoother<KT, MB, ST_JOIN>})
+    ST_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, n));
+  return BN_OK;
+}
+
 // Dynamic LDS above the default limit is opted into once per kernel.
 int set_smem_limits() {
   static int done = 0;
   if (done) return BN_OK;
 #define ST_FILTER_ATTR(KT, MB)                                                                                  \
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_filter<KT, MB>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                   (int)sizeof(double) * filter_smem(KT, MB)))
+                                   (int)sizeof(double) * filter_smem(KT, MB)));                                        \
+  if (int rc = smoother_attr<KT, MB>()) return rc
   ST_FILTER_ATTR(1, 1);
   ST_FILTER_ATTR(1, 2);
   ST_FILTER_ATTR(1, 3);
@@ -2263,10 +2582,6 @@ int set_smem_limits() {
   ST_FILTER_ATTR(2, 3);
   ST_FILTER_ATTR(2, 4);
 #undef ST_FILTER_ATTR
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_gains<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kGainsSmem));
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_gains<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kGainsSmem));
 #define ST_SITES_ATTR1(MT, MD, KD)                                                                             \
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_sites<MT, MD, KD>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                    (int)kSitesSmem))
@@ -2325,6 +2640,44 @@ template <int KT>
 void launch_st_transitions(hipStream_t st, StDims dm, StHyp hy, const double* dt, double* aq) {
   const unsigned nb = (unsigned)(((int64_t)dm.K * dm.T + kT - 1) / kT);
   hipLaunchKernelGGL(k_st_transitions<KT>, dim3(nb), dim3(kT), 0, st, dm, hy, dt, aq);
+}
+
+// The backward pass over blocks of steps from the end of the runs.
+template <int KT, int MB>
+int launch_st_smoother(hipStream_t st, StDims dm, StHyp hy, const double* aq, const double* fmean, const double* fcov,
+                       StSmootherIO io) {
+  using S = StTiles<KT, MB>;
+  const unsigned nt = 64 * S::NR;
+  const size_t smem = sizeof(double) * S::SMEM;
+  hipLaunchKernelGGL((k_st_terminal<KT, MB>), dim3(dm.K), dim3(kT), 0, st, dm, hy, fmean, fcov, io);
+  for (int t1 = dm.T - 1; t1 > 0; t1 = io.t0) {  // steps [t0, t1)
+    io.t0 = t1 > io.tb ? t1 - io.tb : 0;
+    io.nb = t1 - io.t0;
+    io.nc = smoother_chunks(dm, io.nb);
+    const StGainIO gi{aq, fmean, fcov, io.rec, io.t0, io.tb};
+    hipLaunchKernelGGL((k_st_gains<KT, MB>), dim3(io.nb, dm.K), dim3(nt), smem, st, dm, gi);
+    if (io.nc > 1) {
+      hipLaunchKernelGGL((k_st_chain<KT, MB>), dim3(io.nc - 1, dm.K), dim3(nt), smem, st, io);
+      hipLaunchKernelGGL((k_st_smoother<KT, MB, ST_COMPOSE>), dim3(io.nc - 1, dm.K), dim3(nt), smem, st, dm, io);
+      hipLaunchKernelGGL((k_st_smoother<KT, MB, ST_JOIN>), dim3(1, dm.K), dim3(nt), smem, st, dm, io);
+    }
+    hipLaunchKernelGGL((k_st_smoother<KT, MB, ST_WALK>), dim3(io.nc, dm.K), dim3(nt), smem, st, dm, io);
+    ST_HIP_CHECK(hipGetLastError());
+    io.in = 1 - io.in;
+  }
+  return BN_OK;
+}
+
+template <int KT>
+int launch_st_smoother(hipStream_t st, StDims dm, StHyp hy, const double* dt, double* aq, const double* fmean,
+                       const double* fcov, StSmootherIO io) {
+  launch_st_transitions<KT>(st, dm, hy, dt, aq);
+  switch ((dm.M + 15) / 16) {
+    case 1: return launch_st_smoother<KT, 1>(st, dm, hy, aq, fmean, fcov, io);
+    case 2: return launch_st_smoother<KT, 2>(st, dm, hy, aq, fmean, fcov, io);
+    case 3: return launch_st_smoother<KT, 3>(st, dm, hy, aq, fmean, fcov, io);
+    default: return launch_st_smoother<KT, 4>(st, dm, hy, aq, fmean, fcov, io);
+  }
 }
 
 // k_st_sites<MT, MD> for the likelihood kind L.kind (checked by check_lik).
@@ -2457,12 +2810,13 @@ int bn_st_ep_sites(const bn_st_dims* dims, const bn_lik_desc* lik, int32_t mode,
 int64_t bn_st_workspace_bytes(const bn_st_dims* dims) {
   StDims dm;
   if (check_dims(dims, dm) != BN_OK) return -1;
-  // filter: the transitions (2 KT^2) and the determinant (2) of every step.  Smoother, per run: Ps, Dl, GT (3 x D x D) and
-  // m_s (D), then the block of gains and unpacked covariances (gain_block_steps)
-  const int64_t D = dm.D;
-  const int64_t smoother = 5 * D * D + 2 * D * D * gain_block_steps(dm);
-  const int64_t filter = 2 * ((int64_t)dm.KT * dm.KT + 1) * dm.T;
-  return (int64_t)dm.K * (smoother > filter ? smoother : filter) * (int64_t)sizeof(double) + 4096;
+  // per run: the transitions of every step (2 KT^2); then, for the filter, the determinant of every
+  // step (2) or, for the smoother, its states, chunk maps and block of maps
+  const int64_t nc = smoother_max_chunks(dm);
+  const int64_t smoother = (2 + nc) * state_doubles(dm) + (nc + gain_block_steps(dm)) * map_doubles(dm);
+  const int64_t filter = 2 * (int64_t)dm.T;
+  return (int64_t)dm.K * (2 * (int64_t)dm.KT * dm.KT * dm.T + (smoother > filter ? smoother : filter)) *
+             (int64_t)sizeof(double) + 4096;
 }
 
 int bn_st_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, const double* dt, const double* Lw,
@@ -2514,37 +2868,26 @@ int bn_st_smoother_full(const bn_st_dims* dims, const bn_st_hypers* hyp, const d
   if ((smooth_mean == nullptr) != (smooth_cov == nullptr) || (smooth_mean == nullptr) != (smooth_cross == nullptr))
     return st_fail(BN_EINVAL, "bn_st_smoother_full: smooth_mean, smooth_cov and smooth_cross go together");
   if (int rc = set_smem_limits()) return rc;
-  double* ws = (double*)workspace;
-  const int64_t D = dm.D, K = dm.K, DD = D * D;
-  const int tb = gain_block_steps(dm);
-  StSmootherIO io{dt, filter_mean, filter_cov, ws, ws + K * DD, ws + 2 * K * DD, ws + 3 * K * DD,
-                  ws + 5 * K * DD, tb, post_mean, post_cov, smooth_mean, smooth_cov, smooth_cross};
+  const int64_t K = dm.K;
+  const int nc = smoother_max_chunks(dm);
+  // transitions, states, chunk maps, the block's maps (bn_st_workspace_bytes)
+  double* aq = (double*)workspace;
+  StSmootherIO io{};
+  io.state = aq + K * dm.T * 2 * dm.KT * dm.KT;
+  io.slots = 2 + nc;
+  io.comp = io.state + K * io.slots * state_doubles(dm);
+  io.rec = io.comp + K * nc * map_doubles(dm);
+  io.tb = gain_block_steps(dm);
+  io.pm = post_mean;
+  io.pP = post_cov;
+  io.smean = smooth_mean;
+  io.scov = smooth_cov;
+  io.scross = smooth_cross;
   hipStream_t st = (hipStream_t)stream;
   const StHyp hy = make_hyp(hyp);
   BN_TIMED(KID_ST_SMOOTHER, st);
-  // blocks of steps from the end: gains of the block in parallel, then the recursion over it
-  int t1 = dm.T - 2;
-  bool terminal = true;
-  do {
-    const int t0 = t1 - tb + 1 > 0 ? t1 - tb + 1 : 0;
-    if (t1 >= 0) {
-      const dim3 g((unsigned)(t1 - t0 + 1), (unsigned)dm.K);
-      if (dm.KT == 1)
-        hipLaunchKernelGGL(k_st_gains<1>, g, dim3(kT), kGainsSmem, st, dm, hy, io, t0);
-      else
-        hipLaunchKernelGGL(k_st_gains<2>, g, dim3(kT), kGainsSmem, st, dm, hy, io, t0);
-    }
-    if (dm.KT == 1)
-      hipLaunchKernelGGL(k_st_smoother<1>, dim3(dm.K), dim3(kT), kSmootherSeqSmem, st, dm, hy, io, t1, t0,
-                         terminal ? 1 : 0);
-    else
-      hipLaunchKernelGGL(k_st_smoother<2>, dim3(dm.K), dim3(kT), kSmootherSeqSmem, st, dm, hy, io, t1, t0,
-                         terminal ? 1 : 0);
-    ST_HIP_CHECK(hipGetLastError());
-    terminal = false;
-    t1 = t0 - 1;
-  } while (t1 >= 0);
-  return BN_OK;
+  return dm.KT == 1 ? launch_st_smoother<1>(st, dm, hy, dt, aq, filter_mean, filter_cov, io)
+                    : launch_st_smoother<2>(st, dm, hy, dt, aq, filter_mean, filter_cov, io);
 }
 
 int bn_st_marginals(const bn_st_dims* dims, const double* B, const double* cdiag, const double* post_mean,

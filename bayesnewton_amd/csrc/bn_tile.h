@@ -61,6 +61,12 @@ __device__ inline void tile_store_t(double* X, int ld, int r0, int c0, tile4 v, 
   for (int q = 0; q < 4; ++q) p[4 * q] = v[q];
 }
 
+// sign times the four fragments of columns k0 .. k0 + 15
+__device__ inline void frag4(double (&a)[4], const double* X, int ld, int r0, int k0, double sign, int l) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) a[c] = sign * frag(X, ld, r0, k0 + 4 * c, l);
+}
+
 // c += A B' over one 16-wide block of the inner dimension: A rows r0.., B rows j0.., columns k0..
 __device__ inline tile4 tile_mul_t(const double* A, int lda, int r0, const double* B, int ldb, int j0, int ka, int kb,
                                    tile4 c, int l) {
@@ -75,14 +81,14 @@ __device__ inline double lane_bcast(double v, int lane) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-constexpr int kDiagLd = 18;  // row stride of a 16 x 16 block in LDS
+constexpr int kDiagLd = 18;  // row stride of a 16 x 16 block on its own in LDS
 
 // Cholesky factor of a 16 x 16 symmetric positive definite block and its inverse, by one
 // wavefront.  Lanes 0-15 start with the rows of A, the others with the columns of I; the
 // elimination step of pivot k, w_j -= l_jk w_k / sqrt(d), is the same instruction for both
 // (a Cholesky update of row r, a forward substitution of column c), with l_jk broadcast to
 // every lane through a scalar register.  16 pivots deep and latency bound.
-//   D (LDS, stride kDiagLd): A in (A's rows; only the lower triangle is read for the factor),
+//   D (LDS, row stride ld): A in (A's rows; only the lower triangle is read for the factor),
 //   L^-1 out (rows, zero above the diagonal).
 // L itself is not returned: the callers' row tiles get their factors as tile * L^-T.
 // A non-positive pivot gives NaN, which propagates.
@@ -90,13 +96,13 @@ constexpr int kDiagLd = 18;  // row stride of a 16 x 16 block in LDS
 // folded into the scaled column: w (y + y e (1/2 + 3/8 e)), e = 1 - d y^2.
 // Raised wave priority: the pivot chain competes for the FP64 pipe with the matrix
 // instructions of the wavefronts on the same SIMD, each of which holds it for 64 cycles.
-__device__ inline void chol16_inverse(double* D, int l) {
+__device__ inline void chol16_inverse(double* D, int ld, int l) {
   const int r = l & 15;
   double w[16];
   __builtin_amdgcn_s_setprio(3);
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const double a = D[r * kDiagLd + j];
+    const double a = D[r * ld + j];
     w[j] = l < 16 ? a : (j == r ? 1.0 : 0.0);
   }
 #pragma unroll
@@ -112,9 +118,14 @@ __device__ inline void chol16_inverse(double* D, int l) {
   wave_sync();
   if (l >= 16 && l < 32) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) D[j * kDiagLd + r] = w[j];  // column r of L^-1: zero above the diagonal
+    for (int j = 0; j < 16; ++j) D[j * ld + r] = w[j];  // column r of L^-1: zero above the diagonal
   }
   __builtin_amdgcn_s_setprio(0);
 }
+
+// A tile in memory: four consecutive doubles a lane (no alignment beyond a double's is assumed).
+typedef double tile4_mem __attribute__((ext_vector_type(4), aligned(8)));
+__device__ inline tile4 tile_get(const double* p, int l) { return *reinterpret_cast<const tile4_mem*>(p + 4 * l); }
+__device__ inline void tile_put(double* p, tile4 v, int l) { *reinterpret_cast<tile4_mem*>(p + 4 * l) = v; }
 
 }  // namespace bn

@@ -52,11 +52,38 @@ def test_inducing_points_around_tiles(M, kt):
     assert abs(float(gm.energy()) - om.energy()) <= TOL * abs(om.energy())
 
 
-@pytest.mark.parametrize("T", [1, 2, 3])
-def test_shortest_runs(T):
+@pytest.mark.parametrize("T", [1, 2, 3, 9, 10, 11, 40])
+def test_run_lengths_around_one_chunk(T):
+    """Up to 9 steps back one chunk is walked; longer runs are cut into chunks."""
     gm, om = _case(20, 2, T)
     gm.inference(lr=0.2)
     om.inference(lr=0.2)
     _close(gm.posterior_mean, om.posterior_mean)
     _close(gm.posterior_variance, om.posterior_variance)
     assert abs(float(gm.compute_log_lik()) - om.compute_log_lik()) <= TOL * abs(om.compute_log_lik())
+
+
+def test_many_runs_in_blocks_of_steps():
+    """130 runs of 24 steps at M = 64 go back in two blocks of steps, one chunk each; two runs in
+    one block of several chunks.  Same arithmetic up to the order of the covariance sums: 1e-10."""
+    from bayesnewton_amd import kernels as K, likelihoods as L, spacetime as S
+    g = np.linspace(0.0, 1.0, 8)
+    a, b = np.meshgrid(g, g)
+    z = np.stack([a.ravel(), b.ravel()], 1)
+    rng = np.random.default_rng(5)
+    T, nr = 24, 200
+    t = np.arange(T, dtype=np.float64)
+    r = rng.uniform(size=(2, T, nr, 2)).astype(np.float32).astype(np.float64)
+    y = rng.poisson(2.0 * np.exp(np.sin(4 * r[..., 0]))).astype(np.float64)
+    out = []
+    for n in (130, 2):
+        kern = K.SpatioTemporalKernel(K.Matern32(variance=1.0, lengthscale=8.0),
+                                      K.Matern32(variance=1.0, lengthscale=0.25), z=z)
+        idx = [i % 2 for i in range(n)]
+        m = S.SpaceTimeVariationalGP.from_runs(kern, L.Poisson(binsize=2.0), [t] * n, [r[i] for i in idx],
+                                               [y[i] for i in idx])
+        m.inference(lr=0.2, return_terms=False)
+        m.inference(lr=0.2, return_terms=False)
+        out.append((m.posterior_mean[-2:].cpu().numpy(), m.posterior_variance[-2:].cpu().numpy()))
+    for x, w in zip(*out):
+        assert np.max(np.abs(x - w)) <= 1e-10 * np.max(np.abs(w))
