@@ -316,32 +316,6 @@ __device__ double wg_sweep_inv(double* a, int n, int ld, double* row) {
   return logdet;
 }
 
-// In-place lower Cholesky of the n x n SPD matrix a (row stride ld, LDS), upper part zeroed.
-// A non-positive pivot gives NaN, which propagates (the reference's convention).
-__device__ void wg_chol(double* a, int n, int ld) {
-  const int tid = threadIdx.x;
-  __syncthreads();
-  for (int j = 0; j < n; ++j) {
-    const double d = sqrt(a[j * ld + j]);
-    const double id = 1.0 / d;
-    __syncthreads();  // every thread has read the pivot
-    for (int i = j + 1 + tid; i < n; i += kT) a[i * ld + j] *= id;
-    if (tid == 0) a[j * ld + j] = d;
-    __syncthreads();
-    const int r = n - j - 1;
-    for (int e = tid; e < r * r; e += kT) {
-      const int i = j + 1 + e / r, c = j + 1 + e % r;
-      if (c <= i) a[i * ld + c] = fma(-a[i * ld + j], a[c * ld + j], a[i * ld + c]);
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < n * n; e += kT) {
-    const int i = e / n, c = e % n;
-    if (c > i) a[i * ld + c] = 0.0;
-  }
-  __syncthreads();
-}
-
 // Forward substitution L X = B for `nrhs` right-hand-side columns, one thread per
 // column (L lower n x n in LDS with stride ld; B(i, c) = b[i*bs + c*bcs], solved in place).
 __device__ void wg_lower_solve(const double* L, int n, int ld, double* b, int bs, int bcs, int nrhs) {
@@ -536,11 +510,18 @@ constexpr int kRC = 32;  // rows of B per chunk
 constexpr int kLC = kMaxM + 1;  // LDS row stride of a chunk: consecutive rows start in different banks
 static_assert(2 * kRC * kLC >= kMaxM * kMaxM, "the two chunk buffers hold an M x M matrix");
 
+// The update and the projection for callers that go on to invert L L' explicitly
+// (k_mf_pseudo, the tied noise of the infinite-horizon form, the EP cavity): rounding in W and L
+// comes out of that inverse multiplied by the condition of W (1e6 and more on a grid of 64
+// inducing points), so W is summed over the locations in their order and factored pivot by
+// pivot, whatever the number of wavefronts.  k_st_sites is 1.7 times faster (one of two
+// launches 1.09 -> 0.45 ms at 4 runs of 500 steps, M = 64, R = 256) but rounds differently
+// in the last place, which moved mean-field posteriors by 1e-9 to 5e-9.
 // KIND: the likelihood as a compile-time constant (0: the projection, which has none);
 // with only its branch compiled, the site step spills a fraction of what it does with
 // every likelihood's code in the kernel.
 template <int METHOD, int MODE, int KIND>
-__global__ __launch_bounds__(kT, 3) void k_st_sites(StDims dm, LikParams lik, GHTable gh, StSiteIO io, double lr,
+__global__ __launch_bounds__(kT, 3) void k_st_sites_ordered(StDims dm, LikParams lik, GHTable gh, StSiteIO io, double lr,
                                                  int ensure_psd, double power, int mask_pseudo) {
   extern __shared__ double smem[];
   if (KIND != 0) lik.kind = KIND;
@@ -561,7 +542,6 @@ __global__ __launch_bounds__(kT, 3) void k_st_sites(StDims dm, LikParams lik, GH
   const int64_t kt = (int64_t)k * dm.T + t;
   const int LC = M + 1;
   constexpr bool UPDATE = MODE == BN_ST_UPDATE;
-  constexpr bool PROJECT = MODE != BN_ST_ENERGY;
   constexpr bool SITES = MODE != BN_ST_PROJECT;
   const double* gP = io.pP + kt * M * M;
   double* gW = io.Lw + kt * M * M;
@@ -609,16 +589,10 @@ __global__ __launch_bounds__(kT, 3) void k_st_sites(StDims dm, LikParams lik, GH
             io.o_jac[s] = (float)sr.jac;
             io.o_hess[s] = (float)sr.hess;
           }
-        } else if (METHOD == M_EP) {
-          acc0 += ep_lel_from_cavity(lik, gh, yv, mf, vf, power);
-        } else {
-          double t1, t2;
-          energy_terms<METHOD>(lik, gh, yv, mf, vf, 1.0, 1.0, 1.0, t1, t2);
-          acc0 += t1;
         }
       }
     }
-    if (PROJECT) {
+    {
       __syncthreads();
       // X = diag(nat2) C (rows of the chunk), v += C' nat1, W += C' X
       for (int e = tid; e < kRC * M; e += kT) {
@@ -639,7 +613,7 @@ __global__ __launch_bounds__(kT, 3) void k_st_sites(StDims dm, LikParams lik, GH
     const double d1 = wg_sum(acc0, red), d2 = wg_sum(acc1, red);
     if (tid == 0) { io.part0[kt] = d1; io.part1[kt] = d2; }
   }
-  if (PROJECT) {
+  {
     __syncthreads();
     for (int e = tid; e < M * M; e += kT) sW[e] = gW[e] + ((e / M == e % M) ? kPseudoJitter : 0.0);
     const double ld = wg_chol_reg<kMaxM / 16>(sW, M, M, row);
@@ -648,24 +622,356 @@ __global__ __launch_bounds__(kT, 3) void k_st_sites(StDims dm, LikParams lik, GH
     for (int e = tid; e < M * M; e += kT) Lo[e] = sW[e];
     for (int e = tid; e < M; e += kT) io.zw[kt * M + e] = sv[e];
     if (tid == 0) io.ldl[kt] = ld;
+  }
+}
+
+constexpr int kSLd = kMaxM + 2;  // row stride of the site kernel's LDS matrices
+constexpr int kWT = 10;          // tiles (i, j <= i) of a 64 x 64 symmetric matrix
+
+// Sums x[0..3] over the 16 lanes of a row of lanes; lane c of the row gets the sum of x[c / 4].
+__device__ inline double row_sums4(const double (&x)[4], int l) {
+  const bool h = l & 8, m = l & 4;
+  double a = h ? x[2] : x[0], b = h ? x[3] : x[1];
+  a += __shfl_xor(h ? x[0] : x[2], 8, 64);
+  b += __shfl_xor(h ? x[1] : x[3], 8, 64);
+  double s = m ? b : a;
+  s += __shfl_xor(m ? a : b, 4, 64);
+  s += __shfl_xor(s, 2, 64);
+  s += __shfl_xor(s, 1, 64);
+  return s;
+}
+
+// A L^-T for a row tile A, into X (row stride ld) and returned: the product with the explicit
+// inverse I of the diagonal block, then one step of refinement with the block's factor L (row
+// stride kSLd).  Without it L L' would miss W by the condition of the diagonal blocks (16
+// neighbouring inducing points) times the rounding unit, which the mean-field form's explicit
+// inverse of L L' amplifies.
+__device__ inline tile4 solve_tile(double* X, int ld, const double* I, const double* L, tile4 A, int l) {
+  double a[4];
+  tile_store(X, ld, 0, 0, A, l);
+  wave_sync();
+  tile4 v = tile_mul_t(X, ld, 0, I, kDiagLd, 0, 0, 0, tile_zero(), l);
+  wave_sync();
+  tile_store(X, ld, 0, 0, v, l);
+  wave_sync();
+  frag4(a, X, ld, 0, 0, -1.0, l);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) A = mfma16(a[c], frag(L, kSLd, 0, 4 * c, l), A);
+  wave_sync();
+  tile_store(X, ld, 0, 0, A, l);
+  wave_sync();
+  v = tile_mul_t(X, ld, 0, I, kDiagLd, 0, 0, 0, v, l);
+  wave_sync();
+  tile_store(X, ld, 0, 0, v, l);
+  wave_sync();
+  return v;
+}
+
+// KIND: the likelihood as a compile-time constant (0: the projection, which has none).
+//
+// A wavefront works through 16 rows of B at a time on its own: X = C P with P's lower tiles only
+// (diag(C P C') = sum_j C_ij (C_j P_jj + 2 sum_k>j C_k P_kj)_ij), the site step of the 16
+// locations, and its share of the lower tiles of W = B' diag(nat2) B in registers; the four
+// wavefronts meet for the sum of W and its blocked Cholesky factorisation (chol16_inverse).
+// 71 KB of LDS, two workgroups a CU, so that one's factorisation runs under the other's
+// products.  Bound by the FP64 matrix instructions (20 k cycles a SIMD a step at M = 64, R = 256)
+// and the four pivot chains.
+template <int METHOD, int MODE, int KIND>
+__global__ __launch_bounds__(kT, 2) void k_st_sites(StDims dm, LikParams lik, GHTable gh, StSiteIO io, double lr,
+                                                 int ensure_psd, double power, int mask_pseudo) {
+  extern __shared__ double smem[];
+  if (KIND != 0) lik.kind = KIND;
+  const int M = dm.M, R = dm.R, MB = (M + 15) / 16;
+  double* sP = smem;                      // kMaxM x kSLd: posterior covariance; partial sums of W; Lm
+  double* sB = sP + kMaxM * kSLd;         // 4 x 16 x kSLd: the wavefronts' rows of B; partial sums of W; L (ENERGY)
+  double* sI = sB;                        // 4 x 16 x kDiagLd: diagonal blocks, then their inverse factors
+  double* sG = sI + 4 * 16 * kDiagLd;     // 16 x kDiagLd: row tile of v' (both once W is summed)
+  double* sm = sB + kMaxM * kSLd;         // kMaxM: posterior mean
+  double* sv = sm + kMaxM;                // 4 x kMaxM: the wavefronts' parts of v = B' nat1; z
+  double* sn = sv + 4 * kMaxM;            // 4 x 2 x 16: new nat1, nat2 of the wavefronts' rows
+  double* red = sn + 4 * 32;              // 4
+  const int t = blockIdx.x, k = blockIdx.y, tid = threadIdx.x;
+  int l = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t kt = (int64_t)k * dm.T + t;
+  constexpr bool UPDATE = MODE == BN_ST_UPDATE;
+  constexpr bool PROJECT = MODE != BN_ST_ENERGY;
+  constexpr bool SITES = MODE != BN_ST_PROJECT;
+  // mini-batch (inference.py:65-90, group_natural_params basemodels.py:195-199): a step
+  // outside it keeps its sites and adds no data term; its projection is still formed
+  const bool in_batch = io.batch == nullptr || io.batch[kt] != 0.0f;
+  double* cB = sB + w * 16 * kSLd;
+  double* cn = sn + w * 32;
+  const int RT = (R + 15) / 16;
+  double pre[16];  // the next 16 rows of B, one column a lane
+  auto fetch = [&](int rt) {
+    const double* src = io.B + (kt * R + 16 * rt) * M + l;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const bool on = l < M && 16 * rt + i < R;
+      const double v = *(on ? src + i * M : io.B);
+      pre[i] = on ? v : 0.0;
+    }
+  };
+  if (w < RT) fetch(w);
+  if (SITES) {
+    const double* gP = io.pP + kt * M * M;
+#pragma unroll 4
+    for (int i = w; i < 16 * MB; i += 4) sP[i * kSLd + l] = (i < M && l < M) ? gP[i * M + l] : 0.0;
+    if (tid < kMaxM) sm[tid] = tid < M ? io.pm[kt * M + tid] : 0.0;
+  }
+  __syncthreads();
+  tile4 W[kWT];
+  double va[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int i = 0; i < kWT; ++i) W[i] = tile_zero();
+  double acc0 = 0.0, acc1 = 0.0;
+#pragma unroll 1
+  for (int rt = w; rt < RT; rt += 4) {
+    l = fresh_v(l);
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) cB[i * kSLd + l] = pre[i];
+    // the lane's location in the site step: row l/16 + 4 ((l%16) / 4), the first of four lanes writes
+    const int row = (l >> 4) + (l & 12), at = 16 * rt + row;
+    const bool mine = (l & 3) == 0 && at < R;
+    const int64_t s = kt * R + (at < R ? at : 0);
+    double n1 = 0.0, n2 = 0.0, cd = 0.0, yv = 0.0;
+    if (MODE != BN_ST_ENERGY) {
+      n1 = io.nat1[s];
+      n2 = io.nat2[s];
+    }
+    if (SITES) {
+      cd = io.cdiag[s];
+      yv = (double)io.y[s];
+    }
+    if (rt + 4 < RT) fetch(rt + 4);
+    wave_sync();
+    if (SITES) {
+      tile4 X[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) X[j] = tile_zero();
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        if (kk < MB) {
+          double a[4];
+          frag4(a, cB, kSLd, 0, 16 * kk, 1.0, l);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) X[kk] = mfma16(a[c], frag(sP, kSLd, 16 * kk, 16 * kk + 4 * c, l), X[kk]);
+#pragma unroll
+          for (int j = 0; j < kk; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) X[j] = mfma16(2.0 * a[c], frag(sP, kSLd, 16 * j, 16 * kk + 4 * c, l), X[j]);
+        }
+      double mq[4] = {0.0, 0.0, 0.0, 0.0}, vq[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < MB) {
+          const double mj = sm[16 * j + (l & 15)];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const double c = cB[((l >> 4) + 4 * q) * kSLd + 16 * j + (l & 15)];
+            mq[q] = fma(c, mj, mq[q]);
+            vq[q] = fma(c, X[j][q], vq[q]);
+          }
+        }
+      const double mf = row_sums4(mq, l), vf = cd + row_sums4(vq, l);
+      if (!in_batch || !mine) {
+      } else if (UPDATE) {
+        // EP: (pm, pP) is the cavity of the inducing states, so (mf, vf) is the cavity at the data
+        SiteResult sr = METHOD == M_EP ? ep_site_from_cavity(lik, gh, yv, mf, vf, power, mask_pseudo != 0,
+                                                             ensure_psd != 0)
+                                       : site_step<METHOD>(lik, gh, yv, mf, vf, n1, n2, 1.0, ensure_psd != 0);
+        acc0 += fabs(sr.nat1 - n1);
+        acc1 += fabs(sr.nat2 - n2);
+        n1 = (1.0 - lr) * n1 + lr * sr.nat1;
+        n2 = (1.0 - lr) * n2 + lr * sr.nat2;
+        io.nat1[s] = n1;
+        io.nat2[s] = n2;
+        if (io.o_mean != nullptr) {
+          io.o_mean[s] = (float)sr.mean;
+          io.o_jac[s] = (float)sr.jac;
+          io.o_hess[s] = (float)sr.hess;
+        }
+      } else if (METHOD == M_EP) {
+        acc0 += ep_lel_from_cavity(lik, gh, yv, mf, vf, power);
+      } else {
+        double t1, t2;
+        energy_terms<METHOD>(lik, gh, yv, mf, vf, 1.0, 1.0, 1.0, t1, t2);
+        acc0 += t1;
+      }
+    }
+    if (PROJECT) {
+      if ((l & 3) == 0) {
+        cn[row] = at < R ? n1 : 0.0;
+        cn[16 + row] = at < R ? n2 : 0.0;
+      }
+      wave_sync();
+#pragma unroll
+      for (int c = 0; c < 16; c += 4) {
+        const double e1 = cn[c + (l >> 4)], e2 = cn[16 + c + (l >> 4)];
+        double f[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f[j] = j < MB ? frag_t(cB, kSLd, c, 16 * j, l) : 0.0;
+          va[j] = fma(f[j], e1, va[j]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (i < MB) {
+#pragma unroll
+            for (int j = 0; j <= i; ++j) W[i * (i + 1) / 2 + j] = mfma16(f[i], e2 * f[j], W[i * (i + 1) / 2 + j]);
+          }
+      }
+    }
+  }
+  if (UPDATE) {
+    const double d1 = wg_sum(acc0, red), d2 = wg_sum(acc1, red);
+    if (tid == 0) { io.part0[kt] = d1; io.part1[kt] = d2; }
+  }
+  if (PROJECT) {
+    // sum of the wavefronts' parts: 0 + 2 and 1 + 3, then the two
+    constexpr int kPart = kWT * 256;
+    static_assert(2 * kPart <= 2 * kMaxM * kSLd, "two partial sums of W fit the covariance's and the rows' space");
+    __syncthreads();
+    l = fresh_v(l);
+    double* part = sP + (w & 1) * kPart;
+    if (w >= 2) {
+#pragma unroll
+      for (int i = 0; i < kWT; ++i) tile_put(part + i * 256, W[i], l);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      va[j] += __shfl_xor(va[j], 16, 64);
+      va[j] += __shfl_xor(va[j], 32, 64);
+      if (l < 16) sv[w * kMaxM + 16 * j + l] = va[j];
+    }
+    __syncthreads();
+    if (w < 2) {
+#pragma unroll
+      for (int i = 0; i < kWT; ++i) {
+        W[i] += tile_get(part + i * 256, l);
+        tile_put(part + i * 256, W[i], l);
+      }
+    }
+    __syncthreads();
+    // row tile w of W + 1e-12 I (identity padding); wavefront 0 also takes v' as a row tile
+    tile4 V[4], Z[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      V[j] = tile_zero();
+      Z[j] = tile_zero();
+      if (j <= w && w < MB) {
+        const int o = (w * (w + 1) / 2 + j) * 256;
+        V[j] = tile_get(sP + o, l) + tile_get(sP + kPart + o, l);
+      }
+      const int e = 16 * j + (l & 15);
+      if (w == 0) Z[j][0] = l < 16 ? (sv[e] + sv[2 * kMaxM + e]) + (sv[kMaxM + e] + sv[3 * kMaxM + e]) : 0.0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (j == w && (l >> 4) + 4 * q == (l & 15)) V[j][q] += e < M ? kPseudoJitter : 1.0;
+    }
+    __syncthreads();
+    double* Lm = sP;
+    for (int e = tid; e < 16 * kDiagLd; e += kT) sG[e] = 0.0;
+    if (w == 0) {
+      tile_store(sI, kDiagLd, 0, 0, V[0], l);
+      wave_sync();
+      chol16_inverse<true>(sI, kDiagLd, l, Lm, kSLd);
+    }
+#pragma unroll 1
+    for (int b = 0; b < MB; ++b) {
+      const double* Ib = sI + b * 16 * kDiagLd;
+      __syncthreads();  // inverse factor of diagonal block b
+      l = fresh_v(l);
+      if (w > b && w < MB) {
+        solve_tile(Lm + 16 * w * kSLd + 16 * b, kSLd, Ib, Lm + 16 * b * kSLd + 16 * b, V[0], l);
+        if (w == b + 1) {  // the next diagonal block first
+          double a[4];
+          frag4(a, Lm, kSLd, 16 * w, 16 * b, 1.0, l);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) V[1] = mfma16(-a[c], a[c], V[1]);
+          tile_store(sI + (b + 1) * 16 * kDiagLd, kDiagLd, 0, 0, V[1], l);
+        }
+      } else if (w == 0) {
+        const tile4 v = solve_tile(sG, kDiagLd, Ib, Lm + 16 * b * kSLd + 16 * b, Z[0], l);
+        if (l < 16) sm[16 * b + l] = v[0];  // z
+      }
+      __syncthreads();  // column block b of Lm
+      l = fresh_v(l);
+      if (b + 1 < MB) {
+        if (w == b + 1) {
+          chol16_inverse<true>(sI + w * 16 * kDiagLd, kDiagLd, l, Lm + 16 * w * kSLd + 16 * w, kSLd);
+        } else if ((w > b + 1 && w < MB) || w == 0) {
+          double a[4];
+          frag4(a, w == 0 ? sG : Lm + 16 * w * kSLd + 16 * b, w == 0 ? kDiagLd : kSLd, 0, 0, -1.0, l);
+#pragma unroll
+          for (int j = 1; j < 4; ++j)
+            if (b + j < MB) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) {
+                const double f = frag(Lm, kSLd, 16 * (b + j), 16 * b + 4 * c, l);
+                if (w == 0) Z[j] = mfma16(a[c], f, Z[j]);
+                else V[j] = mfma16(a[c], f, V[j]);
+              }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) { V[j] = V[j + 1]; Z[j] = Z[j + 1]; }
+      }
+    }
+    __syncthreads();
+    double* Lo = io.Lw + kt * M * M;
+    for (int i = w; i < M; i += 4)
+      if (l < M) Lo[i * M + l] = (l >> 4) > (i >> 4) ? 0.0 : Lm[i * kSLd + l];
+    if (tid < M) io.zw[kt * M + tid] = sm[tid];
+    if (w == 3) {
+      double ld = l < M ? -log(sI[(l >> 4) * 16 * kDiagLd + (l & 15) * (kDiagLd + 1)]) : 0.0;
+      for (int o = 32; o > 0; o >>= 1) ld += __shfl_xor(ld, o, 64);
+      if (l == 0) io.ldl[kt] = ld;
+    }
   } else if (METHOD == M_EP) {
     // the pseudo term (lel_pseudo) comes from k_st_ep_cavity
     const double e1 = wg_sum(acc0, red);
     if (tid == 0) io.part0[kt] = e1;
   } else {
-    const double e1 = wg_sum(acc0, red);
     // whitened expected density of the pseudo observation:
-    // |z - L' m|^2 and tr(L' P L) = sum_ac L(a,c) (P L)(a,c), L in LDS (sW), P L in sX
+    // |z - L' m|^2 and tr(L' P L) = sum_ac L(a,c) (P L)(a,c)
     const double* L = io.Lw + kt * M * M;
-    const double* z = io.zw + kt * M;
+    const double e1 = wg_sum(acc0, red);  // every wavefront has read its rows of B
+#pragma unroll 4
+    for (int i = w; i < 16 * MB; i += 4) sB[i * kSLd + l] = (i < M && l < M) ? L[i * M + l] : 0.0;
+    __syncthreads();
+    l = fresh_v(l);
     double q2 = 0.0, tr = 0.0;
     if (tid < M) {
-      double u = z[tid];
-      for (int a = tid; a < M; ++a) u = fma(-L[a * M + tid], sm[a], u);   // (z - L' m)_tid
+      double u = io.zw[kt * M + tid];
+#pragma unroll 4
+      for (int a = tid; a < M; ++a) u = fma(-sB[a * kSLd + tid], sm[a], u);  // (z - L' m)_tid
       q2 = u * u;
     }
-    wg_gemm_small(M, M, M, 1.0, MatRef{gP, M, 1}, MatRef{L, M, 1}, 0.0, sW, M, pan);  // P L
-    for (int e = tid; e < M * M; e += kT) tr = fma(L[e], sW[e], tr);
+    if (w < MB) {
+      tile4 X[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) X[j] = tile_zero();
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        if (kk < MB) {
+#pragma unroll
+          for (int c = 0; c < 16; c += 4) {
+            const double a = frag(sP, kSLd, 16 * w, 16 * kk + c, l);
+#pragma unroll
+            for (int j = 0; j <= kk; ++j) X[j] = mfma16(a, frag_t(sB, kSLd, 16 * kk + c, 16 * j, l), X[j]);
+          }
+        }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < MB) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            tr = fma(sB[(16 * w + (l >> 4) + 4 * q) * kSLd + 16 * j + (l & 15)], X[j][q], tr);
+        }
+    }
     const double Q2 = wg_sum(q2, red), TR = wg_sum(tr, red);
     if (tid == 0) {
       io.part0[kt] = e1;
@@ -2534,6 +2840,9 @@ constexpr size_t kPseudoSmem = sizeof(double) * (2 * kPK * kPS + kMaxM * kMaxM +
 constexpr size_t kTiedSmem = sizeof(double) * (2 * kPK * kPS + kMaxM * kMaxM);
 constexpr size_t kIhDareSmem = sizeof(double) * (2 * kPK * kPS + 2 * kMaxM * kMaxM + 2 * kMaxM);
 constexpr size_t kSitesSmem =
+    sizeof(double) * (2 * kMaxM * kSLd + 5 * kMaxM + 4 * 32 + 4);
+static_assert(2 * kSitesSmem <= 160 * 1024, "two workgroups of k_st_sites a CU");
+constexpr size_t kOrderedSmem =
     sizeof(double) * (2 * kPK * kPS + 2 * kRC * kLC + 2 * kMaxM + kRC + 2 * kMaxM + 4);
 constexpr size_t kCavitySmem = sizeof(double) * (2 * kPK * kPS + 2 * kMaxM * kMaxM + 4 * kMaxM + 4);
 
@@ -2582,14 +2891,13 @@ int set_smem_limits() {
   ST_FILTER_ATTR(2, 3);
   ST_FILTER_ATTR(2, 4);
 #undef ST_FILTER_ATTR
-#define ST_SITES_ATTR1(MT, MD, KD)                                                                             \
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_sites<MT, MD, KD>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                   (int)kSitesSmem))
-#define ST_SITES_ATTR(MT, MD)                 \
-  ST_SITES_ATTR1(MT, MD, LIK_GAUSSIAN);        \
-  ST_SITES_ATTR1(MT, MD, LIK_BERNOULLI_PROBIT); \
-  ST_SITES_ATTR1(MT, MD, LIK_POISSON);         \
-  ST_SITES_ATTR1(MT, MD, LIK_STUDENTS_T)
+#define ST_SITES_ATTR1(KERNEL, MT, MD, KD, N)                                                                       \
+  ST_HIP_CHECK(hipFuncSetAttribute((const void*)KERNEL<MT, MD, KD>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)N))
+#define ST_SITES_ATTR(KERNEL, MT, MD, N)                    \
+  ST_SITES_ATTR1(KERNEL, MT, MD, LIK_GAUSSIAN, N);          \
+  ST_SITES_ATTR1(KERNEL, MT, MD, LIK_BERNOULLI_PROBIT, N);  \
+  ST_SITES_ATTR1(KERNEL, MT, MD, LIK_POISSON, N);           \
+  ST_SITES_ATTR1(KERNEL, MT, MD, LIK_STUDENTS_T, N)
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_mf_pseudo, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kPseudoSmem));
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_dare<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2600,13 +2908,16 @@ int set_smem_limits() {
                                    (int)kSmootherSmem));
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_smoother<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kSmootherSmem));
-  ST_SITES_ATTR(M_VI, BN_ST_UPDATE);
-  ST_SITES_ATTR(M_VI, BN_ST_ENERGY);
-  ST_SITES_ATTR1(M_VI, BN_ST_PROJECT, 0);
-  ST_SITES_ATTR(M_NEWTON, BN_ST_UPDATE);
-  ST_SITES_ATTR(M_NEWTON, BN_ST_ENERGY);
-  ST_SITES_ATTR(M_EP, BN_ST_UPDATE);
-  ST_SITES_ATTR(M_EP, BN_ST_ENERGY);
+  ST_SITES_ATTR(k_st_sites, M_VI, BN_ST_UPDATE, kSitesSmem);
+  ST_SITES_ATTR(k_st_sites, M_VI, BN_ST_ENERGY, kSitesSmem);
+  ST_SITES_ATTR1(k_st_sites, M_VI, BN_ST_PROJECT, 0, kSitesSmem);
+  ST_SITES_ATTR(k_st_sites, M_NEWTON, BN_ST_UPDATE, kSitesSmem);
+  ST_SITES_ATTR(k_st_sites, M_NEWTON, BN_ST_ENERGY, kSitesSmem);
+  ST_SITES_ATTR(k_st_sites, M_EP, BN_ST_ENERGY, kSitesSmem);
+  ST_SITES_ATTR(k_st_sites_ordered, M_VI, BN_ST_UPDATE, kOrderedSmem);
+  ST_SITES_ATTR1(k_st_sites_ordered, M_VI, BN_ST_PROJECT, 0, kOrderedSmem);
+  ST_SITES_ATTR(k_st_sites_ordered, M_NEWTON, BN_ST_UPDATE, kOrderedSmem);
+  ST_SITES_ATTR(k_st_sites_ordered, M_EP, BN_ST_UPDATE, kOrderedSmem);
 #undef ST_SITES_ATTR
 #undef ST_SITES_ATTR1
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_st_ep_cavity<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2680,28 +2991,75 @@ int launch_st_smoother(hipStream_t st, StDims dm, StHyp hy, const double* dt, do
   }
 }
 
-// k_st_sites<MT, MD> for the likelihood kind L.kind (checked by check_lik).
+// k_st_sites / k_st_sites_ordered for the likelihood kind L.kind (checked by check_lik).
+#define ST_SITES_LAUNCH(KERNEL, KD, N)                                                                              \
+  hipLaunchKernelGGL((KERNEL<MT, MD, KD>), grid, dim3(kT), N, st, dm, L, gh, io, lr, ensure_psd, power, mask_pseudo)
+#define ST_SITES_SWITCH(KERNEL, N)                                                        \
+  switch (L.kind) {                                                                       \
+    case LIK_GAUSSIAN: ST_SITES_LAUNCH(KERNEL, LIK_GAUSSIAN, N); break;                   \
+    case LIK_BERNOULLI_PROBIT: ST_SITES_LAUNCH(KERNEL, LIK_BERNOULLI_PROBIT, N); break;   \
+    case LIK_POISSON: ST_SITES_LAUNCH(KERNEL, LIK_POISSON, N); break;                     \
+    default: ST_SITES_LAUNCH(KERNEL, LIK_STUDENTS_T, N); break;                           \
+  }
 template <int MT, int MD>
 void launch_st_sites(dim3 grid, hipStream_t st, StDims dm, LikParams L, GHTable gh, StSiteIO io, double lr,
                      int ensure_psd, double power, int mask_pseudo) {
-  switch (L.kind) {
-    case LIK_GAUSSIAN:
-      hipLaunchKernelGGL((k_st_sites<MT, MD, LIK_GAUSSIAN>), grid, dim3(kT), kSitesSmem, st, dm, L, gh, io, lr,
-                         ensure_psd, power, mask_pseudo);
-      break;
-    case LIK_BERNOULLI_PROBIT:
-      hipLaunchKernelGGL((k_st_sites<MT, MD, LIK_BERNOULLI_PROBIT>), grid, dim3(kT), kSitesSmem, st, dm, L, gh, io,
-                         lr, ensure_psd, power, mask_pseudo);
-      break;
-    case LIK_POISSON:
-      hipLaunchKernelGGL((k_st_sites<MT, MD, LIK_POISSON>), grid, dim3(kT), kSitesSmem, st, dm, L, gh, io, lr,
-                         ensure_psd, power, mask_pseudo);
-      break;
-    default:
-      hipLaunchKernelGGL((k_st_sites<MT, MD, LIK_STUDENTS_T>), grid, dim3(kT), kSitesSmem, st, dm, L, gh, io, lr,
-                         ensure_psd, power, mask_pseudo);
-      break;
+  ST_SITES_SWITCH(k_st_sites, kSitesSmem)
+}
+template <int MT>
+void launch_st_update_ordered(dim3 grid, hipStream_t st, StDims dm, LikParams L, GHTable gh, StSiteIO io, double lr,
+                              int ensure_psd, double power, int mask_pseudo) {
+  constexpr int MD = BN_ST_UPDATE;
+  ST_SITES_SWITCH(k_st_sites_ordered, kOrderedSmem)
+}
+#undef ST_SITES_SWITCH
+#undef ST_SITES_LAUNCH
+
+// bn_st_sites (whitened = false) and bn_st_sites_whitened.
+int st_sites(bool whitened, const bn_st_dims* dims, const bn_lik_desc* lik, int32_t method, int32_t mode,
+             int32_t gh_points, double lr, int32_t ensure_psd, const float* y, const double* B, const double* cdiag,
+             const double* post_mean, const double* post_cov, const float* batch, double* nat1, double* nat2,
+             double* Lw, double* zw, double* ldl, double* part0, double* part1, float* out_mean, float* out_jac,
+             float* out_hess, void* stream) {
+  StDims dm;
+  if (int rc = check_dims(dims, dm)) return rc;
+  if (!lik || !y || !B || !cdiag || !post_mean || !post_cov || !nat1 || !nat2 || !Lw || !zw || !ldl || !part0 ||
+      !part1)
+    return st_fail(BN_EINVAL, "NULL argument to bn_st_sites");
+  if (method != BN_VI && method != BN_NEWTON)
+    return st_fail(BN_EUNSUPPORTED, "space-time sites support BN_VI and BN_NEWTON");
+  if (mode != BN_ST_UPDATE && mode != BN_ST_ENERGY && mode != BN_ST_PROJECT)
+    return st_fail(BN_EINVAL, "mode must be BN_ST_UPDATE, BN_ST_ENERGY or BN_ST_PROJECT");
+  LikParams L;
+  if (int rc = check_lik(lik, L)) return rc;
+  GHTable gh;
+  if (int rc = make_gh_table(gh_points, gh)) return rc;
+  if (int rc = set_smem_limits()) return rc;
+  StSiteIO io{y,    B,    cdiag, post_mean, post_cov, nat1,    nat2,     Lw,
+              zw,   ldl,  part0, part1,     out_mean, out_jac, out_hess, batch};
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid(dm.T, dm.K);
+  BN_TIMED(KID_ST_SITES, st);
+  if (mode == BN_ST_PROJECT) {
+    // the projection is method- and likelihood-free
+    if (whitened)
+      hipLaunchKernelGGL((k_st_sites<M_VI, BN_ST_PROJECT, 0>), grid, dim3(kT), kSitesSmem, st, dm, L, gh, io, lr,
+                         ensure_psd, 1.0, 0);
+    else
+      hipLaunchKernelGGL((k_st_sites_ordered<M_VI, BN_ST_PROJECT, 0>), grid, dim3(kT), kOrderedSmem, st, dm, L, gh, io,
+                         lr, ensure_psd, 1.0, 0);
+  } else if (mode == BN_ST_ENERGY) {
+    if (method == BN_VI) launch_st_sites<M_VI, BN_ST_ENERGY>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
+    else launch_st_sites<M_NEWTON, BN_ST_ENERGY>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
+  } else if (whitened) {
+    if (method == BN_VI) launch_st_sites<M_VI, BN_ST_UPDATE>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
+    else launch_st_sites<M_NEWTON, BN_ST_UPDATE>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
+  } else {
+    if (method == BN_VI) launch_st_update_ordered<M_VI>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
+    else launch_st_update_ordered<M_NEWTON>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
   }
+  ST_HIP_CHECK(hipGetLastError());
+  return BN_OK;
 }
 
 }  // namespace
@@ -2729,38 +3087,17 @@ int bn_st_sites(const bn_st_dims* dims, const bn_lik_desc* lik, int32_t method, 
                 const double* post_mean, const double* post_cov, const float* batch, double* nat1, double* nat2,
                 double* Lw, double* zw, double* ldl, double* part0, double* part1, float* out_mean, float* out_jac,
                 float* out_hess, void* stream) {
-  StDims dm;
-  if (int rc = check_dims(dims, dm)) return rc;
-  if (!lik || !y || !B || !cdiag || !post_mean || !post_cov || !nat1 || !nat2 || !Lw || !zw || !ldl || !part0 ||
-      !part1)
-    return st_fail(BN_EINVAL, "NULL argument to bn_st_sites");
-  if (method != BN_VI && method != BN_NEWTON)
-    return st_fail(BN_EUNSUPPORTED, "space-time sites support BN_VI and BN_NEWTON");
-  if (mode != BN_ST_UPDATE && mode != BN_ST_ENERGY && mode != BN_ST_PROJECT)
-    return st_fail(BN_EINVAL, "mode must be BN_ST_UPDATE, BN_ST_ENERGY or BN_ST_PROJECT");
-  LikParams L;
-  if (int rc = check_lik(lik, L)) return rc;
-  GHTable gh;
-  if (int rc = make_gh_table(gh_points, gh)) return rc;
-  if (int rc = set_smem_limits()) return rc;
-  StSiteIO io{y,    B,    cdiag, post_mean, post_cov, nat1,    nat2,     Lw,
-              zw,   ldl,  part0, part1,     out_mean, out_jac, out_hess, batch};
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid(dm.T, dm.K);
-  BN_TIMED(KID_ST_SITES, st);
-  if (mode == BN_ST_PROJECT) {
-    // the projection is method- and likelihood-free
-    hipLaunchKernelGGL((k_st_sites<M_VI, BN_ST_PROJECT, 0>), grid, dim3(kT), kSitesSmem, st, dm, L, gh, io, lr,
-                       ensure_psd, 1.0, 0);
-  } else if (method == BN_VI) {
-    if (mode == BN_ST_UPDATE) launch_st_sites<M_VI, BN_ST_UPDATE>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
-    else launch_st_sites<M_VI, BN_ST_ENERGY>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
-  } else {
-    if (mode == BN_ST_UPDATE) launch_st_sites<M_NEWTON, BN_ST_UPDATE>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
-    else launch_st_sites<M_NEWTON, BN_ST_ENERGY>(grid, st, dm, L, gh, io, lr, ensure_psd, 1.0, 0);
-  }
-  ST_HIP_CHECK(hipGetLastError());
-  return BN_OK;
+  return st_sites(false, dims, lik, method, mode, gh_points, lr, ensure_psd, y, B, cdiag, post_mean, post_cov, batch, nat1,
+                  nat2, Lw, zw, ldl, part0, part1, out_mean, out_jac, out_hess, stream);
+}
+
+int bn_st_sites_whitened(const bn_st_dims* dims, const bn_lik_desc* lik, int32_t method, int32_t mode, int32_t gh_points,
+                double lr, int32_t ensure_psd, const float* y, const double* B, const double* cdiag,
+                const double* post_mean, const double* post_cov, const float* batch, double* nat1, double* nat2,
+                double* Lw, double* zw, double* ldl, double* part0, double* part1, float* out_mean, float* out_jac,
+                float* out_hess, void* stream) {
+  return st_sites(true, dims, lik, method, mode, gh_points, lr, ensure_psd, y, B, cdiag, post_mean, post_cov, batch, nat1,
+                  nat2, Lw, zw, ldl, part0, part1, out_mean, out_jac, out_hess, stream);
 }
 
 int bn_st_ep_sites(const bn_st_dims* dims, const bn_lik_desc* lik, int32_t mode, int32_t gh_points, double lr,
@@ -2798,7 +3135,7 @@ int bn_st_ep_sites(const bn_st_dims* dims, const bn_lik_desc* lik, int32_t mode,
   BN_TIMED(KID_ST_SITES, st);
   if (mode == BN_ST_UPDATE) {
     hipLaunchKernelGGL((k_st_ep_cavity<false>), grid, dim3(kT), kCavitySmem, st, dm, cio, power, mask_pseudo);
-    launch_st_sites<M_EP, BN_ST_UPDATE>(grid, st, dm, L, gh, io, lr, ensure_psd, power, mask_pseudo);
+    launch_st_update_ordered<M_EP>(grid, st, dm, L, gh, io, lr, ensure_psd, power, mask_pseudo);
   } else {
     hipLaunchKernelGGL((k_st_ep_cavity<true>), grid, dim3(kT), kCavitySmem, st, dm, cio, power, mask_pseudo);
     launch_st_sites<M_EP, BN_ST_ENERGY>(grid, st, dm, L, gh, io, lr, ensure_psd, power, mask_pseudo);

@@ -90,13 +90,15 @@ constexpr int kDiagLd = 18;  // row stride of a 16 x 16 block on its own in LDS
 // every lane through a scalar register.  16 pivots deep and latency bound.
 //   D (LDS, row stride ld): A in (A's rows; only the lower triangle is read for the factor),
 //   L^-1 out (rows, zero above the diagonal).
-// L itself is not returned: the callers' row tiles get their factors as tile * L^-T.
+//   L (optional, row stride ldl): the factor, zero above the diagonal.  Row tiles below the block
+//   get their factors as tile * L^-T.
 // A non-positive pivot gives NaN, which propagates.
 // The scaling by 1 / sqrt(d) is the hardware estimate y and one third-order Newton step,
 // folded into the scaled column: w (y + y e (1/2 + 3/8 e)), e = 1 - d y^2.
 // Raised wave priority: the pivot chain competes for the FP64 pipe with the matrix
 // instructions of the wavefronts on the same SIMD, each of which holds it for 64 cycles.
-__device__ inline void chol16_inverse(double* D, int ld, int l) {
+template <bool KEEP = false>
+__device__ inline void chol16_inverse(double* D, int ld, int l, double* L = nullptr, int ldl = 0) {
   const int r = l & 15;
   double w[16];
   __builtin_amdgcn_s_setprio(3);
@@ -119,6 +121,10 @@ __device__ inline void chol16_inverse(double* D, int ld, int l) {
   if (l >= 16 && l < 32) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) D[j * ld + r] = w[j];  // column r of L^-1: zero above the diagonal
+  }
+  if (KEEP && l < 16) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) L[r * ldl + j] = j <= r ? w[j] : 0.0;
   }
   __builtin_amdgcn_s_setprio(0);
 }

@@ -151,10 +151,15 @@ class SpaceTimeMarkovGP:
         return h
 
     # ---- sites ---------------------------------------------------------------------------
+    # the filter takes the projection in whitened form; the forms that invert it explicitly
+    # need bn_st_sites' fixed order of summation
+    _whitened = True
+
     def _sites(self, mode, lr=1.0, cubature=None, ensure_psd=True, terms=None, batch=None):
         lik = self.likelihood.desc()
         om, oj, oh = terms if terms is not None else (None, None, None)
-        nat.check(nat.lib().bn_st_sites(
+        call = nat.lib().bn_st_sites_whitened if self._whitened else nat.lib().bn_st_sites
+        nat.check(call(
             ctypes.byref(self._dims), ctypes.byref(lik), self.method, mode, cub.num_points(cubature), float(lr),
             1 if ensure_psd else 0, nat.ptr(self._y), nat.ptr(self._B), nat.ptr(self._cdiag), nat.ptr(self._pm),
             nat.ptr(self._pP), nat.ptr(batch), nat.ptr(self._nat1), nat.ptr(self._nat2), nat.ptr(self._Lw),
@@ -527,6 +532,7 @@ class SpaceTimeMeanFieldGP(SpaceTimeMarkovGP):
     does), then filtered.  parallel=None picks the associative-scan form, as the reference
     does on a GPU backend (basemodels.py:640-641); parallel=False the sequential form.  The
     two are different approximations when the pseudo noise couples the blocks."""
+    _whitened = False
 
     def _alloc_filter(self):
         K, T, M = self.K, self.T, self.M
@@ -663,6 +669,7 @@ class SpaceTimeInfiniteHorizonGP(SpaceTimeMarkovGP):
     advance with each call.  Heteroscedastic (per-step gains) unless the likelihood is
     Gaussian with no missing data (basemodels.py:1270).  `parallel` is accepted: both of the
     reference's forms compute the same means."""
+    _whitened = False
 
     def __init__(self, kernel, likelihood, X, Y, R, dare_iters=20, parallel=None, device=None):
         self.dare_iters = int(dare_iters)
