@@ -510,13 +510,13 @@ constexpr int kRC = 32;  // rows of B per chunk
 constexpr int kLC = kMaxM + 1;  // LDS row stride of a chunk: consecutive rows start in different banks
 static_assert(2 * kRC * kLC >= kMaxM * kMaxM, "the two chunk buffers hold an M x M matrix");
 
-// The update and the projection for callers that go on to invert L L' explicitly
-// (k_mf_pseudo, the tied noise of the infinite-horizon form, the EP cavity): rounding in W and L
-// comes out of that inverse multiplied by the condition of W (1e6 and more on a grid of 64
-// inducing points), so W is summed over the locations in their order and factored pivot by
-// pivot, whatever the number of wavefronts.  k_st_sites is 1.7 times faster (one of two
-// launches 1.09 -> 0.45 ms at 4 runs of 500 steps, M = 64, R = 256) but rounds differently
-// in the last place, which moved mean-field posteriors by 1e-9 to 5e-9.
+// The update and the projection for the forms that go on to invert L L' explicitly and keep its
+// diagonal (the mean-field form, the EP cavity): rounding in W and L comes out multiplied by the
+// condition of W (1e6 and more on a grid of 64 inducing points), so W is summed over the
+// locations in their order and factored pivot by pivot, whatever the number of wavefronts.
+// k_st_sites is faster (1.09 -> 0.45 ms at 4 runs of 500 steps, M = 64, R = 256) but rounds
+// differently in the last place, which moved mean-field posteriors by 1e-9 to 5e-9 (dense and
+// infinite-horizon ones by 1e-14 to 4e-13).
 // KIND: the likelihood as a compile-time constant (0: the projection, which has none);
 // with only its branch compiled, the site step spills a fraction of what it does with
 // every likelihood's code in the kernel.
@@ -708,9 +708,7 @@ __global__ __launch_bounds__(kT, 2) void k_st_sites(StDims dm, LikParams lik, GH
     const double* src = io.B + (kt * R + 16 * rt) * M + l;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const bool on = l < M && 16 * rt + i < R;
-      const double v = *(on ? src + i * M : io.B);
-      pre[i] = on ? v : 0.0;
+      pre[i] = *(l < M && 16 * rt + i < R ? src + i * M : io.B);  // masked when it is placed
     }
   };
   if (w < RT) fetch(w);
@@ -731,7 +729,7 @@ __global__ __launch_bounds__(kT, 2) void k_st_sites(StDims dm, LikParams lik, GH
     l = fresh_v(l);
     wave_sync();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) cB[i * kSLd + l] = pre[i];
+    for (int i = 0; i < 16; ++i) cB[i * kSLd + l] = l < M && 16 * rt + i < R ? pre[i] : 0.0;
     // the lane's location in the site step: row l/16 + 4 ((l%16) / 4), the first of four lanes writes
     const int row = (l >> 4) + (l & 12), at = 16 * rt + row;
     const bool mine = (l & 3) == 0 && at < R;
@@ -1168,6 +1166,188 @@ constexpr int filter_smem(int KT, int MB) {
   return (KT + 2) * MP * LD + (MB + 1) * 16 * kDiagLd + 2 * MP + KT * MP + 2 * KT * KT;
 }
 
+// The covariance P of a state of KT components of MP = 16 MB entries in registers (the tiles
+// (i, j), i <= j, of its KT x KT blocks), and its update P -= W W' with W = U Lm^-T from the blocked
+// elimination of [Mm; U; q'].
+template <int KT, int MB>
+struct FilterCore {
+  static constexpr int MP = 16 * MB, LD = MP + 2, NW = 2 * MB, NT = 64 * NW;
+  static constexpr int NR = KT * MB;                  // row tiles of U
+  static constexpr int NPOS = MB * (MB + 1) / 2;      // tile positions of P
+  static constexpr int NP = (NPOS + NW - 1) / NW;     // positions per wavefront, at most
+  static constexpr bool kAllR = NR == NW;
+  typedef tile4 Cov[NP][KT][KT];
+
+  // position n of wavefront w: w, then (four tiles a side only, 10 positions) 8 on wavefront 0 and
+  // 9 on wavefront 6, whose SIMDs are not the ones that factor the second and the last block
+  static __device__ inline bool position(int w, int n, int& i, int& j) {
+    int p = n == 0 ? w : (w == 0 ? 8 : w == 6 ? 9 : NPOS);
+    const bool on = p < NPOS;
+    i = 0;
+#pragma unroll
+    for (int r = 0; r < MB - 1; ++r)
+      if (i == r && p >= MB - r) { p -= MB - r; i = r + 1; }
+    j = i + p;
+    return on;
+  }
+
+  // P := (A (x) I) P (A (x) I)' + Q (x) I; the mixed products are added first, so that an entry and
+  // its mirror image round alike
+  static __device__ inline void predict(Cov& P, const double (&A)[KT][KT], const double (&Q)[KT][KT], int M, int w,
+                                        int l) {
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!position(w, n, i, j)) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+        const double on = gi == gj && gi < M ? 1.0 : 0.0;
+        if (KT == 1) {
+          P[n][0][0][q] = fma(A[0][0] * A[0][0], P[n][0][0][q], on * Q[0][0]);
+        } else {
+          constexpr int o = KT - 1;
+          const double a = P[n][0][0][q], b = P[n][0][o][q], c = P[n][o][0][q], d = P[n][o][o][q];
+          const double s = b + c;
+          P[n][0][0][q] = fma(A[0][0] * A[0][0], a, fma(A[0][0] * A[0][o], s, fma(A[0][o] * A[0][o], d, on * Q[0][0])));
+          P[n][o][o][q] = fma(A[o][0] * A[o][0], a, fma(A[o][0] * A[o][o], s, fma(A[o][o] * A[o][o], d, on * Q[o][o])));
+          const double u = fma(A[0][0] * A[o][0], a, fma(A[0][o] * A[o][o], d, on * Q[0][o]));
+          const double x = A[0][0] * A[o][o], y = A[0][o] * A[o][0];
+          P[n][0][o][q] = fma(y, c, fma(x, b, u));
+          P[n][o][0][q] = fma(y, b, fma(x, c, u));
+        }
+      }
+    }
+  }
+
+  // X := P[:, :M]
+  static __device__ inline void publish(const Cov& P, double* X, int w, int l) {
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!position(w, n, i, j)) continue;
+#pragma unroll
+      for (int a = 0; a < KT; ++a) {
+        tile_store(X, LD, (a * MB + i) * 16, 16 * j, P[n][a][0], l);
+        if (i != j) tile_store_t(X, LD, (a * MB + j) * 16, 16 * i, P[n][0][a], l);
+      }
+    }
+  }
+
+  static __device__ inline void update(Cov& P, const double* X, int b, int w, int l) {  // P -= W_b W_b'
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!position(w, n, i, j)) continue;
+#pragma unroll
+      for (int c = 0; c < 16; c += 4) {
+        double ra[KT], rb[KT];
+#pragma unroll
+        for (int a = 0; a < KT; ++a) {
+          ra[a] = -frag(X, LD, (a * MB + i) * 16, 16 * b + c, l);
+          rb[a] = frag(X, LD, (a * MB + j) * 16, 16 * b + c, l);
+        }
+#pragma unroll
+        for (int a = 0; a < KT; ++a)
+#pragma unroll
+          for (int d = 0; d < KT; ++d) P[n][a][d] = mfma16(ra[a], rb[d], P[n][a][d]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // The elimination.  U: row tile w of U (also in X); V: row tile w of Mm (w < MB, column tiles
+  // <= w) or, with QROW, q' (the last wavefront); the first diagonal block's inverse factor is in sI
+  // (wavefront 0).  X: U in, W out; se: e, quad: e' e in the lanes of the last wavefront.
+  // One copy of the block's code: U and V are shifted by one tile after each block, so that tile 0
+  // is always the current one.
+  template <bool QROW>
+  static __device__ inline void eliminate(Cov& P, tile4 (&U)[MB], tile4 (&V)[MB], double& quad, double* X, double* Lm,
+                                          double* sI, double* sG, double* se, const int w0, const int tid0) {
+    int w = w0, l = tid0 & 63;
+    auto phase = [&]() { w = fresh_s(w0); l = fresh_v(tid0) & 63; };
+#pragma unroll 1
+    for (int b = 0; b < MB; ++b) {
+      const double* Ib = sI + b * 16 * kDiagLd;
+      __syncthreads();  // inverse factor of diagonal block b
+      phase();
+      // row tiles times the inverse factor's transpose: column block b of W, Lm and e
+      if (w > b && w < MB) {
+        tile_store(Lm, LD, 16 * w, 16 * b, V[0], l);
+        wave_sync();
+        const tile4 v = tile_mul_t(Lm, LD, 16 * w, Ib, kDiagLd, 0, 16 * b, 0, tile_zero(), l);
+        wave_sync();
+        tile_store(Lm, LD, 16 * w, 16 * b, v, l);
+      } else if (QROW && w == NW - 1) {
+        tile_store(sG, kDiagLd, 0, 0, V[0], l);
+        wave_sync();
+        const tile4 v = tile_mul_t(sG, kDiagLd, 0, Ib, kDiagLd, 0, 0, 0, tile_zero(), l);
+        wave_sync();
+        tile_store(sG, kDiagLd, 0, 0, v, l);
+        if (l < 16) {
+          se[16 * b + l] = v[0];
+          quad = fma(v[0], v[0], quad);
+        }
+      }
+      if (kAllR || w < NR) {
+        if (b > 0) {
+          tile_store(X, LD, 16 * w, 16 * b, U[0], l);
+          wave_sync();
+        }
+        const tile4 v = tile_mul_t(X, LD, 16 * w, Ib, kDiagLd, 0, 16 * b, 0, tile_zero(), l);
+        wave_sync();
+        tile_store(X, LD, 16 * w, 16 * b, v, l);
+      }
+      if (MB > 1 && w == b + 1 && w < MB) {
+        // the next diagonal block first: its factorisation is the critical path
+#pragma unroll
+        for (int c = 0; c < 16; c += 4) {
+          const double a = frag(Lm, LD, 16 * w, 16 * b + c, l);
+          V[MB > 1 ? 1 : 0] = mfma16(-a, a, V[MB > 1 ? 1 : 0]);
+        }
+        tile_store(sI + (b + 1) * 16 * kDiagLd, kDiagLd, 0, 0, V[MB > 1 ? 1 : 0], l);
+      }
+      __syncthreads();  // column block b of W and Lm
+      phase();
+      // remaining columns of the row tiles
+      if (b + 1 < MB) {
+        if (w == b + 1) chol16_inverse(sI + (b + 1) * 16 * kDiagLd, kDiagLd, l);
+        double a[4];
+        const bool qrow = QROW && w == NW - 1;
+        if ((w > b + 1 && w < MB) || qrow) {
+          const double* S = qrow ? sG : Lm + 16 * w * LD + 16 * b;
+          const int ld = qrow ? kDiagLd : LD;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) a[c] = -frag(S, ld, 0, 4 * c, l);
+#pragma unroll
+          for (int j = 1; j < MB; ++j)
+            if (b + j < MB) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) V[j] = mfma16(a[c], frag(Lm, LD, 16 * (b + j), 16 * b + 4 * c, l), V[j]);
+            }
+        }
+        if (kAllR || w < NR) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) a[c] = -frag(X, LD, 16 * w, 16 * b + 4 * c, l);
+#pragma unroll
+          for (int j = 1; j < MB; ++j)
+            if (b + j < MB) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) U[j] = mfma16(a[c], frag(Lm, LD, 16 * (b + j), 16 * b + 4 * c, l), U[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j + 1 < MB; ++j) { U[j] = U[j + 1]; V[j] = V[j + 1]; }
+      }
+      // (a wavefront on the SIMD that factors the next block leaves its part to the last one)
+      const int late = (w & 3) > 0 && (w & 3) < MB ? (w & 3) - 1 : -1;
+      const int n = b == late ? 0 : b == MB - 1 && late >= 0 ? 2 : 1;
+#pragma unroll 1
+      for (int u = 0; u < n; ++u) update(P, X, u == 0 ? b : late, w, l);
+    }
+  }
+};
+
 // Row tile I of the lower triangle of Mm = I + L' U[:M] (column tiles <= I; L' is upper
 // triangular, so inner tiles >= I).
 template <int MB, int I>
@@ -1190,11 +1370,9 @@ __device__ inline void filter_mm_row(const double* LT, const double* X, int ld, 
 
 template <int KT, int MB>
 __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, StFilterIO io) {
-  constexpr int MP = 16 * MB, LD = MP + 2, NW = 2 * MB, NT = 64 * NW;
-  constexpr int NR = KT * MB;                       // row tiles of U
-  constexpr int NPOS = MB * (MB + 1) / 2;           // tile positions (i, j), i <= j, of P
-  constexpr int NP = (NPOS + NW - 1) / NW;          // positions per wavefront, at most
-  constexpr bool kAllR = NR == NW;
+  using C = FilterCore<KT, MB>;
+  constexpr int MP = C::MP, LD = C::LD, NW = C::NW, NT = C::NT, NR = C::NR, NP = C::NP;
+  constexpr bool kAllR = C::kAllR;
   constexpr int NL = (MP * MP + NT - 1) / NT;       // elements of L per thread
   constexpr int NAQ = 2 * KT * KT;
   extern __shared__ double smem[];
@@ -1212,26 +1390,14 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
   const int w0 = __builtin_amdgcn_readfirstlane(tid >> 6);
   int w = w0;
   const int k = blockIdx.x;
-  // position n of a wavefront: w, then (four tiles a side only, 10 positions) 8 on wavefront 0 and
-  // 9 on wavefront 6, whose SIMDs are not the ones that factor the second and the last block
-  auto position = [&](int n, int& i, int& j) {
-    int p = n == 0 ? w : (w == 0 ? 8 : w == 6 ? 9 : NPOS);
-    const bool on = p < NPOS;
-    i = 0;
-#pragma unroll
-    for (int r = 0; r < MB - 1; ++r)
-      if (i == r && p >= MB - r) { p -= MB - r; i = r + 1; }
-    j = i + p;
-    return on;
-  };
-  tile4 P[NP][KT][KT];
+  typename C::Cov P;
   {  // P0 = Pinf (x) I, m0 = 0
     Model<KT, 0> mdl;
     mdl.init(hy.ls_t[k * hy.stride], hy.var_t[k * hy.stride], 1.0, 1.0);
 #pragma unroll
     for (int n = 0; n < NP; ++n) {
       int i, j;
-      const bool held = position(n, i, j);
+      const bool held = C::position(w, n, i, j);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
@@ -1255,9 +1421,7 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
       const int e = tid + n * NT, r = e / MP, c = e % MP;
-      const bool on = r < M && c < M;
-      const double v = L[on ? r * M + c : 0];
-      lreg[n] = on ? v : 0.0;
+      lreg[n] = L[r < M && c < M ? r * M + c : 0];  // masked when it is placed: nothing here waits for the load
     }
     if (tid < M) zreg = io.zw[kt * M + tid];
     if (tid < NAQ) aqreg = io.aq[kt * NAQ + tid];
@@ -1266,31 +1430,10 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
       const int e = tid + n * NT, r = e / MP, c = e % MP;
-      if (NL * NT == MP * MP || e < MP * MP) LT[c * LD + r] = lreg[n];
+      if (NL * NT == MP * MP || e < MP * MP) LT[c * LD + r] = r < M && c < M ? lreg[n] : 0.0;
     }
     if (tid < MP) sq[tid] = zreg;
     if (tid < NAQ) saq[tid] = aqreg;
-  };
-  auto update_P = [&](int b) {  // P -= W_b W_b'
-#pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      int i, j;
-      if (!position(n, i, j)) continue;
-#pragma unroll
-      for (int c = 0; c < 16; c += 4) {
-        double ra[KT], rb[KT];
-#pragma unroll
-        for (int a = 0; a < KT; ++a) {
-          ra[a] = -frag(X, LD, (a * MB + i) * 16, 16 * b + c, l);
-          rb[a] = frag(X, LD, (a * MB + j) * 16, 16 * b + c, l);
-        }
-#pragma unroll
-        for (int a = 0; a < KT; ++a)
-#pragma unroll
-          for (int d = 0; d < KT; ++d) P[n][a][d] = mfma16(ra[a], rb[d], P[n][a][d]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
   };
   auto phase = [&]() { w = fresh_s(w0); tid = fresh_v(tid0); l = tid & 63; };
   fetch(k0);
@@ -1308,36 +1451,8 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
         A[a][b] = saq[a * KT + b];
         Q[a][b] = saq[KT * KT + a * KT + b];
       }
-    // P- = (A (x) I) P (A (x) I)' + Q (x) I; the mixed products are added first, so that
-    // (i, j) and (j, i) round alike
-#pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      int i, j;
-      if (!position(n, i, j)) continue;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
-        const double on = gi == gj && gi < M ? 1.0 : 0.0;
-        if (KT == 1) {
-          P[n][0][0][q] = fma(A[0][0] * A[0][0], P[n][0][0][q], on * Q[0][0]);
-        } else {
-          constexpr int o = KT - 1;
-          const double a = P[n][0][0][q], b = P[n][0][o][q], c = P[n][o][0][q], d = P[n][o][o][q];
-          const double s = b + c;
-          P[n][0][0][q] = fma(A[0][0] * A[0][0], a, fma(A[0][0] * A[0][o], s, fma(A[0][o] * A[0][o], d, on * Q[0][0])));
-          P[n][o][o][q] = fma(A[o][0] * A[o][0], a, fma(A[o][0] * A[o][o], s, fma(A[o][o] * A[o][o], d, on * Q[o][o])));
-          const double u = fma(A[0][0] * A[o][0], a, fma(A[0][o] * A[o][o], d, on * Q[0][o]));
-          const double x = A[0][0] * A[o][o], y = A[0][o] * A[o][0];
-          P[n][0][o][q] = fma(y, c, fma(x, b, u));
-          P[n][o][0][q] = fma(y, b, fma(x, c, u));
-        }
-      }
-#pragma unroll
-      for (int a = 0; a < KT; ++a) {
-        tile_store(X, LD, (a * MB + i) * 16, 16 * j, P[n][a][0], l);
-        if (i != j) tile_store_t(X, LD, (a * MB + j) * 16, 16 * i, P[n][0][a], l);
-      }
-    }
+    C::predict(P, A, Q, M, w, l);
+    C::publish(P, X, w, l);
     if (tid < MP) {
       double x[KT];
 #pragma unroll
@@ -1403,86 +1518,7 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
         V[j][0] = l < 16 ? sq[16 * j + l] : 0.0;
       }
     }
-    // one copy of the block's code (the unrolled loop would not fit the instruction cache): U and
-    // V are shifted by one tile after each block, so that tile 0 is always the current one
-#pragma unroll 1
-    for (int b = 0; b < MB; ++b) {
-      const double* Ib = sI + b * 16 * kDiagLd;
-      __syncthreads();  // inverse factor of diagonal block b
-      phase();
-      // row tiles times the inverse factor's transpose: column block b of W, Lm and e
-      if (w > b && w < MB) {
-        tile_store(Lm, LD, 16 * w, 16 * b, V[0], l);
-        wave_sync();
-        const tile4 v = tile_mul_t(Lm, LD, 16 * w, Ib, kDiagLd, 0, 16 * b, 0, tile_zero(), l);
-        wave_sync();
-        tile_store(Lm, LD, 16 * w, 16 * b, v, l);
-      } else if (w == NW - 1) {
-        tile_store(sG, kDiagLd, 0, 0, V[0], l);
-        wave_sync();
-        const tile4 v = tile_mul_t(sG, kDiagLd, 0, Ib, kDiagLd, 0, 0, 0, tile_zero(), l);
-        wave_sync();
-        tile_store(sG, kDiagLd, 0, 0, v, l);
-        if (l < 16) {
-          se[16 * b + l] = v[0];
-          quad = fma(v[0], v[0], quad);
-        }
-      }
-      if (kAllR || w < NR) {
-        if (b > 0) {
-          tile_store(X, LD, 16 * w, 16 * b, U[0], l);
-          wave_sync();
-        }
-        const tile4 v = tile_mul_t(X, LD, 16 * w, Ib, kDiagLd, 0, 16 * b, 0, tile_zero(), l);
-        wave_sync();
-        tile_store(X, LD, 16 * w, 16 * b, v, l);
-      }
-      if (MB > 1 && w == b + 1 && w < MB) {
-        // the next diagonal block first: its factorisation is the critical path
-#pragma unroll
-        for (int c = 0; c < 16; c += 4) {
-          const double a = frag(Lm, LD, 16 * w, 16 * b + c, l);
-          V[MB > 1 ? 1 : 0] = mfma16(-a, a, V[MB > 1 ? 1 : 0]);
-        }
-        tile_store(sI + (b + 1) * 16 * kDiagLd, kDiagLd, 0, 0, V[MB > 1 ? 1 : 0], l);
-      }
-      __syncthreads();  // column block b of W and Lm
-      phase();
-      // remaining columns of the row tiles
-      if (b + 1 < MB) {
-        if (w == b + 1) chol16_inverse(sI + (b + 1) * 16 * kDiagLd, kDiagLd, l);
-        double a[4];
-        if ((w > b + 1 && w < MB) || w == NW - 1) {
-          const double* S = w == NW - 1 ? sG : Lm + 16 * w * LD + 16 * b;
-          const int ld = w == NW - 1 ? kDiagLd : LD;
-#pragma unroll
-          for (int c = 0; c < 4; ++c) a[c] = -frag(S, ld, 0, 4 * c, l);
-#pragma unroll
-          for (int j = 1; j < MB; ++j)
-            if (b + j < MB) {
-#pragma unroll
-              for (int c = 0; c < 4; ++c) V[j] = mfma16(a[c], frag(Lm, LD, 16 * (b + j), 16 * b + 4 * c, l), V[j]);
-            }
-        }
-        if (kAllR || w < NR) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) a[c] = -frag(X, LD, 16 * w, 16 * b + 4 * c, l);
-#pragma unroll
-          for (int j = 1; j < MB; ++j)
-            if (b + j < MB) {
-#pragma unroll
-              for (int c = 0; c < 4; ++c) U[j] = mfma16(a[c], frag(Lm, LD, 16 * (b + j), 16 * b + 4 * c, l), U[j]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j + 1 < MB; ++j) { U[j] = U[j + 1]; V[j] = V[j + 1]; }
-      }
-      // (a wavefront on the SIMD that factors the next block leaves its part to the last one)
-      const int late = (w & 3) > 0 && (w & 3) < MB ? (w & 3) - 1 : -1;
-      const int n = b == late ? 0 : b == MB - 1 && late >= 0 ? 2 : 1;
-#pragma unroll 1
-      for (int u = 0; u < n; ++u) update_P(u == 0 ? b : late);
-    }
+    C::template eliminate<true>(P, U, V, quad, X, Lm, sI, sG, se, w0, tid0);
     phase();
     if (t + 1 < dm.T) place();  // LT, sq and saq are not read again in this step
     // m = m- + W e, rows 16 w .. (each wavefront its own)
@@ -1521,7 +1557,7 @@ __global__ __launch_bounds__(128 * MB, 2) void k_st_filter(StDims dm, StHyp hy, 
 #pragma unroll
     for (int n = 0; n < NP; ++n) {
       int i, j;
-      if (!position(n, i, j)) continue;
+      if (!C::position(w, n, i, j)) continue;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
@@ -1579,13 +1615,17 @@ struct StGainIO {
   const double* fcov;   // [K,T,D(D+1)/2]
   double* rec;          // [K, tb] maps
   int t0, tb;
+  // STEADY: one map a run, from the filtered covariance fcov [K,D,D] and P- = X [K,D,D] as it stands,
+  // aq [K,2 KT^2]; G [K,D,D] is also written as it is
+  const double* X;
+  double* G;
 };
 
 // Per workgroup: 36 + 64 tiles in registers, Lc in LDS.  Bound by the eight pivot chains
 // (chol16_inverse) and, behind them, by the matrix instructions of the elimination and of the
 // back substitution.  M = 64, D = 128: 999 steps in 293 us (617 us with the sweep inverse of P-
 // in LDS and a product through panels).
-template <int KT, int MB>
+template <int KT, int MB, bool STEADY>
 __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainIO io) {
   using S = StTiles<KT, MB>;
   constexpr int MP = S::MP, NR = S::NR, DP = S::DP, LD = S::LD, NW = NR;
@@ -1597,8 +1637,8 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainI
   int l = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = S::row(w);
   const int k = blockIdx.y, t = io.t0 + blockIdx.x;
-  const int64_t kt = (int64_t)k * dm.T + t;
-  const double* aq = io.aq + (kt + 1) * 2 * KT * KT;
+  const int64_t kt = (int64_t)k * dm.T + t, DD = (int64_t)D * D;
+  const double* aq = io.aq + (STEADY ? k : kt + 1) * 2 * KT * KT;
   double A[KT][KT], Q[KT][KT];
 #pragma unroll
   for (int a = 0; a < KT; ++a)
@@ -1607,7 +1647,19 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainI
       A[a][b] = aq[a * KT + b];
       Q[a][b] = aq[KT * KT + a * KT + b];
     }
-  {  // P_t into LDS, both triangles, zero padding
+  if (STEADY) {  // the filtered covariance, zero padding
+    const double* cov = io.fcov + k * DD;
+#pragma unroll 4
+    for (int pr = w; pr < DP; pr += NW) {
+      const int i = pr % MP;
+#pragma unroll
+      for (int n = 0; n < (DP + 63) / 64; ++n) {
+        const int pc = l + 64 * n, j = pc % MP;
+        const bool on = i < M && j < M;
+        if (pc < DP) X[pr * LD + pc] = on ? cov[(int64_t)(pr / MP * M + i) * D + pc / MP * M + j] : 0.0;
+      }
+    }
+  } else {  // P_t into LDS, both triangles, zero padding
     const double* pk = io.fcov + kt * ((int64_t)D * (D + 1) / 2);
 #pragma unroll 4
     for (int pr = w; pr < DP; pr += NW) {
@@ -1669,6 +1721,7 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainI
             s = fma(ap[a], A[b][a], s);
             u = fma(own[a], A[b][a], u);
           }
+          if (STEADY && gi < M && gj < M) s = io.X[k * DD + (int64_t)(ra * M + gi) * D + b * M + gj];
           Sm[b * MB + jj][q] = s;
           U[b * MB + jj][q] = u;
           R[b * MB + jj][q] = own[b];
@@ -1756,10 +1809,17 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainI
     tile_store(st, kDiagLd, 0, 0, v, l);
     wave_sync();
     frag4(a, st, kDiagLd, 0, 0, 1.0, l);
+    if (STEADY) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * (r % MB) + (l >> 4) + 4 * q, gj = 16 * (b % MB) + (l & 15);
+        if (gi < M && gj < M) io.G[k * DD + (int64_t)(r / MB * M + gi) * D + b / MB * M + gj] = v[q];
+      }
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       g[(4 * b + c) * 64 + l] = a[c];
-      cv = fma(a[c], vp[16 * b + 4 * c + (l >> 4)], cv);
+      if (!STEADY) cv = fma(a[c], vp[16 * b + 4 * c + (l >> 4)], cv);
       a[c] = -a[c];
     }
 #pragma unroll
@@ -1768,6 +1828,7 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_gains(StDims dm, StGainI
       for (int c = 0; c < 4; ++c) U[j] = mfma16(a[c], frag_t(X, LD, 16 * b + 4 * c, 16 * j, l), U[j]);
     wave_sync();
   }
+  if (STEADY) return;
   cv += __shfl_xor(cv, 16, 64);
   cv += __shfl_xor(cv, 32, 64);
   if (l < 16) {
@@ -1788,6 +1849,8 @@ struct StSmootherIO {
   double* smean;     // optional [K,T,D] smoothed state (return_full)
   double* scov;      // optional [K,T,D,D]
   double* scross;    // optional [K,T,D,D]: G_t P_s,t+1 = Cov(x_t, x_t+1 | y); Pinf at the last step
+  double* xs;        // ST_STEADY: [K,D,D] in and out
+  int iters;
 };
 
 // first step of chunk c of a block
@@ -1873,7 +1936,8 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_chain(StSmootherIO io) {
   for (int f = 0; f < NF; ++f) out[f * 64] = frag_t(X, LD, 4 * f, 16 * w, l);
 }
 
-enum { ST_WALK = 0, ST_COMPOSE = 1, ST_JOIN = 2 };
+// ST_STEADY: `iters` times the run's one map, on the covariance xs (the infinite-horizon smoother).
+enum { ST_WALK = 0, ST_COMPOSE = 1, ST_JOIN = 2, ST_STEADY = 3 };
 
 // Per step T = G P_s' (G's row tile from registers, P_s' in LDS, both triangles) and
 // P_s = R + T G' (tiles j <= r; G in LDS, T through a staging tile): 51 k cycles of FP64 matrix
@@ -1893,12 +1957,25 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSm
   int l = tid & 63;
   const int k = blockIdx.y;
   const int c = MODE == ST_COMPOSE ? blockIdx.x + 1 : blockIdx.x;
-  const int s0 = MODE == ST_JOIN ? 1 : chunk_start(io, c), s1 = MODE == ST_JOIN ? io.nc : chunk_start(io, c + 1);
+  const int s0 = MODE == ST_STEADY ? 0 : MODE == ST_JOIN ? 1 : chunk_start(io, c);
+  const int s1 = MODE == ST_STEADY ? io.iters : MODE == ST_JOIN ? io.nc : chunk_start(io, c + 1);
   const double* rec = MODE == ST_JOIN ? io.comp + (int64_t)k * io.nc * S::REC : io.rec + (int64_t)k * io.tb * S::REC;
   double* states = io.state + (int64_t)k * io.slots * S::STATE;
   double* st = sT + w * 16 * kDiagLd;
   tile4 P[NR];
-  if (MODE == ST_COMPOSE) {
+  if (MODE == ST_STEADY) {
+    const double* xs = io.xs + (int64_t)k * D * D;
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int gi = 16 * (r % MB) + (l >> 4) + 4 * q, gj = 16 * (j % MB) + (l & 15);
+          P[j][q] = gi < M && gj < M ? xs[(int64_t)(r / MB * M + gi) * D + j / MB * M + gj] : 0.0;
+        }
+      }
+    for (int e = tid; e < DP; e += NT) ms[e] = 0.0;
+  } else if (MODE == ST_COMPOSE) {
 #pragma unroll
     for (int j = 0; j < NR; ++j) P[j] = tile_zero();
     for (int e = tid; e < DP; e += NT) ms[e] = 0.0;
@@ -1911,7 +1988,7 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSm
   }
   double g[NF];
   auto fetch = [&](int s) {
-    const double* src = rec + (int64_t)s * S::REC + r * 16 * DP + l;
+    const double* src = rec + (MODE == ST_STEADY ? 0 : (int64_t)s * S::REC) + r * 16 * DP + l;
 #pragma unroll
     for (int f = 0; f < NF; ++f) g[f] = src[f * 64];
   };
@@ -1943,7 +2020,7 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSm
     publish();
     __syncthreads();
     if (MODE == ST_WALK && s + 1 < s1) emit(s + 1, ms + cur * DP);
-    const double* rs = rec + (int64_t)s * S::REC + DP * DP;
+    const double* rs = rec + (MODE == ST_STEADY ? 0 : (int64_t)s * S::REC) + DP * DP;
     tile4 T[NR];
     double v = 0.0;
 #pragma unroll
@@ -1952,13 +2029,15 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSm
     for (int f = 0; f < NF; ++f) {
 #pragma unroll
       for (int j = 0; j < NR; ++j) T[j] = mfma16(g[f], frag(X, LD, 16 * j, 4 * f, l), T[j]);
-      v = fma(g[f], ms[cur * DP + 4 * f + (l >> 4)], v);
+      if (MODE != ST_STEADY) v = fma(g[f], ms[cur * DP + 4 * f + (l >> 4)], v);
       if (f % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    cur ^= 1;
-    if (l < 16) ms[cur * DP + 16 * r + l] = rs[S::SYM + 16 * r + l] + v;
+    if (MODE != ST_STEADY) {
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      cur ^= 1;
+      if (l < 16) ms[cur * DP + 16 * r + l] = rs[S::SYM + 16 * r + l] + v;
+    }
     if (MODE == ST_WALK && io.scross) {
       const int64_t kt = (int64_t)k * dm.T + io.t0 + s;
 #pragma unroll
@@ -2000,6 +2079,22 @@ __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSm
         if (j <= r) tile_put(o + S::sym(r, j), P[j], l);
       for (int e = tid; e < DP; e += NT) o[S::SYM + e] = ms[cur * DP + e];
     }
+  }
+  if (MODE == ST_STEADY) {
+    double* xs = io.xs + (int64_t)k * D * D;
+#pragma unroll
+    for (int j = 0; j < NR; ++j)
+      if (j <= r) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int gi = 16 * (r % MB) + (l >> 4) + 4 * q, gj = 16 * (j % MB) + (l & 15);
+          const int u = r / MB * M + gi, v = j / MB * M + gj;
+          if (gi < M && gj < M) {
+            xs[(int64_t)u * D + v] = P[j][q];
+            if (j != r) xs[(int64_t)v * D + u] = P[j][q];
+          }
+        }
+      }
   }
   if (MODE == ST_WALK) {
     publish();
@@ -2401,12 +2496,14 @@ __global__ __launch_bounds__(64) void k_mf_smoother(StDims dm, StHyp hy, MfSmoot
 //                 R_tied = (mean_t B' diag(nat2_t) B)^-1 from the whitened form (L L' - 1e-12 I),
 //                 partial sums over step ranges on the matrix cores
 //   k_ih_dare     `iters` Riccati iterations X <- A (X - X H' S^-1 H X) A' + Q, S = H X H' + R_tied,
-//                 from the previous solution; S_tied^-1 and cov = X - K H X (K = X H' S^-1)
-//   k_ih_sinv     heteroscedastic: S_t = H X H' + R_t inverted per (step, run), log det S_t
-//   k_ih_filter   m_t = A m_{t-1} + X H' S_t^-1 (y_t - H A m_{t-1}), log N(y_t | H A m_{t-1}, S_t)
-//   k_ih_smoother G = cov A' X^-1, Qd = cov - G X G', `iters` iterations X_s <- G X_s G' + Qd
-//                 (from the previous solution), sm_t = fm_t + G (sm_{t+1} - A fm_t) from
-//                 sm = fm_{T-1}; H X_s H' at every step.
+//                 from the previous solution; cov = X - K H X (K = X H' S^-1)
+//   k_ih_sinv     S_tied, or (heteroscedastic) every step's S_t = H X H' + R_t, inverted; log det
+//   k_ih_filter   m_t = A m_{t-1} + X H' S_t^-1 (y_t - H A m_{t-1})
+//   k_ih_ell      log N(y_t | H A m_{t-1}, S_t)
+//   k_st_gains    (STEADY) G = cov A' X^-1, Qd = cov - G X G'
+//   k_st_smoother (ST_STEADY) `iters` iterations X_s <- G X_s G' + Qd from the previous solution
+//   k_ih_means    sm_t = fm_t + G (sm_{t+1} - A fm_t) from sm = fm_{T-1}
+//   k_ih_spread   H X_s H' at every step
 // State layout as in k_st_filter: index c*M + m, H picks the c = 0 block.
 // ---------------------------------------------------------------------------
 constexpr int kTiedParts = 32;  // step ranges summed in parallel per run
@@ -2446,14 +2543,12 @@ __global__ __launch_bounds__(kT) void k_ih_tied(StDims dm, const double* __restr
 }
 
 struct IhIO {
-  const double* step;  // [K] step size of each run
+  const double* aq;    // [K, 2 KT^2] transition of each run's step
   const double* y;     // [K,T,M]
   const double* R;     // [K,T,M,M] (heteroscedastic)
   const double* Rt;    // [K,M,M] tied noise
   double* X;           // [K,D,D] Riccati solution: start in, result out
   double* cov;         // [K,D,D]
-  double* W1;          // [K,D,D] scratch
-  double* W2;          // [K,D,D] scratch
   double* STn;         // [K,M,M] -S_tied^-1
   double* ldT;         // [K]
   double* Sn;          // [K,T,M,M] -S_t^-1 (heteroscedastic)
@@ -2463,203 +2558,334 @@ struct IhIO {
   int32_t iters, hetero;
 };
 
-template <int KT>
-__global__ __launch_bounds__(kT) void k_ih_dare(StDims dm, StHyp hy, IhIO io) {
+// Riccati iterations X <- A (X - W W') A' + Q, W = X H' Ls^-T, Ls Ls' = H X H' + R_tied, on the
+// filter's register tiles (FilterCore), then cov = X - W W'.  One workgroup per run: the chain of
+// iterations bounds it; 12 us an iteration at M = 36, D = 72 (50 us with the sweep inverse and
+// products through LDS panels).
+template <int KT, int MB>
+__global__ __launch_bounds__(128 * MB, 2) void k_ih_dare(StDims dm, IhIO io) {
+  using C = FilterCore<KT, MB>;
+  constexpr int MP = C::MP, LD = C::LD, NT = C::NT, NR = C::NR, NP = C::NP;
   extern __shared__ double smem[];
-  double* pan = smem;                   // 2*kPK*kPS
-  double* sS = pan + 2 * kPK * kPS;     // M*M
-  double* sR = sS + kMaxM * kMaxM;      // M*M
-  double* row = sR + kMaxM * kMaxM;     // 2*kMaxM
-  __shared__ double sA[KT * KT], sQ[KT * KT];
-  const int k = blockIdx.x, M = dm.M, D = dm.D, tid = threadIdx.x;
+  double* X = smem;                    // KT*MP x LD: X H', then W
+  double* Lm = X + KT * MP * LD;       // MP x LD
+  double* sI = Lm + MP * LD;           // MB of 16 x kDiagLd
+  const int M = dm.M, D = dm.D, tid0 = threadIdx.x;
+  const int w0 = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+  int w = w0, l = tid0 & 63;
+  const int k = blockIdx.x;
   const int64_t DD = (int64_t)D * D;
-  double* X = io.X + k * DD;
-  double* W1 = io.W1 + k * DD;
-  double* W2 = io.W2 + k * DD;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  if (tid == 0) temporal_AQ<KT>(ls, var, io.step[k], sA, sQ);
-  for (int e = tid; e < M * M; e += kT) sR[e] = io.Rt[(int64_t)k * M * M + e];
-  __syncthreads();
-  for (int it = 0; it < io.iters; ++it) {
-    for (int e = tid; e < M * M; e += kT) sS[e] = X[(int64_t)(e / M) * D + e % M] + sR[e];
-    wg_sweep_inv<kMaxM / 16, false>(sS, M, M, row);  // sS = -S^-1
-    wg_gemm(D, M, M, -1.0, MatRef{X, D, 1}, MatRef{sS, M, 1}, 0.0, W1, M, pan);  // K = X H' S^-1
-    for (int64_t e = tid; e < DD; e += kT) W2[e] = X[e];
-    __syncthreads();
-    wg_gemm(D, D, M, -1.0, MatRef{W1, M, 1}, MatRef{X, D, 1}, 1.0, W2, D, pan);  // X - K H X
-    __syncthreads();
-    // X = A sym(W2) A' + Q over the KT x KT blocks of M x M
-    for (int e = tid; e < M * M; e += kT) {
-      const int a = e / M, c = e % M;
-      double w[KT][KT];
-      for (int p = 0; p < KT; ++p)
-        for (int q = 0; q < KT; ++q)
-          w[p][q] = 0.5 * (W2[(int64_t)(p * M + a) * D + q * M + c] + W2[(int64_t)(q * M + c) * D + p * M + a]);
-      for (int i = 0; i < KT; ++i)
-        for (int j = 0; j < KT; ++j) {
-          double v = (a == c) ? sQ[i * KT + j] : 0.0;
-          for (int p = 0; p < KT; ++p)
-            for (int q = 0; q < KT; ++q) v = fma(sA[i * KT + p] * w[p][q], sA[j * KT + q], v);
-          X[(int64_t)(i * M + a) * D + j * M + c] = v;
-        }
+  double A[KT][KT], Q[KT][KT];
+#pragma unroll
+  for (int a = 0; a < KT; ++a)
+#pragma unroll
+    for (int b = 0; b < KT; ++b) {
+      A[a][b] = io.aq[k * 2 * KT * KT + a * KT + b];
+      Q[a][b] = io.aq[k * 2 * KT * KT + KT * KT + a * KT + b];
     }
-    __syncthreads();
+  typename C::Cov P;
+#pragma unroll
+  for (int n = 0; n < NP; ++n) {
+    int i, j;
+    const bool held = C::position(w, n, i, j);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+      const bool on = held && gi < M && gj < M;
+#pragma unroll
+      for (int a = 0; a < KT; ++a)
+#pragma unroll
+        for (int b = 0; b < KT; ++b) P[n][a][b][q] = on ? io.X[k * DD + (int64_t)(a * M + gi) * D + b * M + gj] : 0.0;
+    }
   }
-  // tied innovation covariance, gain and the infinite-horizon filtered covariance
-  for (int e = tid; e < M * M; e += kT) sS[e] = X[(int64_t)(e / M) * D + e % M] + sR[e];
-  const double ld = wg_sweep_inv<kMaxM / 16, true>(sS, M, M, row);
-  for (int e = tid; e < M * M; e += kT) io.STn[(int64_t)k * M * M + e] = sS[e];
-  if (tid == 0) io.ldT[k] = ld;
-  wg_gemm(D, M, M, -1.0, MatRef{X, D, 1}, MatRef{sS, M, 1}, 0.0, W1, M, pan);
-  double* cv = io.cov + k * DD;
-  for (int64_t e = tid; e < DD; e += kT) cv[e] = X[e];
-  __syncthreads();
-  wg_gemm(D, D, M, -1.0, MatRef{W1, M, 1}, MatRef{X, D, 1}, 1.0, cv, D, pan);
+  tile4 Rt[MB];  // row tile w of the tied noise, identity padding
+#pragma unroll
+  for (int j = 0; j < MB; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int gi = 16 * w + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+      Rt[j][q] = w >= MB || j > w ? 0.0 : gi < M && gj < M ? io.Rt[((int64_t)k * M + gi) * M + gj] : gi == gj ? 1.0 : 0.0;
+    }
+  auto write = [&](double* out) {
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      int i, j;
+      if (!C::position(w, n, i, j)) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int gi = 16 * i + (l >> 4) + 4 * q, gj = 16 * j + (l & 15);
+        if (gi < M && gj < M) {
+#pragma unroll
+          for (int a = 0; a < KT; ++a)
+#pragma unroll
+            for (int b = 0; b < KT; ++b) {
+              const int u = a * M + gi, v = b * M + gj;
+              out[(int64_t)u * D + v] = P[n][a][b][q];
+              if (i != j) out[(int64_t)v * D + u] = P[n][a][b][q];
+            }
+        }
+      }
+    }
+  };
+#pragma unroll 1
+  for (int it = 0; it <= io.iters; ++it) {
+    w = fresh_s(w0);
+    l = fresh_v(tid0) & 63;
+    C::publish(P, X, w, l);
+    __syncthreads();
+    tile4 U[MB], V[MB];
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        U[j][q] = C::kAllR || w < NR ? X[(16 * w + (l >> 4) + 4 * q) * LD + 16 * j + (l & 15)] : 0.0;
+      V[j] = U[j] + Rt[j];
+    }
+    if (w == 0) {
+      tile_store(sI, kDiagLd, 0, 0, V[0], l);
+      wave_sync();
+      chol16_inverse(sI, kDiagLd, l);
+    }
+    double quad = 0.0;
+    C::template eliminate<false>(P, U, V, quad, X, Lm, sI, nullptr, nullptr, w0, tid0);
+    if (it < io.iters) {
+      w = fresh_s(w0);
+      l = fresh_v(tid0) & 63;
+      C::predict(P, A, Q, M, w, l);
+      if (it + 1 == io.iters) write(io.X + k * DD);
+    } else {
+      write(io.cov + k * DD);
+    }
+    __syncthreads();  // X is read
+  }
 }
 
+// -S^-1 and log det S, S = H X H' + R: every step's noise, or (TIED) the run's tied noise
+template <bool TIED>
 __global__ __launch_bounds__(kT) void k_ih_sinv(StDims dm, IhIO io) {
   __shared__ double sS[kMaxM * kMaxM];
   __shared__ double row[2 * kMaxM];
   const int t = blockIdx.x, k = blockIdx.y, M = dm.M, D = dm.D, tid = threadIdx.x;
-  const int64_t kt = (int64_t)k * dm.T + t;
+  const int64_t kt = TIED ? k : (int64_t)k * dm.T + t;
   const double* X = io.X + (int64_t)k * D * D;
-  const double* Rt = io.R + kt * M * M;
-  for (int e = tid; e < M * M; e += kT) sS[e] = Rt[e] + X[(int64_t)(e / M) * D + e % M];
+  const double* R = (TIED ? io.Rt : io.R) + kt * M * M;
+  for (int e = tid; e < M * M; e += kT) sS[e] = R[e] + X[(int64_t)(e / M) * D + e % M];
   const double ld = wg_sweep_inv<kMaxM / 16, true>(sS, M, M, row);
-  for (int e = tid; e < M * M; e += kT) io.Sn[kt * M * M + e] = sS[e];
-  if (tid == 0) io.ldS[kt] = ld;
+  for (int e = tid; e < M * M; e += kT) (TIED ? io.STn : io.Sn)[kt * M * M + e] = sS[e];
+  if (tid == 0) (TIED ? io.ldT : io.ldS)[kt] = ld;
 }
 
+constexpr int kAhead = 4;  // steps that the mean recursions load ahead: memory latency is several steps
+
+// m_t = A m_{t-1} + X H' S_t^-1 (y_t - H A m_{t-1}), one workgroup per run: a chain of steps of two
+// short products each, bound by their latency.  Eight lanes share an inducing point: they hold
+// its row of X H' (all KT components) in registers, S_t^-1's row arrives kAhead steps before it
+// is used, and the predicted mean stays with them, so a step is two products, two three-stage
+// lane sums and two barriers.  1.2 us a step at M = 36 (4.5 us with one lane a row and S_t^-1 read on
+// the way).
 template <int KT>
-__global__ __launch_bounds__(kT) void k_ih_filter(StDims dm, StHyp hy, IhIO io) {
-  __shared__ double sm[kMaxD], mp[kMaxD], sv[kMaxM], su[kMaxM], red[4];
-  __shared__ double sA[KT * KT], sQ[KT * KT];
-  const int k = blockIdx.x, M = dm.M, D = dm.D, tid = threadIdx.x;
+__global__ __launch_bounds__(8 * kMaxM) void k_ih_filter(StDims dm, IhIO io) {
+  __shared__ double sv[kMaxM], su[kMaxM];
+  const int k = blockIdx.x, M = dm.M, D = dm.D, tid = threadIdx.x, a = tid >> 3, part = tid & 7;
+  constexpr int N = kMaxM / 8;
   const double* X = io.X + (int64_t)k * D * D;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  if (tid == 0) temporal_AQ<KT>(ls, var, io.step[k], sA, sQ);
-  for (int e = tid; e < D; e += kT) sm[e] = 0.0;
-  __syncthreads();
-  for (int t = 0; t < dm.T; ++t) {
-    const int64_t kt = (int64_t)k * dm.T + t;
-    if (tid < D) {
-      const int c = tid / M, a = tid % M;
-      double v = 0.0;
-      for (int p = 0; p < KT; ++p) v = fma(sA[c * KT + p], sm[p * M + a], v);
-      mp[tid] = v;
+  const bool row = a < M;
+  double A[KT][KT], xr[KT][N], sr[kAhead][N], yr[kAhead], mp[KT];
+#pragma unroll
+  for (int c = 0; c < KT; ++c) {
+    mp[c] = 0.0;
+#pragma unroll
+    for (int p = 0; p < KT; ++p) A[c][p] = io.aq[k * 2 * KT * KT + c * KT + p];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int i = part + 8 * n;
+      xr[c][n] = row && i < M ? X[(int64_t)(c * M + a) * D + i] : 0.0;
     }
-    __syncthreads();
-    if (tid < M) sv[tid] = io.y[kt * M + tid] - mp[tid];
-    __syncthreads();
-    const double* Sn = io.hetero ? io.Sn + kt * M * M : io.STn + (int64_t)k * M * M;  // -S^-1
-    double q = 0.0;
-    if (tid < M) {
-      double u = 0.0;
-      for (int j = 0; j < M; ++j) u = fma(-Sn[j * M + tid], sv[j], u);
-      su[tid] = u;
-      q = sv[tid] * u;
-    }
-    const double quad = wg_sum(q, red);
-    if (tid == 0) io.ell[kt] = -0.5 * (quad + M * kLog2Pi + (io.hetero ? io.ldS[kt] : io.ldT[k]));
-    if (tid < D) {
-      // X H' u: column i of X H' is row i of the (symmetric) X
-      double v = mp[tid];
-      for (int i = 0; i < M; ++i) v = fma(X[(int64_t)i * D + tid], su[i], v);
-      sm[tid] = v;
-      io.fmean[kt * D + tid] = v;
-    }
-    __syncthreads();
   }
+  const double* y = io.y + (int64_t)k * dm.T * M + (row ? a : 0);
+  // S_t^-1's row and y_{t+1}; past the end the last step's again, so that no branch (and no copy
+  // that waits for the load) stands between the load and its use
+  auto fetch = [&](int t, double (&s)[N], double& yt) {
+    t = min(t, dm.T - 1);
+    const double* Sn = io.hetero ? io.Sn + ((int64_t)k * dm.T + t) * M * M : io.STn + (int64_t)k * M * M;  // -S^-1
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int j = part + 8 * n;
+      s[n] = Sn[row && j < M ? a * M + j : 0];  // used as it comes: sv is 0 from M on
+    }
+    yt = y[(int64_t)min(t + 1, dm.T - 1) * M];
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) fetch(u, sr[u], yr[u]);
+  if (part == 0) {
+    sv[a] = row ? y[0] : 0.0;
+    su[a] = 0.0;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int t0 = 0; t0 < dm.T; t0 += kAhead) {
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b) {
+      const int t = t0 + b;
+      if (t >= dm.T) break;
+      double u = 0.0, u1 = 0.0;
+#pragma unroll
+      for (int n = 0; n < N; n += 2) {
+        u = fma(-sr[b][n], sv[part + 8 * n], u);
+        u1 = fma(-sr[b][n + 1], sv[part + 8 * n + 8], u1);
+      }
+      u += u1;
+      u += __shfl_xor(u, 1, 64);
+      u += __shfl_xor(u, 2, 64);
+      u += __shfl_xor(u, 4, 64);
+      if (part == 0 && row) su[a] = u;
+      const double yt = yr[b];
+      fetch(t + kAhead, sr[b], yr[b]);
+      __syncthreads();
+      double m[KT];
+#pragma unroll
+      for (int c = 0; c < KT; ++c) {
+        double v = 0.0, v1 = 0.0;
+#pragma unroll
+        for (int n = 0; n < N; n += 2) {
+          v = fma(xr[c][n], su[part + 8 * n], v);
+          v1 = fma(xr[c][n + 1], su[part + 8 * n + 8], v1);
+        }
+        v += v1;
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        v += __shfl_xor(v, 4, 64);
+        m[c] = mp[c] + v;
+      }
+      if (part == 0 && row) {
+#pragma unroll
+        for (int c = 0; c < KT; ++c) io.fmean[((int64_t)k * dm.T + t) * D + c * M + a] = m[c];
+      }
+#pragma unroll
+      for (int c = 0; c < KT; ++c) {
+        mp[c] = 0.0;
+#pragma unroll
+        for (int p = 0; p < KT; ++p) mp[c] = fma(A[c][p], m[p], mp[c]);
+      }
+      if (part == 0 && row) sv[a] = yt - mp[0];
+      __syncthreads();
+    }
+  }
+}
+
+// log N(y_t | H A m_{t-1}, S_t) of every step, one wavefront per (step, run)
+template <int KT>
+__global__ __launch_bounds__(64) void k_ih_ell(StDims dm, IhIO io) {
+  __shared__ double sv[kMaxM];
+  const int t = blockIdx.x, k = blockIdx.y, M = dm.M, D = dm.D, l = threadIdx.x;
+  const int64_t kt = (int64_t)k * dm.T + t;
+  double v = 0.0;
+  if (l < M) {
+    v = io.y[kt * M + l];
+    if (t > 0) {
+      for (int p = 0; p < KT; ++p) v = fma(-io.aq[k * 2 * KT * KT + p], io.fmean[(kt - 1) * D + p * M + l], v);
+    }
+  }
+  sv[l] = v;
+  __syncthreads();
+  const double* Sn = io.hetero ? io.Sn + kt * M * M : io.STn + (int64_t)k * M * M;  // -S^-1
+  double u = 0.0;
+  if (l < M) {
+#pragma unroll 8
+    for (int j = 0; j < M; ++j) u = fma(-Sn[j * M + l], sv[j], u);
+  }
+  double q = u * v;
+  for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o, 64);
+  if (l == 0) io.ell[kt] = -0.5 * (q + M * kLog2Pi + (io.hetero ? io.ldS[kt] : io.ldT[k]));
 }
 
 struct IhSmIO {
-  const double* step;   // [K]
+  const double* aq;     // [K, 2 KT^2]
   const double* fmean;  // [K,T,D]
-  const double* X;      // [K,D,D] filter Riccati solution
-  const double* cov;    // [K,D,D]
-  double* Xs;           // [K,D,D] smoother Riccati solution: start in, result out
-  double* G;            // [K,D,D] gain
-  double* W1;           // [K,D,D] scratch
-  double* W2;           // [K,D,D] scratch
+  const double* Xs;     // [K,D,D] smoother Riccati solution
+  const double* G;      // [K,D,D] gain
   double* pm;           // optional [K,T,M]
   double* pP;           // optional [K,T,M,M]
   double* smean;        // optional [K,T,D]
-  int32_t iters;
 };
 
+// sm_t = fm_t + G (sm_{t+1} - A fm_t) from sm = fm_{T-1}, one workgroup per run, bound by the latency
+// of the chain: four lanes a row with their quarter of G in registers, the filtered means loaded
+// kAhead steps before they are used, one barrier a step.  0.7 us a step at D = 72.
 template <int KT>
-__global__ __launch_bounds__(kT) void k_ih_smoother(StDims dm, StHyp hy, IhSmIO io) {
-  extern __shared__ double smem[];
-  const int k = blockIdx.x, M = dm.M, D = dm.D, tid = threadIdx.x;
-  double* pan = smem;                    // 2*kPK*kPS
-  double* sL = pan + 2 * kPK * kPS;      // D*D
-  double* row = sL + kMaxD * kMaxD;      // 2 D
-  double* ms = row + 2 * kMaxD;          // D
-  double* mf = ms + kMaxD;               // D
-  double* dv = mf + kMaxD;               // D
-  double* tmp = dv + kMaxD;              // D
-  __shared__ double sA[KT * KT], sQ[KT * KT];
-  const int64_t DD = (int64_t)D * D;
-  const double* X = io.X + k * DD;
-  const double* cov = io.cov + k * DD;
-  double* Xs = io.Xs + k * DD;
-  double* G = io.G + k * DD;
-  double* W1 = io.W1 + k * DD;
-  double* W2 = io.W2 + k * DD;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  if (tid == 0) temporal_AQ<KT>(ls, var, io.step[k], sA, sQ);
-  for (int64_t e = tid; e < DD; e += kT) sL[e] = X[e];
-  (void)wg_sweep_inv<kMaxD / 16, false>(sL, D, D, row);  // sL = -X^-1
-  // W1 = A' X^-1 ; G = cov W1
-  for (int64_t e = tid; e < DD; e += kT) {
-    const int r = (int)(e / D), j = (int)(e % D), c = r / M, m = r % M;
-    double v = 0.0;
-    for (int a = 0; a < KT; ++a) v = fma(-sA[a * KT + c], sL[(int64_t)(a * M + m) * D + j], v);
-    W1[e] = v;
+__global__ __launch_bounds__(4 * kMaxD) void k_ih_means(StDims dm, IhSmIO io) {
+  __shared__ double sd[2][kMaxD];
+  const int k = blockIdx.x, M = dm.M, D = dm.D, T = dm.T, tid = threadIdx.x, r = tid >> 2, part = tid & 3;
+  constexpr int N = kMaxD / 4;
+  const bool row = r < D;
+  const int c = row ? r / M : 0, a = row ? r % M : 0;
+  double g[N], Ar[KT];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int j = part + 4 * n;
+    g[n] = row && j < D ? io.G[(int64_t)k * D * D + (int64_t)r * D + j] : 0.0;
   }
-  wg_gemm(D, D, D, 1.0, MatRef{cov, D, 1}, MatRef{W1, D, 1}, 0.0, G, D, pan);
-  // Qd = cov - G X G' -> W2
-  wg_gemm(D, D, D, 1.0, MatRef{G, D, 1}, MatRef{X, D, 1}, 0.0, W1, D, pan);
-  for (int64_t e = tid; e < DD; e += kT) W2[e] = cov[e];
-  wg_gemm(D, D, D, -1.0, MatRef{W1, D, 1}, MatRef{G, 1, D}, 1.0, W2, D, pan);
-  for (int it = 0; it < io.iters; ++it) {
-    wg_gemm(D, D, D, 1.0, MatRef{G, D, 1}, MatRef{Xs, D, 1}, 0.0, W1, D, pan);
-    for (int64_t e = tid; e < DD; e += kT) Xs[e] = W2[e];
-    wg_gemm(D, D, D, 1.0, MatRef{W1, D, 1}, MatRef{G, 1, D}, 1.0, Xs, D, pan);
-  }
-  // G' into LDS for the mean recursion
-  for (int64_t e = tid; e < DD; e += kT) sL[(e % D) * D + e / D] = G[e];
-  {
-    const int64_t kt = (int64_t)k * dm.T + dm.T - 1;
-    for (int e = tid; e < D; e += kT) ms[e] = io.fmean[kt * D + e];
+#pragma unroll
+  for (int p = 0; p < KT; ++p) Ar[p] = io.aq[k * 2 * KT * KT + c * KT + p];
+  const double* fm = io.fmean + (int64_t)k * T * D;
+  double f[kAhead][KT];  // filtered means of the row's components, kAhead steps
+  auto fetch = [&](int t, double (&x)[KT]) {
+#pragma unroll
+    for (int p = 0; p < KT; ++p) x[p] = fm[(int64_t)(t > 0 ? t : 0) * D + p * M + a];
+  };
+  auto delta = [&](double ms, const double (&x)[KT]) {  // sm_{t+1} - A fm_t
+#pragma unroll
+    for (int p = 0; p < KT; ++p) ms = fma(-Ar[p], x[p], ms);
+    return row ? ms : 0.0;
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) fetch(T - 1 - u, f[u]);
+  int cur = 0;
+  if (part == 0) {
+    double own = f[0][0];
+#pragma unroll
+    for (int p = 1; p < KT; ++p) own = c == p ? f[0][p] : own;
+    sd[0][r] = delta(own, f[0]);
   }
   __syncthreads();
-  for (int t = dm.T - 1; t >= 0; --t) {
-    const int64_t kt = (int64_t)k * dm.T + t;
-    for (int e = tid; e < D; e += kT) mf[e] = io.fmean[kt * D + e];
-    __syncthreads();
-    if (tid < D) {
-      const int c = tid / M, a = tid % M;
-      double v = 0.0;
-      for (int p = 0; p < KT; ++p) v = fma(sA[c * KT + p], mf[p * M + a], v);
-      dv[tid] = ms[tid] - v;
+#pragma unroll 1
+  for (int s0 = 0; s0 < T; s0 += kAhead) {
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b) {
+      const int t = T - 1 - s0 - b;
+      if (t < 0) break;
+      double v = 0.0, v1 = 0.0;
+#pragma unroll
+      for (int n = 0; n < N; n += 2) {
+        v = fma(g[n], sd[cur][part + 4 * n], v);
+        v1 = fma(g[n + 1], sd[cur][part + 4 * n + 4], v1);
+      }
+      v += v1;
+      v += __shfl_xor(v, 1, 64);
+      v += __shfl_xor(v, 2, 64);
+      double ms = f[b][0];
+#pragma unroll
+      for (int p = 1; p < KT; ++p) ms = c == p ? f[b][p] : ms;
+      ms += v;
+      if (part == 0 && row) {
+        const int64_t kt = (int64_t)k * T + t;
+        if (io.smean) io.smean[kt * D + r] = ms;
+        if (io.pm && r < M) io.pm[kt * M + r] = ms;
+      }
+      fetch(t - kAhead, f[b]);
+      cur ^= 1;
+      if (part == 0) sd[cur][r] = delta(ms, f[(b + 1) % kAhead]);
+      __syncthreads();
     }
-    __syncthreads();
-    if (tid < D) {
-      double v = mf[tid];
-      for (int j = 0; j < D; ++j) v = fma(sL[(int64_t)j * D + tid], dv[j], v);
-      tmp[tid] = v;
-    }
-    __syncthreads();
-    if (tid < D) {
-      ms[tid] = tmp[tid];
-      if (io.smean) io.smean[kt * D + tid] = tmp[tid];
-      if (io.pm && tid < M) io.pm[kt * M + tid] = tmp[tid];
-    }
-    if (io.pP)
-      for (int e = tid; e < M * M; e += kT) io.pP[kt * M * M + e] = Xs[(int64_t)(e / M) * D + e % M];
-    __syncthreads();
   }
+}
+
+// H X_s H' at every step
+__global__ __launch_bounds__(kT) void k_ih_spread(StDims dm, IhSmIO io) {
+  const int k = blockIdx.y, M = dm.M, D = dm.D;
+  const int64_t kt = (int64_t)k * dm.T + blockIdx.x;
+  for (int e = threadIdx.x; e < M * M; e += kT)
+    io.pP[kt * M * M + e] = io.Xs[(int64_t)k * D * D + (int64_t)(e / M) * D + e % M];
 }
 
 // ---------------------------------------------------------------------------
@@ -2835,10 +3061,8 @@ __global__ __launch_bounds__(kT) void k_st_predict(StDims dm, StHyp hy, StPredIO
   }
 }
 
-constexpr size_t kSmootherSmem = sizeof(double) * (2 * kPK * kPS + kMaxD * kMaxD + 6 * kMaxD);
 constexpr size_t kPseudoSmem = sizeof(double) * (2 * kPK * kPS + kMaxM * kMaxM + 3 * kMaxM);
 constexpr size_t kTiedSmem = sizeof(double) * (2 * kPK * kPS + kMaxM * kMaxM);
-constexpr size_t kIhDareSmem = sizeof(double) * (2 * kPK * kPS + 2 * kMaxM * kMaxM + 2 * kMaxM);
 constexpr size_t kSitesSmem =
     sizeof(double) * (2 * kMaxM * kSLd + 5 * kMaxM + 4 * 32 + 4);
 static_assert(2 * kSitesSmem <= 160 * 1024, "two workgroups of k_st_sites a CU");
@@ -2867,7 +3091,10 @@ StHyp make_hyp(const bn_st_hypers* h) { return StHyp{h->ls_t, h->var_t, h->var_s
 template <int KT, int MB>
 int smoother_attr() {
   const int n = (int)sizeof(double) * StTiles<KT, MB>::SMEM;
-  for (const void* f : {(const void*)k_st_gains<KT, MB>, (const void*)k_st_chain<KT, MB>,
+  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_dare<KT, MB>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)sizeof(double) * filter_smem(KT, MB)));
+  for (const void* f : {(const void*)k_st_gains<KT, MB, false>, (const void*)k_st_gains<KT, MB, true>,
+                        (const void*)k_st_chain<KT, MB>, (const void*)k_st_smoother<KT, MB, ST_STEADY>,
                         (const void*)k_st_smoother<KT, MB, ST_WALK>, (const void*)k_st_smoother<KT, MB, ST_COMPOSE>,
                         (const void*)k_st_smoother<KT, MB, ST_JOIN>})
     ST_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, n));
@@ -2900,14 +3127,6 @@ int set_smem_limits() {
   ST_SITES_ATTR1(KERNEL, MT, MD, LIK_STUDENTS_T, N)
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_mf_pseudo, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kPseudoSmem));
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_dare<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kIhDareSmem));
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_dare<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kIhDareSmem));
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_smoother<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kSmootherSmem));
-  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_ih_smoother<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)kSmootherSmem));
   ST_SITES_ATTR(k_st_sites, M_VI, BN_ST_UPDATE, kSitesSmem);
   ST_SITES_ATTR(k_st_sites, M_VI, BN_ST_ENERGY, kSitesSmem);
   ST_SITES_ATTR1(k_st_sites, M_VI, BN_ST_PROJECT, 0, kSitesSmem);
@@ -2965,8 +3184,8 @@ int launch_st_smoother(hipStream_t st, StDims dm, StHyp hy, const double* aq, co
     io.t0 = t1 > io.tb ? t1 - io.tb : 0;
     io.nb = t1 - io.t0;
     io.nc = smoother_chunks(dm, io.nb);
-    const StGainIO gi{aq, fmean, fcov, io.rec, io.t0, io.tb};
-    hipLaunchKernelGGL((k_st_gains<KT, MB>), dim3(io.nb, dm.K), dim3(nt), smem, st, dm, gi);
+    const StGainIO gi{aq, fmean, fcov, io.rec, io.t0, io.tb, nullptr, nullptr};
+    hipLaunchKernelGGL((k_st_gains<KT, MB, false>), dim3(io.nb, dm.K), dim3(nt), smem, st, dm, gi);
     if (io.nc > 1) {
       hipLaunchKernelGGL((k_st_chain<KT, MB>), dim3(io.nc - 1, dm.K), dim3(nt), smem, st, io);
       hipLaunchKernelGGL((k_st_smoother<KT, MB, ST_COMPOSE>), dim3(io.nc - 1, dm.K), dim3(nt), smem, st, dm, io);
@@ -2988,6 +3207,50 @@ int launch_st_smoother(hipStream_t st, StDims dm, StHyp hy, const double* dt, do
     case 2: return launch_st_smoother<KT, 2>(st, dm, hy, aq, fmean, fcov, io);
     case 3: return launch_st_smoother<KT, 3>(st, dm, hy, aq, fmean, fcov, io);
     default: return launch_st_smoother<KT, 4>(st, dm, hy, aq, fmean, fcov, io);
+  }
+}
+
+// Doubles at the head of the infinite-horizon workspace: transitions, the smoother's map and gain.
+int64_t ih_head(const StDims& dm) {
+  return (int64_t)dm.K * (2 * dm.KT * dm.KT + map_doubles(dm) + (int64_t)dm.D * dm.D);
+}
+
+// The transition of each run's step: one step a run.
+void launch_ih_transitions(hipStream_t st, StDims dm, StHyp hy, const double* step, double* aq) {
+  dm.T = 1;
+  if (dm.KT == 1) launch_st_transitions<1>(st, dm, hy, step, aq);
+  else launch_st_transitions<2>(st, dm, hy, step, aq);
+}
+
+template <int KT, int MB>
+void launch_ih_dare(hipStream_t st, StDims dm, IhIO io) {
+  hipLaunchKernelGGL((k_ih_dare<KT, MB>), dim3(dm.K), dim3(128 * MB), sizeof(double) * filter_smem(KT, MB), st, dm, io);
+}
+template <int KT>
+void launch_ih_dare(hipStream_t st, StDims dm, IhIO io) {
+  switch ((dm.M + 15) / 16) {
+    case 1: return launch_ih_dare<KT, 1>(st, dm, io);
+    case 2: return launch_ih_dare<KT, 2>(st, dm, io);
+    case 3: return launch_ih_dare<KT, 3>(st, dm, io);
+    default: return launch_ih_dare<KT, 4>(st, dm, io);
+  }
+}
+
+template <int KT, int MB>
+void launch_ih_smoother(hipStream_t st, StDims dm, StGainIO gi, StSmootherIO si) {
+  using S = StTiles<KT, MB>;
+  const size_t smem = sizeof(double) * S::SMEM;
+  hipLaunchKernelGGL((k_st_gains<KT, MB, true>), dim3(1, dm.K), dim3(64 * S::NR), smem, st, dm, gi);
+  if (si.iters > 0)
+    hipLaunchKernelGGL((k_st_smoother<KT, MB, ST_STEADY>), dim3(1, dm.K), dim3(64 * S::NR), smem, st, dm, si);
+}
+template <int KT>
+void launch_ih_smoother(hipStream_t st, StDims dm, StGainIO gi, StSmootherIO si) {
+  switch ((dm.M + 15) / 16) {
+    case 1: return launch_ih_smoother<KT, 1>(st, dm, gi, si);
+    case 2: return launch_ih_smoother<KT, 2>(st, dm, gi, si);
+    case 3: return launch_ih_smoother<KT, 3>(st, dm, gi, si);
+    default: return launch_ih_smoother<KT, 4>(st, dm, gi, si);
   }
 }
 
@@ -3341,8 +3604,8 @@ int bn_mf_smoother(const bn_st_dims* dims, const bn_st_hypers* hyp, const double
 int64_t bn_ih_workspace_bytes(const bn_st_dims* dims, int32_t heteroscedastic) {
   StDims dm;
   if (check_dims(dims, dm) != BN_OK) return -1;
-  const int64_t K = dm.K, D = dm.D, M = dm.M, T = dm.T;
-  int64_t n = 3 * K * D * D + K * M * M + K + K * kTiedParts * M * M;
+  const int64_t K = dm.K, M = dm.M, T = dm.T;
+  int64_t n = ih_head(dm) + K * M * M + K + K * kTiedParts * M * M;
   if (heteroscedastic) n += K * T * M * M + K * T;
   return n * (int64_t)sizeof(double) + 256;
 }
@@ -3352,8 +3615,8 @@ int bn_ih_tied(const bn_st_dims* dims, const double* Lw, double* noise_tied, voi
   if (int rc = check_dims(dims, dm)) return rc;
   if (!Lw || !noise_tied || !workspace) return st_fail(BN_EINVAL, "NULL argument to bn_ih_tied");
   // partial sums after bn_ih_filter's regions (see bn_ih_workspace_bytes)
-  const int64_t K = dm.K, D = dm.D, M = dm.M;
-  double* part = (double*)workspace + 3 * K * D * D + K * M * M + K;
+  const int64_t K = dm.K, M = dm.M;
+  double* part = (double*)workspace + ih_head(dm) + K * M * M + K;
   hipStream_t st = (hipStream_t)stream;
   BN_TIMED(KID_IH_TIED, st);
   hipLaunchKernelGGL(k_ih_tied_part, dim3(kTiedParts, dm.K), dim3(kT), kTiedSmem, st, dm, Lw, part);
@@ -3374,18 +3637,16 @@ int bn_ih_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, const double* 
     return st_fail(BN_EINVAL, "NULL argument to bn_ih_filter");
   if (iters < 0) return st_fail(BN_EINVAL, "bn_ih_filter: iters must be >= 0");
   if (int rc = set_smem_limits()) return rc;
-  const int64_t K = dm.K, D = dm.D, M = dm.M;
+  const int64_t K = dm.K, M = dm.M;
   double* ws = (double*)workspace;
   IhIO io{};
-  io.step = step;
+  io.aq = ws;
   io.y = y;
   io.R = noise;
   io.Rt = noise_tied;
   io.X = dare;
   io.cov = filter_cov;
-  io.W1 = ws;
-  io.W2 = ws + K * D * D;
-  io.STn = ws + 3 * K * D * D;
+  io.STn = ws + ih_head(dm);
   io.ldT = io.STn + K * M * M;
   io.Sn = heteroscedastic ? io.ldT + K + K * kTiedParts * M * M : nullptr;
   io.ldS = heteroscedastic ? io.Sn + K * dm.T * M * M : nullptr;
@@ -3397,19 +3658,26 @@ int bn_ih_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, const double* 
   hipStream_t st = (hipStream_t)stream;
   {
     BN_TIMED(KID_IH_DARE, st);
-    if (dm.KT == 1) hipLaunchKernelGGL(k_ih_dare<1>, dim3(dm.K), dim3(kT), kIhDareSmem, st, dm, hy, io);
-    else hipLaunchKernelGGL(k_ih_dare<2>, dim3(dm.K), dim3(kT), kIhDareSmem, st, dm, hy, io);
+    launch_ih_transitions(st, dm, hy, step, ws);
+    if (dm.KT == 1) launch_ih_dare<1>(st, dm, io);
+    else launch_ih_dare<2>(st, dm, io);
     ST_HIP_CHECK(hipGetLastError());
   }
-  if (heteroscedastic) {
+  {
     BN_TIMED(KID_IH_SINV, st);
-    hipLaunchKernelGGL(k_ih_sinv, dim3(dm.T, dm.K), dim3(kT), 0, st, dm, io);
+    if (heteroscedastic) hipLaunchKernelGGL(k_ih_sinv<false>, dim3(dm.T, dm.K), dim3(kT), 0, st, dm, io);
+    else hipLaunchKernelGGL(k_ih_sinv<true>, dim3(1, dm.K), dim3(kT), 0, st, dm, io);
     ST_HIP_CHECK(hipGetLastError());
   }
   {
     BN_TIMED(KID_IH_FILTER, st);
-    if (dm.KT == 1) hipLaunchKernelGGL(k_ih_filter<1>, dim3(dm.K), dim3(kT), 0, st, dm, hy, io);
-    else hipLaunchKernelGGL(k_ih_filter<2>, dim3(dm.K), dim3(kT), 0, st, dm, hy, io);
+    if (dm.KT == 1) {
+      hipLaunchKernelGGL(k_ih_filter<1>, dim3(dm.K), dim3(8 * kMaxM), 0, st, dm, io);
+      hipLaunchKernelGGL(k_ih_ell<1>, dim3(dm.T, dm.K), dim3(64), 0, st, dm, io);
+    } else {
+      hipLaunchKernelGGL(k_ih_filter<2>, dim3(dm.K), dim3(8 * kMaxM), 0, st, dm, io);
+      hipLaunchKernelGGL(k_ih_ell<2>, dim3(dm.T, dm.K), dim3(64), 0, st, dm, io);
+    }
     ST_HIP_CHECK(hipGetLastError());
   }
   {
@@ -3430,27 +3698,29 @@ int bn_ih_smoother(const bn_st_dims* dims, const bn_st_hypers* hyp, const double
     return st_fail(BN_EINVAL, "NULL argument to bn_ih_smoother");
   if (iters < 0) return st_fail(BN_EINVAL, "bn_ih_smoother: iters must be >= 0");
   if (int rc = set_smem_limits()) return rc;
-  const int64_t K = dm.K, D = dm.D;
+  const int64_t K = dm.K;
   double* ws = (double*)workspace;
-  IhSmIO io{};
-  io.step = step;
-  io.fmean = filter_mean;
-  io.X = dare;
-  io.cov = filter_cov;
-  io.Xs = dare_smoother;
-  io.G = gain ? gain : ws + 2 * K * D * D;
-  io.W1 = ws;
-  io.W2 = ws + K * D * D;
-  io.pm = post_mean;
-  io.pP = post_cov;
-  io.smean = smooth_mean;
-  io.iters = iters;
+  double* rec = ws + K * 2 * dm.KT * dm.KT;
+  double* G = gain ? gain : rec + K * map_doubles(dm);
+  const StGainIO gi{ws, nullptr, filter_cov, rec, 0, 1, dare, G};
+  StSmootherIO si{};
+  si.rec = rec;
+  si.tb = 1;
+  si.xs = dare_smoother;
+  si.iters = iters;
+  const IhSmIO io{ws, filter_mean, dare_smoother, G, post_mean, post_cov, smooth_mean};
+  const StHyp hy = make_hyp(hyp);
   hipStream_t st = (hipStream_t)stream;
   BN_TIMED(KID_IH_SMOOTHER, st);
-  if (dm.KT == 1)
-    hipLaunchKernelGGL(k_ih_smoother<1>, dim3(dm.K), dim3(kT), kSmootherSmem, st, dm, make_hyp(hyp), io);
-  else
-    hipLaunchKernelGGL(k_ih_smoother<2>, dim3(dm.K), dim3(kT), kSmootherSmem, st, dm, make_hyp(hyp), io);
+  launch_ih_transitions(st, dm, hy, step, ws);
+  if (dm.KT == 1) {
+    launch_ih_smoother<1>(st, dm, gi, si);
+    hipLaunchKernelGGL(k_ih_means<1>, dim3(dm.K), dim3(4 * kMaxD), 0, st, dm, io);
+  } else {
+    launch_ih_smoother<2>(st, dm, gi, si);
+    hipLaunchKernelGGL(k_ih_means<2>, dim3(dm.K), dim3(4 * kMaxD), 0, st, dm, io);
+  }
+  if (post_cov) hipLaunchKernelGGL(k_ih_spread, dim3(dm.T, dm.K), dim3(kT), 0, st, dm, io);
   ST_HIP_CHECK(hipGetLastError());
   return BN_OK;
 }

@@ -151,8 +151,7 @@ class SpaceTimeMarkovGP:
         return h
 
     # ---- sites ---------------------------------------------------------------------------
-    # the filter takes the projection in whitened form; the forms that invert it explicitly
-    # need bn_st_sites' fixed order of summation
+    # bn_st_sites_whitened, unless rounding in the projection comes out magnified (the mean-field form)
     _whitened = True
 
     def _sites(self, mode, lr=1.0, cubature=None, ensure_psd=True, terms=None, batch=None):
@@ -669,7 +668,6 @@ class SpaceTimeInfiniteHorizonGP(SpaceTimeMarkovGP):
     advance with each call.  Heteroscedastic (per-step gains) unless the likelihood is
     Gaussian with no missing data (basemodels.py:1270).  `parallel` is accepted: both of the
     reference's forms compute the same means."""
-    _whitened = False
 
     def __init__(self, kernel, likelihood, X, Y, R, dare_iters=20, parallel=None, device=None):
         self.dare_iters = int(dare_iters)
