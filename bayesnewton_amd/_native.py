@@ -60,6 +60,7 @@ SIGNATURES = {
     "bn_workspace_bytes": (i64, [vp, vp]),
     "bn_plan_gather_f32": (i32, [vp, vp, vp, i32, f32, vp]),
     "bn_plan_scatter_f32": (i32, [vp, vp, vp, i32, vp]),
+    "bn_plan_scatter_planes": (i32, [vp, vp, vp, i32, vp]),
     "bn_plan_gather_f64": (i32, [vp, vp, vp, i32, f64, vp]),
     "bn_plan_scatter_f64": (i32, [vp, vp, vp, i32, vp]),
     "bn_plan_gather_u8": (i32, [vp, vp, vp, u8, vp]),

@@ -686,6 +686,17 @@ __global__ void k_scatter_f32(PlanView pl, const float* __restrict__ src, float*
   for (int32_t f = 0; f < width; ++f) dst[csr * width + f] = src[f * pl.n_slots + slot];
 }
 
+// Planes of FP32 words to FP64 rows, one field after the other: what a model returns (its arrays
+// are FP64) in one launch instead of one per field and one more per conversion.
+__global__ void k_scatter_planes(PlanView pl, const float* __restrict__ src, double* __restrict__ dst, int32_t width,
+                                 int64_t n_steps) {
+  const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (slot >= pl.n_slots) return;
+  int64_t csr;
+  if (!slot_to_step(pl, slot, csr)) return;
+  for (int32_t f = 0; f < width; ++f) dst[f * n_steps + csr] = (double)src[f * pl.n_slots + slot];
+}
+
 template <int K1, int K2>
 __global__ void k_discretise(HyperView hv, int64_t n, const float* __restrict__ dt, float* __restrict__ A,
                              float* __restrict__ Q) {
@@ -1375,6 +1386,16 @@ int bn_plan_scatter_f32(const bn_plan* plan, const float* src, float* dst, int32
   const int64_t n = plan->host.n_slots;
   hipLaunchKernelGGL(k_scatter_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, plan->view,
                      src, dst, width);
+  BN_HIP_CHECK(hipGetLastError());
+  return BN_OK;
+}
+
+int bn_plan_scatter_planes(const bn_plan* plan, const float* src, double* dst, int32_t width, void* stream) {
+  if (check_plan(plan)) return BN_EINVAL;
+  if (width < 1) return fail(BN_EINVAL, "width must be >= 1");
+  const int64_t n = plan->host.n_slots;
+  hipLaunchKernelGGL(k_scatter_planes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, plan->view,
+                     src, dst, width, plan->host.n_steps);
   BN_HIP_CHECK(hipGetLastError());
   return BN_OK;
 }

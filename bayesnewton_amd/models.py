@@ -260,11 +260,11 @@ class MarkovGaussianProcess:
 
     @property
     def posterior_mean(self):
-        return self.plan.scatter(self._pm[None]).to(torch.float64).reshape(-1, 1, 1)
+        return self.plan.scatter_planes(self._pm[None]).reshape(-1, 1, 1)
 
     @property
     def posterior_variance(self):
-        return self.plan.scatter(self._pv[None]).to(torch.float64).reshape(-1, 1, 1)
+        return self.plan.scatter_planes(self._pv[None]).reshape(-1, 1, 1)
 
     # ---- inference (inference.py:65-90) ----------------------------------------------
     def _batch_mask(self, batch_ind):
@@ -292,12 +292,8 @@ class MarkovGaussianProcess:
         self._ensure_posterior()
         P = self.plan
         dev = self.device
-        if return_terms:
-            om = torch.empty(P.n_slots, dtype=torch.float32, device=dev)
-            oj = torch.empty_like(om)
-            oh = torch.empty_like(om)
-        else:
-            om = oj = oh = None
+        planes = torch.empty((3, P.n_slots), dtype=torch.float32, device=dev) if return_terms else (None,) * 3
+        om, oj, oh = planes
         lik = self.likelihood.desc()
         nat.check(nat.lib().bn_site_update(
             P.handle, ctypes.byref(self._desc), ctypes.byref(lik), self.method, cub.num_points(cubature), float(lr),
@@ -308,10 +304,11 @@ class MarkovGaussianProcess:
             nat.stream_ptr()))
         self._sites_version += 1
         self.update_posterior()
-        diff1 = self._d1.sum() / self.num_data
-        diff2 = self._d2.sum() / self.num_data
+        one = self.num_series == 1
+        diff1 = (self._d1[0] if one else self._d1.sum()) / self.num_data
+        diff2 = (self._d2[0] if one else self._d2.sum()) / self.num_data
         if return_terms:
-            terms = tuple(P.scatter(a[None]).to(torch.float64).reshape(-1, 1, 1) for a in (om, oj, oh))
+            terms = tuple(a.reshape(-1, 1, 1) for a in P.scatter_planes(planes))
             if batch is not None:
                 sel = torch.as_tensor(np.asarray(batch_ind).reshape(-1), dtype=torch.int64, device=dev)
                 terms = tuple(a[sel] for a in terms)

@@ -107,6 +107,13 @@ class SeriesPlan:
         nat.check(nat.lib().bn_plan_gather_u8(self._h, nat.ptr(m), nat.ptr(out), 1, nat.stream_ptr()))
         return out
 
+    def scatter_planes(self, t):
+        """tiled float32 [w, n_slots] -> float64 [w, N]."""
+        t = t.contiguous()
+        out = torch.empty((t.shape[0], self.n_steps), dtype=torch.float64, device=self.device)
+        nat.check(nat.lib().bn_plan_scatter_planes(self._h, nat.ptr(t), nat.ptr(out), t.shape[0], nat.stream_ptr()))
+        return out
+
     def scatter(self, t):
         """tiled [w, n_slots] -> [N, w]."""
         if t.dim() == 1:

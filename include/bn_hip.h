@@ -119,6 +119,8 @@ int64_t bn_workspace_bytes(const bn_plan *plan, const bn_kernel_desc *kern);
  * tiled planes of num_slots words each. */
 int bn_plan_gather_f32(const bn_plan *plan, const float *src, float *dst, int32_t width, float pad, void *stream);
 int bn_plan_scatter_f32(const bn_plan *plan, const float *src, float *dst, int32_t width, void *stream);
+/* tiled float planes src [width, n_slots] -> double dst [width, n_steps] (every field contiguous) */
+int bn_plan_scatter_planes(const bn_plan *plan, const float *src, double *dst, int32_t width, void *stream);
 int bn_plan_gather_f64(const bn_plan *plan, const double *src, double *dst, int32_t width, double pad, void *stream);
 int bn_plan_scatter_f64(const bn_plan *plan, const double *src, double *dst, int32_t width, void *stream);
 int bn_plan_gather_u8(const bn_plan *plan, const uint8_t *src, uint8_t *dst, uint8_t pad, void *stream);

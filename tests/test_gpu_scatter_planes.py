@@ -1,0 +1,20 @@
+"""The conversion of float32 planes to float64 rows of the series."""
+import numpy as np
+import pytest
+import torch
+
+from bayesnewton_amd.plan import SeriesPlan
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths,chunk", [([1], 1), ([70, 1, 33], 8), ([0, 5, 0], 4), ([300, 129], 128)])
+@pytest.mark.parametrize("w", [1, 3])
+def test_planes_to_double_rows(lengths, chunk, w):
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    plan = SeriesPlan(off, chunk_len=chunk)
+    x = torch.randn(int(off[-1]), w, device="cuda")
+    t = plan.gather(x, pad=7.0)
+    out = plan.scatter_planes(t)
+    assert out.dtype == torch.float64 and out.shape == (w, int(off[-1]))
+    assert torch.equal(out, plan.scatter(t).double().t())
+    assert torch.equal(out, x.double().t())
