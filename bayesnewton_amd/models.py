@@ -23,7 +23,7 @@ from . import cubature as cub
 from . import ops
 from . import spacetime
 from .kernels import SpatioTemporalKernel
-from .plan import SeriesPlan, default_chunk_len
+from .plan import SeriesPlan, model_chunk_len
 
 
 def input_admin(t, y):
@@ -124,7 +124,7 @@ class MarkovGaussianProcess:
         dev = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
         self.device = dev
         if chunk_len is None:
-            chunk_len = default_chunk_len(lens, self.parallel)
+            chunk_len = model_chunk_len(lens, self.parallel)
         self._desc = kernel.desc()
         n_comp = self._desc.n_comp
         if ls is not None or var is not None:

@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _native as nat
-from .plan import SeriesPlan
+from .plan import SeriesPlan, model_chunk_len
 
 
 def _device():
@@ -50,7 +50,7 @@ def discretise(kernel, dt):
 
 
 def _single_plan(n, parallel, dev):
-    return SeriesPlan(np.array([0, n], dtype=np.int64), parallel=parallel, device=dev)
+    return SeriesPlan(np.array([0, n], dtype=np.int64), chunk_len=model_chunk_len([n], parallel), device=dev)
 
 
 def kalman_filter(dt, kernel, y, noise_cov, mask=None, parallel=False, return_predict=False, plan=None,

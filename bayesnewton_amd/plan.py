@@ -27,6 +27,33 @@ def default_chunk_len(lengths, parallel=True):
     return c
 
 
+def model_chunk_len(lengths, parallel=True):
+    """Chunk length of a model's (or a single operation's) own plan.
+
+    The lane-per-chunk kernels take about 1 us a step of the longest chunk and a few
+    wavefronts leave the chip idle, while the scans over the chunks' elements grow with the
+    logarithm of their number.  Measured on MI355X (fused pass, chunk 32 -> this rule):
+    10,000 steps 115 -> 66 us (Matern52) and 213 -> 147 us (Matern52 + Matern32), flat
+    between 2 and 8; 200,000 steps 246 -> 206 us; 256 series with 276,000 steps
+    204 -> 163 us; 2000 series with 3.3 M steps 429 -> 378 us (8 steps a chunk would take
+    835 us: past about 60,000 chunks the chip is full, and short chunks only add scan
+    work); 4096 series with 15.7 M steps best at 123-128.
+    Below 4096 steps in all the length stays 32, though 300 steps would take 47 us instead
+    of 100: the float32 rows of the smoother are rounded from the chunk's end onwards, and in
+    the energy of so few steps another length moves that rounding by as much as its whole
+    error.  Series of at most 32 steps stay in one chunk each: no scan at all."""
+    if not parallel:
+        return default_chunk_len(lengths, parallel)
+    lengths = np.asarray(lengths, dtype=np.int64)
+    nmax = max(int(lengths.max()) if lengths.size else 1, 1)
+    total = int(lengths.sum())
+    if nmax <= 32:
+        return nmax
+    if total < 4096:
+        return 32
+    return max(8, -(-nmax // (128 * 128)), min(128, -(-total // 57344)))
+
+
 class SeriesPlan:
     """Device-side decomposition of B sorted series (CSR offsets) into chunks.
 

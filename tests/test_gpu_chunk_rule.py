@@ -1,0 +1,37 @@
+"""The chunk length that models and single operations choose, at the edges of its rule."""
+import numpy as np
+import pytest
+import torch
+
+from bayesnewton_amd.plan import default_chunk_len, model_chunk_len
+
+
+@pytest.mark.parametrize("lengths", [[], [0], [1], [31, 32], [33], [4095], [4000, 96], [131072], [131073], [458753],
+                                     [3840] * 4096, [40_000_000], [5_000_000] * 10])
+def test_rule_bounds_each_series_to_its_scan(lengths):
+    c = model_chunk_len(lengths)
+    nmax = max([1] + lengths)
+    assert 1 <= c <= max(32, 128, -(-nmax // 16384))
+    assert -(-nmax // c) <= 128 * 128
+    if nmax <= 32:
+        assert c == nmax
+    elif sum(lengths) < 4096:
+        assert c == default_chunk_len(lengths)
+    assert model_chunk_len(lengths, parallel=False) == default_chunk_len(lengths, parallel=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 32, 33, 4095, 4096, 4097, 131073])
+def test_parallel_filter_at_the_rule_edges_equals_the_sequential_one(n):
+    """FP64 on both sides: the two orders of the same sums agree to 1e-9."""
+    from bayesnewton_amd import kernels as K, ops
+    rng = np.random.default_rng(n)
+    dt = torch.as_tensor(rng.uniform(0.05, 0.5, n), dtype=torch.float64, device="cuda")
+    y = torch.as_tensor(rng.standard_normal(n), dtype=torch.float64, device="cuda")
+    r = torch.full((n,), 0.1, dtype=torch.float64, device="cuda")
+    k = K.Matern52(variance=1.0, lengthscale=2.0)
+    a, (am, aP) = ops.kalman_filter(dt, k, y, r, parallel=True)
+    b, (bm, bP) = ops.kalman_filter(dt, k, y, r, parallel=False)
+    assert abs(float(a) - float(b)) <= 1e-9 * abs(float(b))
+    assert float((am - bm).abs().max()) <= 1e-9 * float(bm.abs().max())
+    assert float((aP - bP).abs().max()) <= 1e-9 * float(bP.abs().max())
