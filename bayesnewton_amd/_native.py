@@ -53,7 +53,10 @@ SIGNATURES = {
     "bn_last_error": (ctypes.c_char_p, []),
     "bn_version": (i32, []),
     "bn_plan_create": (i32, [vp, i32, i32, ctypes.POINTER(vp)]),
+    "bn_plan_single_bytes": (i64, [i64, i32]),
+    "bn_plan_create_single": (i32, [i64, i32, vp, i64, vp, ctypes.POINTER(vp)]),
     "bn_plan_destroy": (i32, [vp]),
+    "bn_fill_f64": (i32, [vp, vp, i32, vp]),
     "bn_plan_num_slots": (i64, [vp]),
     "bn_plan_num_chunks": (i32, [vp]),
     "bn_plan_num_tiles": (i32, [vp]),

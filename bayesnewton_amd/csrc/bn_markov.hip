@@ -697,6 +697,55 @@ __global__ void k_scatter_planes(PlanView pl, const float* __restrict__ src, dou
   for (int32_t f = 0; f < width; ++f) dst[f * n_steps + csr] = (double)src[f * pl.n_slots + slot];
 }
 
+// The tables of one series' plan, which are closed forms of the chunk's number: a plan that lives
+// for one call is made in the stream's order, with no allocation, copy or free of its own.  Those
+// took 80 us, and the free waited for the kernels that the call had launched: 775 -> 371 us for a
+// filter and a smoother of 100,000 steps, of which the kernels run 350.
+__global__ void k_plan_single(PlanView pl, int64_t n) {
+  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= pl.n_chunks) return;
+  const int32_t c = pl.chunk_len, nc = pl.n_chunks, nt = pl.n_tiles;
+  const int64_t start = (int64_t)j * c;
+  const auto len_of = [&](int32_t k) { return (int32_t)min((int64_t)c, n - (int64_t)k * c); };
+  const_cast<int32_t*>(pl.chunk_series)[j] = 0;
+  const_cast<int32_t*>(pl.chunk_len_)[j] = len_of(j);
+  const_cast<uint8_t*>(pl.chunk_flags)[j] = (uint8_t)((j == 0 ? 1 : 0) | (j == nc - 1 ? 2 : 0));
+  const_cast<int32_t*>(pl.chunk_tile)[j] = j / kTile;
+  const_cast<int64_t*>(pl.chunk_start)[j] = start;
+  if (j < (nc + 63) / 64) const_cast<int32_t*>(pl.wave_maxlen)[j] = len_of(j * 64);
+  if (j < nt) {
+    const int32_t cnt = min(kTile, nc - j * kTile);
+    const_cast<int32_t*>(pl.tile_first)[j] = j * kTile;
+    const_cast<int32_t*>(pl.tile_count)[j] = cnt;
+    const_cast<int32_t*>(pl.tile_series)[j] = 0;
+    const_cast<uint8_t*>(pl.tile_flags)[j] = (uint8_t)((j == 0 ? 1 : 0) | (j == nt - 1 ? 2 : 0));
+    if (j < pl.n_groups) {  // every tile in a group of its own; only the last can be a short one
+      int w = 1;
+      while (w < kGroupMax && cnt <= kTile / (2 * w)) w *= 2;
+      int32_t* g = const_cast<int32_t*>(pl.group_tiles) + (int64_t)j * kGroupMax;
+      for (int h = 0; h < kGroupMax; ++h) g[h] = h == 0 ? j : -1;
+      const_cast<uint8_t*>(pl.group_w)[j] = (uint8_t)w;
+    }
+  }
+  if (j == 0) {
+    const_cast<int32_t*>(pl.series_first_tile)[0] = 0;
+    const_cast<int32_t*>(pl.series_ntiles)[0] = nt;
+    const_cast<int32_t*>(pl.series_first_chunk)[0] = 0;
+    const_cast<int32_t*>(pl.series_nchunks)[0] = nc;
+  }
+}
+
+// A few words given by value: hyperparameters reach the device in the stream's order (a copy from
+// pageable host memory waits for everything launched before it).
+constexpr int32_t kFillMax = 16;
+struct FillValues {
+  double v[kFillMax];
+};
+__global__ void k_fill_f64(FillValues f, double* __restrict__ dst, int32_t n) {
+  const int32_t i = threadIdx.x;
+  if (i < n) dst[i] = f.v[i];
+}
+
 template <int K1, int K2>
 __global__ void k_discretise(HyperView hv, int64_t n, const float* __restrict__ dt, float* __restrict__ A,
                              float* __restrict__ Q) {
@@ -1151,6 +1200,36 @@ int run_pairs_filter(HyperView hv, int32_t n_series, const int64_t* off, const d
     }                                                                           \
   }()
 
+// Scan groups of one series' plan: one a tile, none for a single chunk (build_scan_groups).
+int32_t single_groups(const PlanHost& h) { return h.n_chunks > 1 ? h.n_tiles : 0; }
+
+void bind_tables(const PlanHost& h, const PlanTables& tb, int32_t n_groups, char* d, PlanView& v) {
+  v.n_series = h.n_series;
+  v.n_chunks = h.n_chunks;
+  v.n_chunks_pad = h.n_chunks_pad;
+  v.n_tiles = h.n_tiles;
+  v.chunk_len = h.chunk_len;
+  v.gshift = h.gshift;
+  v.n_slots = h.n_slots;
+  v.chunk_series = (const int32_t*)(d + tb.off[PlanTables::kChunkSeries]);
+  v.chunk_len_ = (const int32_t*)(d + tb.off[PlanTables::kChunkLen]);
+  v.chunk_flags = (const uint8_t*)(d + tb.off[PlanTables::kChunkFlags]);
+  v.chunk_tile = (const int32_t*)(d + tb.off[PlanTables::kChunkTile]);
+  v.chunk_start = (const int64_t*)(d + tb.off[PlanTables::kChunkStart]);
+  v.tile_first = (const int32_t*)(d + tb.off[PlanTables::kTileFirst]);
+  v.tile_count = (const int32_t*)(d + tb.off[PlanTables::kTileCount]);
+  v.tile_series = (const int32_t*)(d + tb.off[PlanTables::kTileSeries]);
+  v.tile_flags = (const uint8_t*)(d + tb.off[PlanTables::kTileFlags]);
+  v.series_first_tile = (const int32_t*)(d + tb.off[PlanTables::kSeriesFirstTile]);
+  v.series_ntiles = (const int32_t*)(d + tb.off[PlanTables::kSeriesNtiles]);
+  v.series_first_chunk = (const int32_t*)(d + tb.off[PlanTables::kSeriesFirstChunk]);
+  v.series_nchunks = (const int32_t*)(d + tb.off[PlanTables::kSeriesNchunks]);
+  v.n_groups = n_groups;
+  v.group_tiles = (const int32_t*)(d + tb.off[PlanTables::kGroupTiles]);
+  v.group_w = (const uint8_t*)(d + tb.off[PlanTables::kGroupW]);
+  v.wave_maxlen = (const int32_t*)(d + tb.off[PlanTables::kWaveMaxlen]);
+}
+
 int check_plan(const bn_plan* plan) {
   if (plan == nullptr) return fail(BN_EINVAL, "plan is NULL");
   return BN_OK;
@@ -1293,64 +1372,71 @@ int bn_plan_create(const int64_t* offsets_host, int32_t n_series, int32_t chunk_
     return fail(BN_EINVAL, err);
   }
   const PlanHost& h = p->host;
-  // one device allocation for every table, 256-byte aligned pieces
-  struct Piece { const void* src; size_t bytes; size_t off; };
-  Piece pcs[16] = {
-      {h.chunk_series.data(), h.chunk_series.size() * 4, 0}, {h.chunk_len_.data(), h.chunk_len_.size() * 4, 0},
-      {h.chunk_flags.data(), h.chunk_flags.size(), 0},       {h.chunk_tile.data(), h.chunk_tile.size() * 4, 0},
-      {h.chunk_start.data(), h.chunk_start.size() * 8, 0},   {h.tile_first.data(), h.tile_first.size() * 4, 0},
-      {h.tile_count.data(), h.tile_count.size() * 4, 0},     {h.tile_series.data(), h.tile_series.size() * 4, 0},
-      {h.tile_flags.data(), h.tile_flags.size(), 0},         {h.series_first_tile.data(), h.series_first_tile.size() * 4, 0},
-      {h.series_ntiles.data(), h.series_ntiles.size() * 4, 0}, {h.series_first_chunk.data(), h.series_first_chunk.size() * 4, 0},
-      {h.series_nchunks.data(), h.series_nchunks.size() * 4, 0}, {h.group_tiles.data(), h.group_tiles.size() * 4, 0},
-      {h.group_w.data(), h.group_w.size(), 0},               {h.wave_maxlen.data(), h.wave_maxlen.size() * 4, 0}};
-  size_t total = 0;
-  for (auto& pc : pcs) {
-    pc.off = total;
-    total += (pc.bytes + 255) & ~size_t(255);
-  }
-  if (total == 0) total = 256;
-  hipError_t e = hipMalloc(&p->dev, total);
+  const PlanTables tb(h, h.group_w.size());
+  const void* src[PlanTables::kCount] = {
+      h.chunk_series.data(), h.chunk_len_.data(), h.chunk_flags.data(), h.chunk_tile.data(), h.chunk_start.data(),
+      h.tile_first.data(), h.tile_count.data(), h.tile_series.data(), h.tile_flags.data(), h.series_first_tile.data(),
+      h.series_ntiles.data(), h.series_first_chunk.data(), h.series_nchunks.data(), h.group_tiles.data(),
+      h.group_w.data(), h.wave_maxlen.data()};
+  hipError_t e = hipMalloc(&p->dev, tb.total);
   if (e != hipSuccess) {
     delete p;
     return fail(BN_ENOMEM, std::string("hipMalloc(plan): ") + hipGetErrorString(e));
   }
-  std::vector<char> staging(total, 0);
-  for (auto& pc : pcs)
-    if (pc.bytes) std::memcpy(staging.data() + pc.off, pc.src, pc.bytes);
-  e = hipMemcpy(p->dev, staging.data(), total, hipMemcpyHostToDevice);
+  std::vector<char> staging(tb.total, 0);
+  for (int i = 0; i < PlanTables::kCount; ++i)
+    if (tb.bytes[i]) std::memcpy(staging.data() + tb.off[i], src[i], tb.bytes[i]);
+  e = hipMemcpy(p->dev, staging.data(), tb.total, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     (void)hipFree(p->dev);
     delete p;
     return fail(BN_EHIP, std::string("hipMemcpy(plan): ") + hipGetErrorString(e));
   }
-  char* d = (char*)p->dev;
-  PlanView& v = p->view;
-  v.n_series = h.n_series;
-  v.n_chunks = h.n_chunks;
-  v.n_chunks_pad = h.n_chunks_pad;
-  v.n_tiles = h.n_tiles;
-  v.chunk_len = h.chunk_len;
-  v.gshift = h.gshift;
-  v.n_slots = h.n_slots;
-  v.chunk_series = (const int32_t*)(d + pcs[0].off);
-  v.chunk_len_ = (const int32_t*)(d + pcs[1].off);
-  v.chunk_flags = (const uint8_t*)(d + pcs[2].off);
-  v.chunk_tile = (const int32_t*)(d + pcs[3].off);
-  v.chunk_start = (const int64_t*)(d + pcs[4].off);
-  v.tile_first = (const int32_t*)(d + pcs[5].off);
-  v.tile_count = (const int32_t*)(d + pcs[6].off);
-  v.tile_series = (const int32_t*)(d + pcs[7].off);
-  v.tile_flags = (const uint8_t*)(d + pcs[8].off);
-  v.series_first_tile = (const int32_t*)(d + pcs[9].off);
-  v.series_ntiles = (const int32_t*)(d + pcs[10].off);
-  v.series_first_chunk = (const int32_t*)(d + pcs[11].off);
-  v.series_nchunks = (const int32_t*)(d + pcs[12].off);
-  v.n_groups = (int32_t)h.group_w.size();
-  v.group_tiles = (const int32_t*)(d + pcs[13].off);
-  v.group_w = (const uint8_t*)(d + pcs[14].off);
-  v.wave_maxlen = (const int32_t*)(d + pcs[15].off);
+  bind_tables(h, tb, (int32_t)h.group_w.size(), (char*)p->dev, p->view);
   *out = p;
+  return BN_OK;
+}
+
+int64_t bn_plan_single_bytes(int64_t n_steps, int32_t chunk_len) {
+  PlanHost h;
+  std::string err;
+  if (!single_plan(n_steps, chunk_len, h, err)) {
+    (void)fail(BN_EINVAL, err);
+    return -1;
+  }
+  return (int64_t)PlanTables(h, single_groups(h)).total;
+}
+
+int bn_plan_create_single(int64_t n_steps, int32_t chunk_len, void* tables, int64_t bytes, void* stream,
+                          bn_plan** out) {
+  if (tables == nullptr || out == nullptr) return fail(BN_EINVAL, "NULL argument to bn_plan_create_single");
+  *out = nullptr;
+  PlanHost h;
+  std::string err;
+  if (!single_plan(n_steps, chunk_len, h, err)) return fail(BN_EINVAL, err);
+  const int32_t groups = single_groups(h);
+  const PlanTables tb(h, groups);
+  if (bytes < (int64_t)tb.total) return fail(BN_EINVAL, "table memory is too small for the plan");
+  if ((uintptr_t)tables & 15) return fail(BN_EINVAL, "table memory must be 16-byte aligned");
+  PlanView v = {};
+  bind_tables(h, tb, groups, (char*)tables, v);
+  hipLaunchKernelGGL(k_plan_single, dim3((unsigned)((h.n_chunks + 255) / 256)), dim3(256), 0, (hipStream_t)stream, v,
+                     n_steps);
+  BN_HIP_CHECK(hipGetLastError());
+  bn_plan* p = new bn_plan();
+  p->host = h;
+  p->view = v;
+  *out = p;
+  return BN_OK;
+}
+
+int bn_fill_f64(double* dst, const double* values_host, int32_t n, void* stream) {
+  if (dst == nullptr || values_host == nullptr) return fail(BN_EINVAL, "NULL argument to bn_fill_f64");
+  if (n < 1 || n > kFillMax) return fail(BN_EINVAL, "n must be in [1, 16]");
+  FillValues f = {};
+  for (int32_t i = 0; i < n; ++i) f.v[i] = values_host[i];
+  hipLaunchKernelGGL(k_fill_f64, dim3(1), dim3(64), 0, (hipStream_t)stream, f, dst, n);
+  BN_HIP_CHECK(hipGetLastError());
   return BN_OK;
 }
 

@@ -56,6 +56,16 @@ inline void build_scan_groups(PlanHost& p) {
     }
   }
 }
+// Lanes are grouped 64 to a wavefront; with fewer than 64 chunks the group
+// shrinks to the next power of two so the tiled layout does not pad 64x.
+inline void set_lane_groups(PlanHost& p) {
+  p.gshift = 6;
+  while (p.gshift > 0 && (1 << (p.gshift - 1)) >= p.n_chunks) --p.gshift;
+  const int32_t G = 1 << p.gshift;
+  p.n_chunks_pad = ((p.n_chunks + G - 1) / G) * G;
+  p.n_slots = (int64_t)(p.n_chunks_pad / G) * p.chunk_len * G;
+}
+
 inline bool build_plan(const int64_t* offsets, int32_t n_series, int32_t chunk_len, PlanHost& p, std::string& err) {
   if (n_series < 1) { err = "n_series must be >= 1"; return false; }
   if (chunk_len < 1 || chunk_len > (1 << 24)) { err = "chunk_len must be in [1, 2^24]"; return false; }
@@ -110,15 +120,49 @@ inline bool build_plan(const int64_t* offsets, int32_t n_series, int32_t chunk_l
   // Empty series inside a batch are fine (no chunk, log-likelihood 0); a batch
   // with no step at all would launch empty grids, so it is refused here.
   if (p.n_chunks == 0) { err = "offsets describe no steps (every series is empty)"; return false; }
-  // Lanes are grouped 64 to a wavefront; with fewer than 64 chunks the group
-  // shrinks to the next power of two so the tiled layout does not pad 64x.
-  p.gshift = 6;
-  while (p.gshift > 0 && (1 << (p.gshift - 1)) >= p.n_chunks) --p.gshift;
-  const int32_t G = 1 << p.gshift;
-  p.n_chunks_pad = ((p.n_chunks + G - 1) / G) * G;
-  p.n_slots = (int64_t)(p.n_chunks_pad / G) * chunk_len * G;
+  set_lane_groups(p);
   p.n_steps = offsets[n_series];
   return true;
 }
+
+// The counts of one series' plan (its tables are closed forms of the chunk's number and are
+// written by a kernel); refuses what build_plan refuses.
+inline bool single_plan(int64_t n, int32_t chunk_len, PlanHost& p, std::string& err) {
+  if (chunk_len < 1 || chunk_len > (1 << 24)) { err = "chunk_len must be in [1, 2^24]"; return false; }
+  if (n < 0) { err = "offsets must be non-decreasing"; return false; }
+  if (n == 0) { err = "offsets describe no steps (every series is empty)"; return false; }
+  const int64_t nc = (n - 1) / chunk_len + 1;
+  if (nc > (int64_t)kTile * kTile) {
+    err = "series 0 needs " + std::to_string(nc) + " chunks (> kTile^2): raise chunk_len";
+    return false;
+  }
+  p = PlanHost();
+  p.n_series = 1;
+  p.chunk_len = chunk_len;
+  p.n_chunks = (int32_t)nc;
+  p.n_tiles = (int32_t)((nc + kTile - 1) / kTile);
+  p.needs_scan = nc > 1;
+  p.n_steps = n;
+  set_lane_groups(p);
+  return true;
+}
+
+// Byte offsets of a plan's device tables in one allocation, 256-byte aligned pieces.
+struct PlanTables {
+  enum { kChunkSeries, kChunkLen, kChunkFlags, kChunkTile, kChunkStart, kTileFirst, kTileCount, kTileSeries,
+         kTileFlags, kSeriesFirstTile, kSeriesNtiles, kSeriesFirstChunk, kSeriesNchunks, kGroupTiles, kGroupW,
+         kWaveMaxlen, kCount };
+  size_t bytes[kCount], off[kCount], total = 0;
+  PlanTables(const PlanHost& p, size_t n_groups) {
+    const size_t c = (size_t)p.n_chunks, t = (size_t)p.n_tiles, s = (size_t)p.n_series;
+    const size_t b[kCount] = {c * 4, c * 4, c, c * 4, c * 8, t * 4, t * 4, t * 4, t, s * 4, s * 4, s * 4, s * 4,
+                              n_groups * kGroupMax * 4, n_groups, (c + 63) / 64 * 4};
+    for (int i = 0; i < kCount; ++i) {
+      bytes[i] = b[i];
+      off[i] = total;
+      total += (b[i] + 255) & ~size_t(255);
+    }
+  }
+};
 
 }  // namespace bn

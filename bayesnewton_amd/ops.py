@@ -42,15 +42,28 @@ def discretise(kernel, dt):
     A = torch.empty((n, d, d), dtype=torch.float32, device=dev)
     Q = torch.empty((n, d, d), dtype=torch.float32, device=dev)
     desc = kernel.desc()
-    ls, var = kernel.hypers(dev)
+    ls, var = _hypers(kernel, dev)
     import ctypes
     nat.check(nat.lib().bn_discretise(ctypes.byref(desc), nat.ptr(ls), nat.ptr(var), n, nat.ptr(dt), nat.ptr(A),
                                       nat.ptr(Q), nat.stream_ptr()))
     return A, Q
 
 
+def _hypers(kernel, dev):
+    """kernel.hypers(dev) for the launches of one call, in the order of the current stream: a
+    copy from the host would wait for everything launched before it."""
+    comps = kernel.components
+    values = [c.lengthscale for c in comps] + [c.variance for c in comps]
+    if len(values) > 16 or torch.cuda.is_current_stream_capturing():
+        return kernel.hypers(dev)
+    words = np.array(values, dtype=np.float64)
+    both = torch.empty(len(values), dtype=torch.float64, device=dev)
+    nat.check(nat.lib().bn_fill_f64(nat.ptr(both), words.ctypes.data, len(values), nat.stream_ptr()))
+    return both[:len(comps)], both[len(comps):]
+
+
 def _single_plan(n, parallel, dev):
-    return SeriesPlan(np.array([0, n], dtype=np.int64), chunk_len=model_chunk_len([n], parallel), device=dev)
+    return SeriesPlan.for_call(n, model_chunk_len([n], parallel), dev)
 
 
 def kalman_filter(dt, kernel, y, noise_cov, mask=None, parallel=False, return_predict=False, plan=None,
@@ -75,7 +88,7 @@ def kalman_filter(dt, kernel, y, noise_cov, mask=None, parallel=False, return_pr
         plan = _single_plan(N, parallel, dev)
     d = kernel.state_dim
     desc = kernel.desc()
-    ls, var = kernel.hypers(dev)
+    ls, var = _hypers(kernel, dev)
     dt_t, y_t, r_t = plan.gather(dt), plan.gather(y), plan.gather(r, pad=1.0)
     mk = plan.gather_mask(_as_tensor(mask, torch.bool, dev)) if mask is not None else None
     means = torch.empty((d, plan.n_slots), dtype=torch.float64, device=dev)
@@ -107,7 +120,7 @@ def rauch_tung_striebel_smoother(dt, kernel, filter_mean, filter_cov, return_ful
     if plan is None:
         plan = _single_plan(N, parallel, dev)
     desc = kernel.desc()
-    ls, var = kernel.hypers(dev)
+    ls, var = _hypers(kernel, dev)
     dt_t, fm_t, fP_t = plan.gather(dt), plan.gather(fm), plan.gather(fP)
     w_m, w_P = (d, d * d) if return_full else (1, 1)
     om = torch.empty((w_m, plan.n_slots), dtype=torch.float64, device=dev)
@@ -386,7 +399,7 @@ def kalman_filter_pairs(dt, kernel, y, noise_cov, mask=None, parallel=False):
     Po = torch.empty((n, 2 * d, 2 * d), **f64)
     ll = torch.empty(1, **f64)
     desc = kernel.desc()
-    ls, var = kernel.hypers(dev)
+    ls, var = _hypers(kernel, dev)
     nat.check(nat.lib().bn_pairs_filter(ctypes.byref(desc), nat.ptr(ls), nat.ptr(var), 0, 1, nat.ptr(off),
                                         nat.ptr(dtv), nat.ptr(yv), nat.ptr(R), nat.ptr(mo), nat.ptr(Po), nat.ptr(ll),
                                         nat.stream_ptr()))

@@ -70,13 +70,37 @@ class SeriesPlan:
         self.n_steps = int(off[-1])
         if chunk_len is None:
             chunk_len = default_chunk_len(self.lengths, parallel)
-        self.chunk_len = int(chunk_len)
         self.device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
-        L = nat.lib()
         h = ctypes.c_void_p()
         with torch.cuda.device(self.device):
-            nat.check(L.bn_plan_create(off.ctypes.data_as(ctypes.c_void_p), self.n_series, self.chunk_len,
-                                       ctypes.byref(h)))
+            nat.check(nat.lib().bn_plan_create(off.ctypes.data_as(ctypes.c_void_p), self.n_series, int(chunk_len),
+                                               ctypes.byref(h)))
+        self._adopt(h, chunk_len)
+
+    @classmethod
+    def for_call(cls, n, chunk_len, device):
+        """Plan of one series that is used and dropped on the current stream of the current
+        device: its tables are made and given back in the stream's order, so that neither
+        waits for the device.  Not under graph capture, where a plan has to exist before."""
+        off = np.array([0, n], dtype=np.int64)
+        if torch.cuda.is_current_stream_capturing():
+            return cls(off, chunk_len=chunk_len, device=device)
+        L = nat.lib()
+        nbytes = int(L.bn_plan_single_bytes(n, chunk_len))
+        nat.check(0 if nbytes > 0 else -1)
+        self = cls.__new__(cls)
+        self.offsets, self.lengths, self.n_series, self.n_steps = off, np.diff(off), 1, int(n)
+        self.device = device
+        self._tables = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        h = ctypes.c_void_p()
+        nat.check(L.bn_plan_create_single(n, chunk_len, nat.ptr(self._tables), nbytes, nat.stream_ptr(),
+                                          ctypes.byref(h)))
+        self._adopt(h, chunk_len)
+        return self
+
+    def _adopt(self, h, chunk_len):
+        L = nat.lib()
+        self.chunk_len = int(chunk_len)
         self._h = h
         self.n_slots = int(L.bn_plan_num_slots(h))
         self.n_chunks = int(L.bn_plan_num_chunks(h))

@@ -108,7 +108,16 @@ int bn_version(void);
  * most 128 * 128 chunks (level-1 tiles of 128 chunks, at most 128 tiles).  Replaces input_admin's bookkeeping (utils.py:234-265) for
  * many series at once; the reference handles one series per model. */
 int bn_plan_create(const int64_t *offsets_host, int32_t n_series, int32_t chunk_len, bn_plan **out);
+/* The plan of one series of n_steps, its tables written by a kernel on `stream` into device
+ * memory of the caller (16-byte aligned, at least bn_plan_single_bytes() of it, which is -1 for
+ * what bn_plan_create refuses).  The memory must outlive the plan and every launch that uses
+ * it; another stream waits for `stream` before it uses the plan. */
+int64_t bn_plan_single_bytes(int64_t n_steps, int32_t chunk_len);
+int bn_plan_create_single(int64_t n_steps, int32_t chunk_len, void *tables, int64_t bytes, void *stream,
+                          bn_plan **out);
 int bn_plan_destroy(bn_plan *plan);
+/* dst[i] = values_host[i] for 1 <= n <= 16 words, in the stream's order. */
+int bn_fill_f64(double *dst, const double *values_host, int32_t n, void *stream);
 int64_t bn_plan_num_slots(const bn_plan *plan);
 int32_t bn_plan_num_chunks(const bn_plan *plan);
 int32_t bn_plan_num_tiles(const bn_plan *plan);
