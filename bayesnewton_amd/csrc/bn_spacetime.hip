@@ -2360,35 +2360,102 @@ __global__ __launch_bounds__(kT) void k_mf_sdiag(StDims dm, StHyp hy, MfFilterIO
   }
 }
 
-// Scalar-observation filter of every block over the per-step (reff, yeff), lane per
-// (run, block).
+// The recursions over time of the mean-field blocks: one wavefront walks 64 (run, block) pairs
+// and is bound by its own chain of dependent FP64 operations, so everything that does not depend
+// on the previous step is made by other wavefronts of the workgroup, a tile of steps ahead, and
+// handed over in LDS.  Transitions depend on the run and the step alone: the workgroup makes
+// them once for each of the runs that its lanes belong to.
+constexpr int kMfTile = 8;
+
+// Lanes of a walker: 64, but 32 where the smoother's fields and the transitions of so many runs
+// would exceed the LDS.
+inline int mf_lanes(const StDims& dm) { return dm.M <= 2 ? 32 : 64; }
+inline int mf_runs(const StDims& dm) { return (mf_lanes(dm) + dm.M - 2) / dm.M + 1; }  // most of one walker
+inline size_t mf_table_doubles(const StDims& dm) { return (size_t)2 * mf_runs(dm) * kMfTile * 2 * dm.KT * dm.KT; }
+
+// Transitions of the steps first + dir * (0 .. kMfTile - 1) of the runs k0 .. k0 + nr - 1; steps
+// outside a run repeat its first or last.
 template <int KT>
-__global__ __launch_bounds__(64) void k_mf_blocks(StDims dm, StHyp hy, MfFilterIO io) {
-  const int64_t g = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (g >= (int64_t)dm.K * dm.M) return;
-  const int k = (int)(g / dm.M), i = (int)(g % dm.M), M = dm.M;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  double m[KT], P[KT][KT], mp[KT], Pp[KT][KT];
-  mf_pinf<KT>(ls, var, P);
-  for (int a = 0; a < KT; ++a) m[a] = 0.0;
-  for (int t = 0; t < dm.T; ++t) {
-    const int64_t kt = (int64_t)k * dm.T + t;
+__device__ void mf_transitions(const StDims& dm, const StHyp& hy, const double* dt, int k0, int nr, int first, int dir,
+                               double* aq, int tid, int n) {
+  for (int e = tid; e < nr * kMfTile; e += n) {
+    const int k = k0 + e / kMfTile;
+    const int t = min(max(first + dir * (e % kMfTile), 0), dm.T - 1);
     double A[KT * KT], Q[KT * KT];
-    temporal_AQ<KT>(ls, var, io.dt[kt], A, Q);
-    mf_predict<KT>(A, Q, m, P, mp, Pp);
-    const double S = Pp[0][0] + io.reff[kt * M + i];
-    const double v = io.yeff[kt * M + i] - mp[0];
-    double* fm = io.fmean + (kt * M + i) * KT;
-    double* fc = io.fcov + (kt * M + i) * KT * KT;
-    for (int a = 0; a < KT; ++a) {
-      const double Ka = Pp[a][0] / S;
-      m[a] = fma(Ka, v, mp[a]);
-      fm[a] = m[a];
-      for (int b = 0; b < KT; ++b) {
-        P[a][b] = fma(-Ka, Pp[b][0], Pp[a][b]);
-        fc[a * KT + b] = P[a][b];
-      }
+    temporal_AQ<KT>(hy.ls_t[k * hy.stride], hy.var_t[k * hy.stride], dt[(int64_t)k * dm.T + t], A, Q);
+    double* o = aq + e * 2 * KT * KT;
+    for (int j = 0; j < KT * KT; ++j) { o[j] = A[j]; o[KT * KT + j] = Q[j]; }
+  }
+}
+
+// Scalar-observation filter of every block over the per-step (reff, yeff): wavefront 0 walks, a
+// lane per (run, block), two more make the next tile's transitions.  4 runs of 500 steps at
+// M = 64: 377 -> 136 us (with the transitions in the walk, and every load waited for
+// where it is used).
+constexpr int kMfBlocksT = 192;
+template <int KT>
+__global__ __launch_bounds__(kMfBlocksT) void k_mf_blocks(StDims dm, StHyp hy, MfFilterIO io, int lanes) {
+  extern __shared__ double smem[];
+  const int M = dm.M, T = dm.T, lane = threadIdx.x & 63;
+  const bool walker = threadIdx.x < 64;
+  const int64_t total = (int64_t)dm.K * M, g0 = (int64_t)blockIdx.x * lanes;
+  const int64_t last = min(g0 + lanes, total) - 1;
+  const bool mine = walker && lane < lanes && g0 + lane < total;
+  const int64_t g = min(g0 + min(lane, lanes - 1), total - 1);
+  const int k0 = (int)(g0 / M), nr = (int)(last / M) - k0 + 1;
+  const int k = (int)(g / M), i = (int)(g % M);
+  const int table = nr * kMfTile * 2 * KT * KT;
+  const int64_t row0 = (int64_t)k * T * M + i;  // of step 0; steps are M apart
+  double m[KT], P[KT][KT], r[kMfTile], y[kMfTile];
+  mf_pinf<KT>(hy.ls_t[k * hy.stride], hy.var_t[k * hy.stride], P);
+  for (int a = 0; a < KT; ++a) m[a] = 0.0;
+  if (walker) {
+#pragma unroll
+    for (int s = 0; s < kMfTile; ++s) {
+      const int64_t e = row0 + (int64_t)min(s, T - 1) * M;
+      r[s] = io.reff[e];
+      y[s] = io.yeff[e];
     }
+  } else {
+    mf_transitions<KT>(dm, hy, io.dt, k0, nr, 0, 1, smem, threadIdx.x - 64, kMfBlocksT - 64);
+  }
+  __syncthreads();
+  for (int t0 = 0, n = 0; t0 < T; t0 += kMfTile, ++n) {
+    if (walker) {
+      const double* aq = smem + (n & 1) * table + (k - k0) * kMfTile * 2 * KT * KT;
+      double rn[kMfTile], yn[kMfTile];
+#pragma unroll
+      for (int s = 0; s < kMfTile; ++s) {
+        const int64_t e = row0 + (int64_t)min(t0 + kMfTile + s, T - 1) * M;
+        rn[s] = io.reff[e];
+        yn[s] = io.yeff[e];
+      }
+#pragma unroll
+      for (int s = 0; s < kMfTile; ++s) {
+        double mp[KT], Pp[KT][KT], A[KT * KT], Q[KT * KT];
+        for (int j = 0; j < KT * KT; ++j) { A[j] = aq[s * 2 * KT * KT + j]; Q[j] = aq[(s * 2 + 1) * KT * KT + j]; }
+        mf_predict<KT>(A, Q, m, P, mp, Pp);
+        const double S = Pp[0][0] + r[s], v = y[s] - mp[0];
+        for (int a = 0; a < KT; ++a) {
+          const double Ka = Pp[a][0] / S;
+          m[a] = fma(Ka, v, mp[a]);
+          for (int b = 0; b < KT; ++b) P[a][b] = fma(-Ka, Pp[b][0], Pp[a][b]);
+        }
+        if (mine && t0 + s < T) {
+          const int64_t e = row0 + (int64_t)(t0 + s) * M;
+          for (int a = 0; a < KT; ++a) {
+            io.fmean[e * KT + a] = m[a];
+            for (int b = 0; b < KT; ++b) io.fcov[(e * KT + a) * KT + b] = P[a][b];
+          }
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < kMfTile; ++s) { r[s] = rn[s]; y[s] = yn[s]; }
+    } else if (t0 + kMfTile < T) {
+      mf_transitions<KT>(dm, hy, io.dt, k0, nr, t0 + kMfTile, 1, smem + ((n + 1) & 1) * table, threadIdx.x - 64,
+                         kMfBlocksT - 64);
+    }
+    __syncthreads();
   }
 }
 
@@ -2405,86 +2472,146 @@ struct MfSmootherIO {
 };
 
 // RTS smoother of every block (ops.py:611-641; the associative form 644-678 gives the
-// same result), lane per (run, block), from the last step back.
+// same result), lane per (run, block), from the last step back.  Wavefront 0 walks a tile of
+// steps while eight others, a step each, make the next tile's gains and predictions (about 130
+// of the 200 operations of a step, its four divisions among them) and after that the transitions
+// of the tile after next.  4 runs of 500 steps at M = 64: 310 -> 119 us.
+constexpr int kMfSmootherT = 64 * (kMfTile + 1);
 template <int KT>
-__global__ __launch_bounds__(64) void k_mf_smoother(StDims dm, StHyp hy, MfSmootherIO io) {
-  const int64_t g = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (g >= (int64_t)dm.K * dm.M) return;
-  const int k = (int)(g / dm.M), i = (int)(g % dm.M), M = dm.M;
-  const double ls = hy.ls_t[k * hy.stride], var = hy.var_t[k * hy.stride];
-  double sm[KT], sP[KT][KT];
+constexpr int kMfFields = 2 * KT + 3 * KT * KT;  // fm, pm, fP, pP, G
+
+template <int KT>
+__global__ __launch_bounds__(kMfSmootherT) void k_mf_smoother(StDims dm, StHyp hy, MfSmootherIO io, int lanes) {
+  extern __shared__ double smem[];
+  constexpr int K2 = KT * KT, F = kMfFields<KT>;
+  const int M = dm.M, T = dm.T, lane = threadIdx.x & 63, s_own = (int)(threadIdx.x >> 6) - 1;
+  const int64_t total = (int64_t)dm.K * M, g0 = (int64_t)blockIdx.x * lanes;
+  const int64_t last = min(g0 + lanes, total) - 1;
+  const bool mine = lane < lanes && g0 + lane < total;
+  const int64_t g = min(g0 + min(lane, lanes - 1), total - 1);
+  const int k0 = (int)(g0 / M), nr = (int)(last / M) - k0 + 1;
+  const int k = (int)(g / M), i = (int)(g % M);
+  const int table = nr * kMfTile * 2 * K2;
+  double* fields = smem;                      // [2][kMfTile][F][64]
+  double* aq = smem + 2 * kMfTile * F * 64;   // [2][nr][kMfTile][2 K2]
+  const int tiles = (T + kMfTile - 1) / kMfTile;
+  const int64_t row0 = (int64_t)k * T * M + i;
+  double sm[KT], sP[KT][KT];                  // walker
+  double nm[KT], nP[KT][KT];                  // the others: filtered moments of the next step that they make
   {
-    const int64_t kt = (int64_t)k * dm.T + dm.T - 1;
+    const int64_t e = row0 + (int64_t)max(T - 1 - max(s_own, 0), 0) * M;
     for (int a = 0; a < KT; ++a) {
-      sm[a] = io.fmean[(kt * M + i) * KT + a];
-      for (int b = 0; b < KT; ++b) sP[a][b] = io.fcov[((kt * M + i) * KT + a) * KT + b];
+      sm[a] = nm[a] = io.fmean[e * KT + a];
+      for (int b = 0; b < KT; ++b) sP[a][b] = nP[a][b] = io.fcov[(e * KT + a) * KT + b];
     }
   }
-  for (int t = dm.T - 1; t >= 0; --t) {
-    const int64_t kt = (int64_t)k * dm.T + t;
-    double fm[KT], fP[KT][KT], pm[KT], pP[KT][KT], A[KT * KT], Q[KT * KT];
-    for (int a = 0; a < KT; ++a) {
-      fm[a] = io.fmean[(kt * M + i) * KT + a];
-      for (int b = 0; b < KT; ++b) fP[a][b] = io.fcov[((kt * M + i) * KT + a) * KT + b];
-    }
-    temporal_AQ<KT>(ls, var, io.dt[kt], A, Q);
-    mf_predict<KT>(A, Q, fm, fP, pm, pP);
-    // G = (A fP)' pP^-1 = fP A' pP^-1
-    double AfP[KT][KT], iP[KT][KT], G[KT][KT];
-    for (int a = 0; a < KT; ++a)
-      for (int b = 0; b < KT; ++b) {
-        double s = 0.0;
-        for (int q = 0; q < KT; ++q) s = fma(A[a * KT + q], fP[q][b], s);
-        AfP[a][b] = s;
+  // round it: transitions of tile it, gains of tile it - 1, walk of tile it - 2
+  for (int it = 0; it < tiles + 2; ++it) {
+    if (s_own >= 0) {
+      if (it >= 1 && it <= tiles) {
+        const int t = T - 1 - ((it - 1) * kMfTile + s_own);
+        double fm[KT], fP[KT][KT], pm[KT], pP[KT][KT], A[K2], Q[K2];
+        const double* o = aq + ((it - 1) & 1) * table + ((k - k0) * kMfTile + s_own) * 2 * K2;
+        for (int j = 0; j < K2; ++j) { A[j] = o[j]; Q[j] = o[K2 + j]; }
+        const int64_t e = row0 + (int64_t)max(t - kMfTile, 0) * M;
+        for (int a = 0; a < KT; ++a) {
+          fm[a] = nm[a];
+          for (int b = 0; b < KT; ++b) fP[a][b] = nP[a][b];
+        }
+        for (int a = 0; a < KT; ++a) {
+          nm[a] = io.fmean[e * KT + a];
+          for (int b = 0; b < KT; ++b) nP[a][b] = io.fcov[(e * KT + a) * KT + b];
+        }
+        mf_predict<KT>(A, Q, fm, fP, pm, pP);
+        // G = (A fP)' pP^-1 = fP A' pP^-1
+        double AfP[KT][KT], iP[KT][KT], G[KT][KT];
+        for (int a = 0; a < KT; ++a)
+          for (int b = 0; b < KT; ++b) {
+            double w = 0.0;
+            for (int q = 0; q < KT; ++q) w = fma(A[a * KT + q], fP[q][b], w);
+            AfP[a][b] = w;
+          }
+        if (KT == 1) {
+          iP[0][0] = 1.0 / pP[0][0];
+        } else {
+          const double det = pP[0][0] * pP[KT - 1][KT - 1] - pP[0][KT - 1] * pP[KT - 1][0];
+          iP[0][0] = pP[KT - 1][KT - 1] / det;
+          iP[KT - 1][KT - 1] = pP[0][0] / det;
+          iP[0][KT - 1] = -pP[0][KT - 1] / det;
+          iP[KT - 1][0] = -pP[KT - 1][0] / det;
+        }
+        for (int a = 0; a < KT; ++a)
+          for (int b = 0; b < KT; ++b) {
+            double w = 0.0;
+            for (int q = 0; q < KT; ++q) w = fma(AfP[q][a], iP[q][b], w);
+            G[a][b] = w;
+          }
+        double* f = fields + (((it - 1) & 1) * kMfTile + s_own) * F * 64 + lane;
+        for (int a = 0; a < KT; ++a) {
+          f[a * 64] = fm[a];
+          f[(KT + a) * 64] = pm[a];
+          for (int b = 0; b < KT; ++b) {
+            f[(2 * KT + a * KT + b) * 64] = fP[a][b];
+            f[(2 * KT + K2 + a * KT + b) * 64] = pP[a][b];
+            f[(2 * KT + 2 * K2 + a * KT + b) * 64] = G[a][b];
+          }
+        }
+        if (io.gain && mine && t >= 0)
+          for (int j = 0; j < K2; ++j) io.gain[(row0 + (int64_t)t * M) * K2 + j] = G[j / KT][j % KT];
       }
-    if (KT == 1) {
-      iP[0][0] = 1.0 / pP[0][0];
-    } else {
-      const double det = pP[0][0] * pP[KT - 1][KT - 1] - pP[0][KT - 1] * pP[KT - 1][0];
-      iP[0][0] = pP[KT - 1][KT - 1] / det;
-      iP[KT - 1][KT - 1] = pP[0][0] / det;
-      iP[0][KT - 1] = -pP[0][KT - 1] / det;
-      iP[KT - 1][0] = -pP[KT - 1][0] / det;
-    }
-    for (int a = 0; a < KT; ++a)
-      for (int b = 0; b < KT; ++b) {
-        double s = 0.0;
-        for (int q = 0; q < KT; ++q) s = fma(AfP[q][a], iP[q][b], s);
-        G[a][b] = s;
+      if (it < tiles)
+        mf_transitions<KT>(dm, hy, io.dt, k0, nr, T - 1 - it * kMfTile, -1, aq + (it & 1) * table, threadIdx.x - 64,
+                           kMfSmootherT - 64);
+    } else if (it >= 2) {
+#pragma unroll
+      for (int s = 0; s < kMfTile; ++s) {
+        const int t = T - 1 - ((it - 2) * kMfTile + s);
+        const double* f = fields + ((it & 1) * kMfTile + s) * F * 64 + lane;
+        double fm[KT], fP[KT][KT], pm[KT], pP[KT][KT], G[KT][KT];
+        for (int a = 0; a < KT; ++a) {
+          fm[a] = f[a * 64];
+          pm[a] = f[(KT + a) * 64];
+          for (int b = 0; b < KT; ++b) {
+            fP[a][b] = f[(2 * KT + a * KT + b) * 64];
+            pP[a][b] = f[(2 * KT + K2 + a * KT + b) * 64];
+            G[a][b] = f[(2 * KT + 2 * K2 + a * KT + b) * 64];
+          }
+        }
+        double dm_[KT], dP[KT][KT], GdP[KT][KT];
+        for (int a = 0; a < KT; ++a) {
+          dm_[a] = sm[a] - pm[a];
+          for (int b = 0; b < KT; ++b) dP[a][b] = sP[a][b] - pP[a][b];
+        }
+        for (int a = 0; a < KT; ++a) {
+          double w = fm[a];
+          for (int q = 0; q < KT; ++q) w = fma(G[a][q], dm_[q], w);
+          sm[a] = w;
+          for (int b = 0; b < KT; ++b) {
+            double x = 0.0;
+            for (int q = 0; q < KT; ++q) x = fma(G[a][q], dP[q][b], x);
+            GdP[a][b] = x;
+          }
+        }
+        for (int a = 0; a < KT; ++a)
+          for (int b = 0; b < KT; ++b) {
+            double w = fP[a][b];
+            for (int q = 0; q < KT; ++q) w = fma(GdP[a][q], G[b][q], w);
+            sP[a][b] = w;
+          }
+        for (int a = 0; a < KT; ++a)
+          for (int b = a + 1; b < KT; ++b) sP[a][b] = sP[b][a] = 0.5 * (sP[a][b] + sP[b][a]);
+        if (mine && t >= 0) {
+          const int64_t kt = (int64_t)k * T + t, e = kt * M + i;
+          if (io.hmean) io.hmean[e] = sm[0];
+          if (io.hvar) io.hvar[kt * io.var_step + i * io.var_elem] = sP[0][0];
+          if (io.smean)
+            for (int a = 0; a < KT; ++a) io.smean[e * KT + a] = sm[a];
+          if (io.scov)
+            for (int j = 0; j < K2; ++j) io.scov[e * K2 + j] = sP[j / KT][j % KT];
+        }
       }
-    double dm_[KT], dP[KT][KT], GdP[KT][KT];
-    for (int a = 0; a < KT; ++a) {
-      dm_[a] = sm[a] - pm[a];
-      for (int b = 0; b < KT; ++b) dP[a][b] = sP[a][b] - pP[a][b];
     }
-    for (int a = 0; a < KT; ++a) {
-      double s = fm[a];
-      for (int q = 0; q < KT; ++q) s = fma(G[a][q], dm_[q], s);
-      sm[a] = s;
-      for (int b = 0; b < KT; ++b) {
-        double w = 0.0;
-        for (int q = 0; q < KT; ++q) w = fma(G[a][q], dP[q][b], w);
-        GdP[a][b] = w;
-      }
-    }
-    for (int a = 0; a < KT; ++a)
-      for (int b = 0; b < KT; ++b) {
-        double s = fP[a][b];
-        for (int q = 0; q < KT; ++q) s = fma(GdP[a][q], G[b][q], s);
-        sP[a][b] = s;
-      }
-    for (int a = 0; a < KT; ++a)
-      for (int b = a + 1; b < KT; ++b) sP[a][b] = sP[b][a] = 0.5 * (sP[a][b] + sP[b][a]);
-    if (io.hmean) io.hmean[kt * M + i] = sm[0];
-    if (io.hvar) io.hvar[kt * io.var_step + i * io.var_elem] = sP[0][0];
-    if (io.smean)
-      for (int a = 0; a < KT; ++a) io.smean[(kt * M + i) * KT + a] = sm[a];
-    if (io.scov)
-      for (int a = 0; a < KT; ++a)
-        for (int b = 0; b < KT; ++b) io.scov[((kt * M + i) * KT + a) * KT + b] = sP[a][b];
-    if (io.gain)
-      for (int a = 0; a < KT; ++a)
-        for (int b = 0; b < KT; ++b) io.gain[((kt * M + i) * KT + a) * KT + b] = G[a][b];
+    __syncthreads();
   }
 }
 
@@ -3125,6 +3252,8 @@ int set_smem_limits() {
   ST_SITES_ATTR1(KERNEL, MT, MD, LIK_BERNOULLI_PROBIT, N);  \
   ST_SITES_ATTR1(KERNEL, MT, MD, LIK_POISSON, N);           \
   ST_SITES_ATTR1(KERNEL, MT, MD, LIK_STUDENTS_T, N)
+  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_mf_smoother<1>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+  ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_mf_smoother<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
   ST_HIP_CHECK(hipFuncSetAttribute((const void*)k_mf_pseudo, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)kPseudoSmem));
   ST_SITES_ATTR(k_st_sites, M_VI, BN_ST_UPDATE, kSitesSmem);
@@ -3551,7 +3680,9 @@ int bn_mf_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, int32_t parall
     ST_HIP_CHECK(hipGetLastError());
   } else {
     const dim3 grid(dm.T, dm.K);
-    const int nb = (int)((dm.K * (int64_t)dm.M + 63) / 64);
+    const int lanes = mf_lanes(dm);
+    const int nb = (int)((dm.K * (int64_t)dm.M + lanes - 1) / lanes);
+    const size_t lds = mf_table_doubles(dm) * 8;
     {
       BN_TIMED(KID_MF_SDIAG, st);
       if (dm.KT == 1) hipLaunchKernelGGL((k_mf_sdiag<1, false>), grid, dim3(kT), 0, st, dm, hy, io);
@@ -3560,8 +3691,8 @@ int bn_mf_filter(const bn_st_dims* dims, const bn_st_hypers* hyp, int32_t parall
     }
     {
       BN_TIMED(KID_MF_BLOCKS, st);
-      if (dm.KT == 1) hipLaunchKernelGGL(k_mf_blocks<1>, dim3(nb), dim3(64), 0, st, dm, hy, io);
-      else hipLaunchKernelGGL(k_mf_blocks<2>, dim3(nb), dim3(64), 0, st, dm, hy, io);
+      if (dm.KT == 1) hipLaunchKernelGGL(k_mf_blocks<1>, dim3(nb), dim3(kMfBlocksT), lds, st, dm, hy, io, lanes);
+      else hipLaunchKernelGGL(k_mf_blocks<2>, dim3(nb), dim3(kMfBlocksT), lds, st, dm, hy, io, lanes);
       ST_HIP_CHECK(hipGetLastError());
     }
     {
@@ -3593,10 +3724,14 @@ int bn_mf_smoother(const bn_st_dims* dims, const bn_st_hypers* hyp, const double
   MfSmootherIO io{dt, filter_mean, filter_cov, post_mean, post_var, var_step_stride, var_elem_stride,
                   smooth_mean, smooth_cov, gains};
   hipStream_t st = (hipStream_t)stream;
-  const int nb = (int)((dm.K * (int64_t)dm.M + 63) / 64);
+  const int lanes = mf_lanes(dm);
+  const int nb = (int)((dm.K * (int64_t)dm.M + lanes - 1) / lanes);
+  const size_t lds =
+      (mf_table_doubles(dm) + (size_t)2 * kMfTile * (dm.KT == 1 ? kMfFields<1> : kMfFields<2>) * 64) * 8;
+  if (int rc = set_smem_limits()) return rc;
   BN_TIMED(KID_MF_SMOOTHER, st);
-  if (dm.KT == 1) hipLaunchKernelGGL(k_mf_smoother<1>, dim3(nb), dim3(64), 0, st, dm, make_hyp(hyp), io);
-  else hipLaunchKernelGGL(k_mf_smoother<2>, dim3(nb), dim3(64), 0, st, dm, make_hyp(hyp), io);
+  if (dm.KT == 1) hipLaunchKernelGGL(k_mf_smoother<1>, dim3(nb), dim3(kMfSmootherT), lds, st, dm, make_hyp(hyp), io, lanes);
+  else hipLaunchKernelGGL(k_mf_smoother<2>, dim3(nb), dim3(kMfSmootherT), lds, st, dm, make_hyp(hyp), io, lanes);
   ST_HIP_CHECK(hipGetLastError());
   return BN_OK;
 }
