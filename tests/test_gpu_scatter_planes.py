@@ -18,3 +18,18 @@ def test_planes_to_double_rows(lengths, chunk, w):
     assert out.dtype == torch.float64 and out.shape == (w, int(off[-1]))
     assert torch.equal(out, plan.scatter(t).double().t())
     assert torch.equal(out, x.double().t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths,chunk", [([1], 1), ([7], 100), ([70, 1, 33], 8), ([0, 5, 0], 4), ([300, 129, 2, 64], 3),
+                                           ([513], 4), ([4000], 4000)])
+@pytest.mark.parametrize("w", [2, 5, 25, 36, 100, 101])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_rows_of_words_to_planes_and_back(lengths, chunk, w, dtype):
+    off = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int64)
+    plan = SeriesPlan(off, chunk_len=chunk)
+    x = torch.randn(int(off[-1]), w, device="cuda", dtype=dtype)
+    t = plan.gather(x, pad=7.0)
+    assert torch.equal(t, torch.cat([plan.gather(x[:, f].contiguous(), pad=7.0) for f in range(w)]))
+    back = plan.scatter(t)
+    assert back.shape == x.shape and torch.equal(back, x)
