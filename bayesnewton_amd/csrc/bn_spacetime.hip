@@ -11,13 +11,20 @@
 //   k_st_sites        block per (step, run): posterior -> data (basemodels.py:743-764), site
 //                     update (inference.py:65-90, 105-195) or energy terms, and the projected
 //                     pseudo observation in whitened form: W = B' diag(nat2) B + 1e-12 I = L L',
-//                     z = L^-1 B' nat1 (basemodels.py:676-687 without forming W^-1)
-//   k_st_filter       block per run, loop over T: predict, measurement update with
-//                     U = P-[:, :M] L, Mm = I + L' Sh L (inverted in LDS by the sweep operator),
-//                     q = z - L' H m-, m = m- + U Mm^-1 q, P = P- - U Mm^-1 U', log N terms.
+//                     z = L^-1 B' nat1 (basemodels.py:676-687 without forming W^-1), on register
+//                     tiles.  k_st_sites_ordered: the same with every sum in one fixed order,
+//                     for the mean-field filter and the EP update, which invert L L' explicitly
+//                     and so amplify a last place of it.
+//   k_st_transitions  A_t, Q_t of every step.
+//   k_st_filter       block per run, loop over T: predict, measurement update in whitened form
+//                     with Mm = I + L' Sh L = Lm Lm', W = U Lm^-T, P = P- - W W'.
 //                     Equal to ops.py:159-171 with noise (W + 1e-12 I)^-1.
-//   k_st_smoother     block per run, loop back over T: the RTS smoother of ops.py:288-311
-//                     (G' = P-^-1 A P with P-^-1 by an in-LDS sweep, P_s = P + G (P_s' - P-) G').
+//   k_st_ell          log likelihood terms of every step from what the filter leaves.
+//   k_st_gains        block per (step, run): the RTS map of a step (ops.py:288-311) as an affine
+//                     map of the next smoothed moments, by a blocked Cholesky of P-.
+//   k_st_smoother     the maps applied from the last step back: a walk over all steps of a run,
+//                     or, for few runs, chunks of steps composed, joined and walked side by side
+//                     (k_st_chain, k_st_terminal: the chunks' ends).
 //                     An adjoint (Bryson-Frazier) backward pass avoids the factorisation but
 //                     its covariance error grows geometrically over long runs with
 //                     precise sites, so the filtered moments are stored instead.
@@ -28,7 +35,8 @@
 //                     covariance, ops.py:429-706): per-run sequential filter with one M x M
 //                     inverse per step, the associative form as per-step M x M work plus a
 //                     scalar filter per (run, block) lane, and a per-lane RTS smoother.
-// Dense products are workgroup GEMMs on FP64 operands staged through LDS.
+// Dense products are FP64 matrix instructions on 16 x 16 tiles held in registers (bn_tile.h), in
+// the remaining kernels workgroup GEMMs on operands staged through LDS.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -47,7 +55,6 @@ constexpr int kT = 256;      // threads per workgroup
 constexpr int kMaxM = 64;    // inducing points per run
 constexpr int kMaxKT = 2;    // temporal state dim (Matern12 / Matern32)
 constexpr int kMaxD = kMaxKT * kMaxM;  // state dim
-static_assert(kT == 2 * kMaxD, "the smoother's mean update splits the workgroup in two halves of kMaxD");
 constexpr int kPK = 16;      // GEMM K-panel
 constexpr int kPS = 68;      // LDS panel row stride (doubles)
 constexpr double kPseudoJitter = 1e-12;  // basemodels.py:683
@@ -69,96 +76,9 @@ struct MatRef {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-// C = alpha A B + beta Cin (m x n, inner k; Cin may be C, neither may alias A or B) for
-// m, n > 64: 128 x 128 output tiles, wave w owns the 64 x 64 quadrant (rows (w/2)*64,
-// columns (w%2)*64) as 4 x 4 blocks of v_mfma_f64_16x16x4f64.  K panels of 8 go
-// through LDS (row stride 136 doubles: the four k rows a fragment read touches fall on
-// disjoint bank halves), the next panel is fetched into registers while the current
-// one is used.  `sm` holds 2 * 8 * 136 doubles.
-constexpr int kBPK = 8, kBLD = 136;
-static_assert(2 * kBPK * kBLD <= 2 * kPK * kPS, "wg_gemm_128 panels fit the wg_gemm panel space");
-__device__ __noinline__ void wg_gemm_128(int m, int n, int k, double alpha, MatRef A, MatRef B, double beta, const double* Cin,
-                            int64_t ldci, double* C, int64_t ldc, double* sm) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
-  __syncthreads();  // the caller's writes to the operands are complete
-  double* As = sm;                // [kBPK][kBLD]: As[kk][ii] = A(i0+ii, k0+kk)
-  double* Bs = sm + kBPK * kBLD;  // [kBPK][kBLD]: Bs[kk][jj] = B(k0+kk, j0+jj)
-  constexpr int NL = kBPK * 128 / kT;
-  for (int i0 = 0; i0 < m; i0 += 128) {
-    for (int j0 = 0; j0 < n; j0 += 128) {
-      f64x4 acc[4][4];
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = f64x4{0.0, 0.0, 0.0, 0.0};
-      // per-thread panel elements: A(i0 + ai[q], k0 + ak[q]), B(k0 + bk[q], j0 + bj[q])
-      int ai[NL], ak[NL], bk[NL], bjx[NL];
-#pragma unroll
-      for (int q = 0; q < NL; ++q) {
-        const int e = tid + q * kT;
-        if (A.cs == 1) { ai[q] = e >> 3; ak[q] = e & 7; } else { ak[q] = e >> 7; ai[q] = e & 127; }
-        if (B.cs == 1) { bk[q] = e >> 7; bjx[q] = e & 127; } else { bjx[q] = e >> 3; bk[q] = e & 7; }
-      }
-      double ra[NL], rb[NL];
-      auto fetch = [&](int k0) {
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-          const int gi = i0 + ai[q], gk = k0 + ak[q], gj = j0 + bjx[q], gk2 = k0 + bk[q];
-          ra[q] = (gi < m && gk < k) ? A.p[gi * A.rs + gk * A.cs] : 0.0;
-          rb[q] = (gj < n && gk2 < k) ? B.p[gk2 * B.rs + gj * B.cs] : 0.0;
-        }
-      };
-      fetch(0);
-#pragma unroll 1
-      for (int k0 = 0; k0 < k; k0 += kBPK) {
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-          As[ak[q] * kBLD + ai[q]] = ra[q];
-          Bs[bk[q] * kBLD + bjx[q]] = rb[q];
-        }
-        __syncthreads();
-        if (k0 + kBPK < k) fetch(k0 + kBPK);
-#pragma unroll
-        for (int kk = 0; kk < kBPK; kk += 4) {
-          double af[4], bf[4];
-#pragma unroll
-          for (int bi = 0; bi < 4; ++bi) af[bi] = As[(kk + (lane >> 4)) * kBLD + wr + bi * 16 + (lane & 15)];
-#pragma unroll
-          for (int bj = 0; bj < 4; ++bj) bf[bj] = Bs[(kk + (lane >> 4)) * kBLD + wc + bj * 16 + (lane & 15)];
-#pragma unroll
-          for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-              acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[bi], bf[bj], acc[bi][bj], 0, 0, 0);
-        }
-        __syncthreads();
-      }
-      // block (bi, bj), register r -> row wr + bi*16 + lane/16 + 4r, column wc + bj*16 + lane%16
-#pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int gi = i0 + wr + bi * 16 + (lane >> 4) + 4 * r;
-            const int gj = j0 + wc + bj * 16 + (lane & 15);
-            if (gi < m && gj < n) {
-              double v = alpha * acc[bi][bj][r];
-              if (beta != 0.0) v = fma(beta, Cin[gi * ldci + gj], v);
-              C[gi * ldc + gj] = v;
-            }
-          }
-    }
-  }
-  __syncthreads();
-}
-
 // C[i*ldc + j] = alpha * sum_k A(i,k) B(k,j) + beta * C[i*ldc + j], 0 <= i < m, 0 <= j < n.
 // The whole workgroup (kT threads = 4 waves) calls it; every 64x64 output block is
-// computed by FP64 matrix-core instructions, one 32x32 quadrant per wave
-// (wg_gemm dispatches m, n > 64 to wg_gemm_128).  Panels of A
+// computed by FP64 matrix-core instructions, one 32x32 quadrant per wave.  Panels of A
 // and B go through LDS (`sm`: 2 * kPK * kPS doubles); the next panel is fetched from
 // memory into registers while the current one is multiplied.
 // Operands and C may live in global memory or LDS; C must not alias A or B.
@@ -239,16 +159,6 @@ __device__ void wg_gemm_small(int m, int n, int k, double alpha, MatRef A, MatRe
     }
   }
   __syncthreads();
-}
-
-// Out-of-line entry for the filter and smoother: one call site per product keeps the
-// callers' register budgets free of the GEMM's accumulators.
-__device__ __noinline__ void wg_gemm(int m, int n, int k, double alpha, MatRef A, MatRef B, double beta, double* C,
-                                     int64_t ldc, double* sm) {
-  if (m > 64 && n > 64)
-    wg_gemm_128(m, n, k, alpha, A, B, beta, C, ldc, C, ldc, sm);
-  else
-    wg_gemm_small(m, n, k, alpha, A, B, beta, C, ldc, sm);
 }
 
 // In-place inverse of an n x n symmetric positive definite matrix a (LDS, stride ld) by
