@@ -35,3 +35,20 @@ def test_parallel_filter_at_the_rule_edges_equals_the_sequential_one(n):
     assert abs(float(a) - float(b)) <= 1e-9 * abs(float(b))
     assert float((am - bm).abs().max()) <= 1e-9 * float(bm.abs().max())
     assert float((aP - bP).abs().max()) <= 1e-9 * float(bP.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,runs", [(4095, 1), (4096, 1), (5000, 2)])
+@pytest.mark.parametrize("two", [False, True])
+def test_lengths_that_models_take(n, runs, two):
+    """One series under a sum keeps the default length (its gradient shows every rounding)."""
+    from bayesnewton_amd import kernels as K, likelihoods as L, models as M
+    k = K.Matern32(variance=1.0, lengthscale=1.0)
+    if two:
+        k = K.Sum([k, K.Matern52(variance=0.5, lengthscale=4.0)])
+    x = np.arange(n) * 0.1
+    lik = L.Gaussian(variance=0.01)
+    m = (M.MarkovVariationalGP(k, lik, x, np.sin(x)) if runs == 1
+         else M.MarkovVariationalGP.from_series(k, lik, [x] * runs, [np.sin(x)] * runs))
+    want = (default_chunk_len if two and runs == 1 else model_chunk_len)([n] * runs)
+    assert m.plan.chunk_len == want
