@@ -242,7 +242,12 @@ BN_HD void comp_step_col(double lam, double var, double ls, double dt, const dou
 // of a chunk are independent given the primal trajectory, which every lane recomputes.
 // HK is the column's class, fixed at compile time so that each instance carries only its
 // own source terms: -1 a unit tangent (no sources), 0 a lengthscale, 1 a variance
-// (h = 2 comp + HK).
+// (h = 2 comp + HK).  On the device `col` of a hyperparameter column is the same for every lane
+// of a wavefront, so the branches on the component are scalar ones: where lanes chose it, ROCm
+// 7.2 put register copies of the Matern32 + Matern52 instance, whose registers are all in use,
+// before the point where the lanes that had skipped a component come back.  Those lanes kept
+// what the registers held before, and the second lengthscale's derivative was wrong, and not
+// the same twice.
 template <int K1, int K2, int HK>
 BN_HD void lane_grad_col(const PlanView& pl, const HyperView& hv, const float* __restrict__ dt,
                          const float* __restrict__ y, const float* __restrict__ r, const uint8_t* __restrict__ mask,

@@ -273,27 +273,28 @@ __global__ __launch_bounds__(kBlock) void k_smoother_mbf(PlanView pl, HyperView 
 }
 
 // Two launches over the column classes of lane_grad_col: the NZ unit tangents (HK = -1)
-// and the NH hyperparameter tangents (HK = 2: each wave takes the lengthscale or the
-// variance instance, so both run in one launch and neither carries the other's terms).
+// and the NH hyperparameter tangents (HK = 2: each row of workgroups takes one column, with the
+// lengthscale or the variance instance, so both run in one launch and neither carries the
+// other's terms).
 template <int K1, int K2, int HK>
 __global__ __launch_bounds__(kBlock) void k_grad_chunk(PlanView pl, HyperView hv, const float* __restrict__ dt,
                                                        const float* __restrict__ y, const float* __restrict__ r,
                                                        const uint8_t* __restrict__ mask, CSoA fagg, CSoA fcarry,
                                                        GradOut out) {
-  // lane l -> column u = l / stride of the class, chunk l % stride: a wave covers
-  // consecutive chunks of one column
   using GD = GradDims<K1, K2>;
-  constexpr int NU = HK < 0 ? GD::NZ : (HK == 2 ? GD::NH : GD::NH / 2);
   const int64_t l = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int u = (int)(l / out.stride);
-  const int32_t j = (int32_t)(l - (int64_t)u * out.stride);
-  if (u >= NU || j >= pl.n_chunks) return;
   if constexpr (HK < 0) {
+    // lane l -> column u = l / stride, chunk l % stride: a wave covers consecutive chunks of
+    // one column
+    const int u = (int)(l / out.stride);
+    const int32_t j = (int32_t)(l - (int64_t)u * out.stride);
+    if (u >= GD::NZ || j >= pl.n_chunks) return;
     lane_grad_col<K1, K2, -1>(pl, hv, dt, y, r, mask, fagg, fcarry, out, j, u);
-  } else if ((u & 1) == 0) {  // column NZ + u: lengthscale for even u, variance for odd
-    lane_grad_col<K1, K2, 0>(pl, hv, dt, y, r, mask, fagg, fcarry, out, j, GD::NZ + u);
   } else {
-    lane_grad_col<K1, K2, 1>(pl, hv, dt, y, r, mask, fagg, fcarry, out, j, GD::NZ + u);
+    if (l >= pl.n_chunks) return;
+    const int u = (int)blockIdx.y;  // column NZ + u: lengthscale for even u, variance for odd
+    if ((u & 1) == 0) lane_grad_col<K1, K2, 0>(pl, hv, dt, y, r, mask, fagg, fcarry, out, (int32_t)l, GD::NZ + u);
+    else lane_grad_col<K1, K2, 1>(pl, hv, dt, y, r, mask, fagg, fcarry, out, (int32_t)l, GD::NZ + u);
   }
 }
 
@@ -988,8 +989,7 @@ int run_loglik_grad(const bn_plan* plan, HyperView hv, const float* dt, const fl
   constexpr int64_t NZ = GradDims<K1, K2>::NZ, NH = GradDims<K1, K2>::NH;
   hipLaunchKernelGGL((k_grad_chunk<K1, K2, -1>), dim3((unsigned)((NZ * p.n_chunks_pad + kBlock - 1) / kBlock)),
                      dim3(kBlock), 0, st, plan->view, hv, dt, y, r, mask, cs(b.fagg), cs(b.ftcarry), go);
-  hipLaunchKernelGGL((k_grad_chunk<K1, K2, 2>), dim3((unsigned)((NH * p.n_chunks_pad + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, st, plan->view, hv, dt, y, r, mask, cs(b.fagg), cs(b.ftcarry), go);
+  hipLaunchKernelGGL((k_grad_chunk<K1, K2, 2>), dim3(lane_grid(p).x, (unsigned)NH), dim3(kBlock), 0, st, plan->view, hv, dt, y, r, mask, cs(b.fagg), cs(b.ftcarry), go);
   constexpr int NT = GradDims<K1, K2>::NF <= 128 ? 128 : 256;
   int32_t max_nc = 1;
   for (int32_t v : p.series_nchunks) max_nc = std::max(max_nc, v);
