@@ -23,7 +23,7 @@ from . import cubature as cub
 from . import ops
 from . import spacetime
 from .kernels import SpatioTemporalKernel
-from .plan import SeriesPlan, default_chunk_len, model_chunk_len
+from .plan import SeriesPlan, model_chunk_len
 
 
 def input_admin(t, y):
@@ -126,12 +126,7 @@ class MarkovGaussianProcess:
         self._desc = kernel.desc()
         n_comp = self._desc.n_comp
         if chunk_len is None:
-            # For a sum, the energy's derivative in the smoother component's lengthscale is a
-            # difference of far larger numbers where steps are short against it (1,500 steps: 7 % of
-            # it are rounding, 100,000: all of it).  A last place anywhere in the pass shows there,
-            # so one series under a sum, which is what gets trained, keeps the length it had.
-            rule = default_chunk_len if n_comp > 1 and len(ts) == 1 else model_chunk_len
-            chunk_len = rule(lens, self.parallel)
+            chunk_len = model_chunk_len(lens, self.parallel)
         if ls is not None or var is not None:
             B = self.num_series
             base_ls, base_var = [c.lengthscale for c in kernel.components], [c.variance for c in kernel.components]

@@ -41,7 +41,7 @@ def test_parallel_filter_at_the_rule_edges_equals_the_sequential_one(n):
 @pytest.mark.parametrize("n,runs", [(4095, 1), (4096, 1), (5000, 2)])
 @pytest.mark.parametrize("two", [False, True])
 def test_lengths_that_models_take(n, runs, two):
-    """One series under a sum keeps the default length (its gradient shows every rounding)."""
+    """One rule for one series and for batches, under one component and under a sum."""
     from bayesnewton_amd import kernels as K, likelihoods as L, models as M
     k = K.Matern32(variance=1.0, lengthscale=1.0)
     if two:
@@ -50,5 +50,4 @@ def test_lengths_that_models_take(n, runs, two):
     lik = L.Gaussian(variance=0.01)
     m = (M.MarkovVariationalGP(k, lik, x, np.sin(x)) if runs == 1
          else M.MarkovVariationalGP.from_series(k, lik, [x] * runs, [np.sin(x)] * runs))
-    want = (default_chunk_len if two and runs == 1 else model_chunk_len)([n] * runs)
-    assert m.plan.chunk_len == want
+    assert m.plan.chunk_len == model_chunk_len([n] * runs)
