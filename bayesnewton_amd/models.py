@@ -23,7 +23,18 @@ from . import cubature as cub
 from . import ops
 from . import spacetime
 from .kernels import SpatioTemporalKernel
-from .plan import SeriesPlan, model_chunk_len
+from .plan import SeriesPlan, default_chunk_len, model_chunk_len
+
+
+# The energy's gradient takes a lane for each of the D (D + 3) / 2 unit tangents of every chunk.
+# Past this many lanes the chip is full, and a model whose own chunks are less than half the
+# default length runs its gradient on a plan of the default length instead: each chunk's start,
+# stored element and composition then cost more than its steps, and more than the two launches
+# that move the pseudo observations.  Own chunks of 8 steps -> the default 32 (MI355X, us a
+# gradient): D = 5, 105,000 steps 471 -> 539, 150,000 577 -> 553, 450,000 1395 -> 906; D = 4,
+# 150,000 321 -> 365, 225,000 422 -> 375.  Not below D = 4, whose elements are small: D = 3,
+# 300,000 steps in 5000 series 265 -> 302, 461,000 in 256 series 333 -> 356.
+GRAD_LANES = 350_000
 
 
 def input_admin(t, y):
@@ -125,7 +136,8 @@ class MarkovGaussianProcess:
         self.device = dev
         self._desc = kernel.desc()
         n_comp = self._desc.n_comp
-        if chunk_len is None:
+        own_chunks = chunk_len is None
+        if own_chunks:
             chunk_len = model_chunk_len(lens, self.parallel)
         if ls is not None or var is not None:
             B = self.num_series
@@ -167,8 +179,9 @@ class MarkovGaussianProcess:
         # sites N(0, 1e2) (basemodels.py:130-133): nat1 = 0, nat2 = 1e-2
         self._nat1 = torch.zeros(P.n_slots, dtype=torch.float64, device=dev)
         self._nat2 = torch.full((P.n_slots,), 1e-2, dtype=torch.float64, device=dev)
-        self._py = torch.empty(P.n_slots, dtype=torch.float32, device=dev)
-        self._pr = torch.empty(P.n_slots, dtype=torch.float32, device=dev)
+        self._pseudo = torch.empty((2, P.n_slots), dtype=torch.float32, device=dev)
+        self._py, self._pr = self._pseudo
+        self._grad_plan = None if own_chunks else P  # _grad_inputs
         nat.check(nat.lib().bn_site_reparametrise(P.handle, nat.ptr(self._nat1), nat.ptr(self._nat2),
                                                   nat.ptr(self._py), nat.ptr(self._pr), nat.stream_ptr()))
         self._pm = torch.zeros(P.n_slots, dtype=torch.float32, device=dev)
@@ -475,6 +488,27 @@ class MarkovGaussianProcess:
         for (o, a), v in zip(self._trainables(), np.asarray(raw, dtype=np.float64).reshape(-1)):
             setattr(o, a, float(v))
 
+    def _grad_inputs(self):
+        """Plan and tiled dt, pseudo observations, noise and mask that the gradient runs on
+        (GRAD_LANES).  The plan of the default length is made by the first gradient; one that
+        is captured before that, when a plan cannot be made, runs on the model's own."""
+        P, D = self.plan, self.kernel.state_dim
+        if self._grad_plan is None and not torch.cuda.is_current_stream_capturing():
+            longer = default_chunk_len(P.lengths)
+            if D > 3 and 2 * P.chunk_len < longer and D * (D + 3) // 2 * P.n_chunks > GRAD_LANES:
+                G = SeriesPlan(self.offsets, chunk_len=longer, device=self.device)
+                missing = torch.isnan(torch.as_tensor(self.Y[:, 0], device=self.device))
+                self._grad_fixed = G.gather(P.scatter(self._dt)), G.gather_mask(missing)
+                torch.cuda.current_stream().synchronize()  # later calls may come on other streams
+                self._grad_plan = G
+            else:
+                self._grad_plan = P
+        if self._grad_plan is None or self._grad_plan is P:
+            return P, self._dt, self._py, self._pr, self._mask
+        G, (dt, mask) = self._grad_plan, self._grad_fixed
+        py, pr = G.gather(P.scatter(self._pseudo), pad=1.0)
+        return G, dt, py, pr, mask
+
     def energy_and_grad_per_series(self, cubature=None):
         """Energy of every series and its gradient w.r.t. the natural-scale hypers
         with the sites and posterior held fixed (the gradient objax.GradValues(energy)
@@ -482,15 +516,16 @@ class MarkovGaussianProcess:
         P = self.plan
         ls, var = self._hypers()
         nh = 2 * self._desc.n_comp
+        G, dt, py, pr, mask = self._grad_inputs()
         gk = torch.empty((self.num_series, nh), dtype=torch.float64, device=self.device)
         gws = getattr(self, "_gws", None)
         if gws is None:
-            nbytes = int(nat.lib().bn_grad_workspace_bytes(P.handle, ctypes.byref(self._desc)))
+            nbytes = int(nat.lib().bn_grad_workspace_bytes(G.handle, ctypes.byref(self._desc)))
             gws = self._gws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=self.device)
         nat.check(nat.lib().bn_filter_loglik_grad(
-            P.handle, ctypes.byref(self._desc), nat.ptr(ls), nat.ptr(var), self._hyper_stride, nat.ptr(self._dt),
-            nat.ptr(self._py), nat.ptr(self._pr), nat.ptr(self._mask), nat.ptr(self._loglik), nat.ptr(gk),
-            nat.ptr(P.workspace(self._desc)), nat.ptr(gws), nat.stream_ptr()))
+            G.handle, ctypes.byref(self._desc), nat.ptr(ls), nat.ptr(var), self._hyper_stride, nat.ptr(dt), nat.ptr(py),
+            nat.ptr(pr), nat.ptr(mask), nat.ptr(self._loglik), nat.ptr(gk), nat.ptr(G.workspace(self._desc)),
+            nat.ptr(gws), nat.stream_ptr()))
         self._ll_key = self._state_key()
         E = self.energy_per_series(cubature)
         gl = torch.empty(self.num_series, dtype=torch.float64, device=self.device)
