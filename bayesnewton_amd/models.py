@@ -138,7 +138,7 @@ class MarkovGaussianProcess:
         n_comp = self._desc.n_comp
         own_chunks = chunk_len is None
         if own_chunks:
-            chunk_len = model_chunk_len(lens, self.parallel)
+            chunk_len = model_chunk_len(lens, self.parallel, kernel.state_dim)
         if ls is not None or var is not None:
             B = self.num_series
             base_ls, base_var = [c.lengthscale for c in kernel.components], [c.variance for c in kernel.components]

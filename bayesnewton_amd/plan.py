@@ -27,7 +27,7 @@ def default_chunk_len(lengths, parallel=True):
     return c
 
 
-def model_chunk_len(lengths, parallel=True):
+def model_chunk_len(lengths, parallel=True, state_dim=1):
     """Chunk length of a model's (or a single operation's) own plan.
 
     The lane-per-chunk kernels take about 1 us a step of the longest chunk and a few
@@ -35,9 +35,14 @@ def model_chunk_len(lengths, parallel=True):
     logarithm of their number.  Measured on MI355X (fused pass, chunk 32 -> this rule):
     10,000 steps 115 -> 66 us (Matern52) and 213 -> 147 us (Matern52 + Matern32), flat
     between 2 and 8; 200,000 steps 246 -> 206 us; 256 series with 276,000 steps
-    204 -> 163 us; 2000 series with 3.3 M steps 429 -> 378 us (8 steps a chunk would take
-    835 us: past about 60,000 chunks the chip is full, and short chunks only add scan
-    work); 4096 series with 15.7 M steps best at 123-128.
+    204 -> 163 us; past about 60,000 chunks the chip is full, and short chunks only add
+    scan work.
+    Longer chunks than the default 32 save scan work but leave the site kernels, which take
+    four lanes a chunk, fewer wavefronts: site update and pass of 4 M steps at 32 and 70 steps
+    a chunk 406 and 484 us (state dimension 1), 531 and 587 (3), 589 and 627 (4), 703 and 728
+    (5); of 8 M steps at 32 and 128 950 and 1005 (3), 1084 and 1060 (4), 1273 and 1216 (5); of
+    15.7 M 1754 and 1838 (3), 2015 and 1918 (4), 2397 and 2145 (5).  (The gradient alone would
+    take the longer ones a little sooner: 6016 and 5617 us at 4 M steps, state dimension 5.)
     Below 4096 steps in all the length stays 32, though 300 steps would take 47 us instead
     of 100: the float32 rows of the smoother are rounded from the chunk's end onwards, and in
     the energy of so few steps another length moves that rounding by as much as its whole
@@ -51,7 +56,9 @@ def model_chunk_len(lengths, parallel=True):
         return nmax
     if total < 4096:
         return 32
-    return max(8, -(-nmax // (128 * 128)), min(128, -(-total // 57344)))
+    if state_dim > 3 and total >= 128 * 57344:
+        return max(128, -(-nmax // (128 * 128)))
+    return max(8, -(-nmax // (128 * 128)), min(32, -(-total // 57344)))
 
 
 class SeriesPlan:

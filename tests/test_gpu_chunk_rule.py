@@ -20,6 +20,17 @@ def test_rule_bounds_each_series_to_its_scan(lengths):
     assert model_chunk_len(lengths, parallel=False) == default_chunk_len(lengths, parallel=False)
 
 
+@pytest.mark.parametrize("lengths,longer", [([2000] * 1000, False), ([2000] * 2000, False), ([2000] * 3670, False),
+                                            ([2000] * 3671, True), ([3840] * 4096, True)])
+def test_chunks_longer_than_the_default(lengths, longer):
+    """Only under a sum, from 128 * 57344 = 7,340,032 steps on: elsewhere they slow the site update."""
+    for d in (1, 2, 3):
+        assert model_chunk_len(lengths, state_dim=d) == 32
+    for d in (4, 5, 6):
+        assert model_chunk_len(lengths, state_dim=d) == (128 if longer else 32)
+    assert model_chunk_len([40_000_000], state_dim=5) == -(-40_000_000 // 16384)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 32, 33, 4095, 4096, 4097, 131073])
 def test_parallel_filter_at_the_rule_edges_equals_the_sequential_one(n):
