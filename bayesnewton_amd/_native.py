@@ -12,7 +12,7 @@ LIB_PATH = os.path.join(_HERE, "_lib", "libbn_hip.so")
 BN_MATERN12, BN_MATERN32, BN_MATERN52 = 1, 2, 3
 BN_RETURN_PREDICT = 0x1
 BN_RETURN_FULL = 0x2
-BN_NOALLOC_SCRATCH_BYTES = 64 * 1024 * 1024
+BN_NOALLOC_SCRATCH_BYTES = 96 * 1024 * 1024
 BN_STATUS_INNOVATION_NONPD, BN_STATUS_NONFINITE, BN_STATUS_SMOOTHER_NONPD = 1, 2, 4
 BN_SPARSE_UPDATE, BN_SPARSE_ENERGY = 0, 1
 

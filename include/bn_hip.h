@@ -163,8 +163,10 @@ int bn_filter_smoother(const bn_plan *plan, const bn_kernel_desc *kern, const do
  * that size is rejected with BN_EINVAL.  The call allocates nothing (the plan is
  * created beforehand with bn_plan_create) and records no timing events.  Calls
  * on one GPU share the array: calls that overlap on one GPU (other streams,
- * other host threads) race and must be serialised by the caller. */
-#define BN_NOALLOC_SCRATCH_BYTES (64u * 1024u * 1024u)
+ * other host threads) race and must be serialised by the caller.  The size holds
+ * the plans of models up to 284,000 steps at state dimension 5 and 8 steps a chunk
+ * (322 bytes a step), 390,000 at 4 and 578,000 at 3. */
+#define BN_NOALLOC_SCRATCH_BYTES (96u * 1024u * 1024u)
 int bn_filter_smoother_noalloc(const bn_plan *plan, const bn_kernel_desc *kern, const double *lengthscale,
                                const double *variance, int32_t hyper_stride, const float *dt, const float *y,
                                const float *r, const uint8_t *mask, float *post_mean, float *post_var,

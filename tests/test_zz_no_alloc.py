@@ -92,3 +92,29 @@ def test_noalloc_refuses_a_plan_beyond_its_scratch():
                                               nat.ptr(buf), nat.ptr(buf), nat.ptr(buf), None, nat.ptr(buf),
                                               nat.ptr(buf), nat.ptr(ll), None, nat.stream_ptr())
     assert rc == -1 and b"scratch" in nat.lib().bn_last_error()
+
+
+@pytest.mark.parametrize("names,runs,n", [(("Matern52", "Matern32"), 100, 2750), (("Matern52", "Matern52"), 100, 2090),
+                                          (("Matern32", "Matern32"), 100, 3850), (("Matern52",), 283, 2000),
+                                          (("Matern32",), 100, 9300)])
+def test_models_plans_fit_the_scratch(names, runs, n):
+    """The largest models whose pass needs at most 64 MiB at 32 steps a chunk: their own chunks
+    are shorter and need more, and still run without allocation."""
+    import torch
+    from bayesnewton_amd import _native as nat, kernels as K, likelihoods as L, models as M, ops
+    from bayesnewton_amd.plan import SeriesPlan, default_chunk_len
+    ks = [getattr(K, n)(variance=0.5, lengthscale=s) for n, s in zip(names, (5.0, 2.0))]
+    k = K.Sum(ks) if len(ks) > 1 else ks[0]
+    xs = [np.arange(n) * 0.1] * runs
+    m = M.MarkovVariationalGP.from_series(k, L.Gaussian(variance=0.01), xs, [np.sin(x) for x in xs])
+
+    def need(plan):
+        return int(nat.lib().bn_workspace_bytes(plan.handle, ctypes.byref(k.desc())))
+
+    assert 60 << 20 < need(SeriesPlan(m.offsets, chunk_len=default_chunk_len([n] * runs))) <= 64 << 20
+    m.update_posterior()
+    ls, var = m._hypers()
+    got = ops.filter_smoother(m.plan, k.desc(), ls, var, m._dt, m._py, m._pr, m._mask, noalloc=True)
+    for a, b in zip(got[:2], (m._pm, m._pv)):
+        assert torch.equal(m.plan.scatter(a), m.plan.scatter(b))
+    assert torch.equal(got[2], m._loglik)
