@@ -167,6 +167,8 @@ class SeriesPlan:
 
     def scatter_planes(self, t):
         """tiled float32 [w, n_slots] -> float64 [w, N]."""
+        if t.dtype != torch.float32:
+            raise TypeError(f"scatter_planes supports float32, got {t.dtype}")
         t = t.contiguous()
         out = torch.empty((t.shape[0], self.n_steps), dtype=torch.float64, device=self.device)
         nat.check(nat.lib().bn_plan_scatter_planes(self._h, nat.ptr(t), nat.ptr(out), t.shape[0], nat.stream_ptr()))

@@ -20,6 +20,13 @@ def test_planes_to_double_rows(lengths, chunk, w):
     assert torch.equal(out, x.double().t())
 
 
+def test_planes_of_other_types_are_refused():
+    plan = object.__new__(SeriesPlan)  # the check comes before any use of the plan
+    for dtype in (torch.float64, torch.float16, torch.int32):
+        with pytest.raises(TypeError):
+            plan.scatter_planes(torch.zeros(1, 8, dtype=dtype))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("lengths,chunk", [([1], 1), ([7], 100), ([70, 1, 33], 8), ([0, 5, 0], 4), ([300, 129, 2, 64], 3),
                                            ([513], 4), ([4000], 4000)])
