@@ -991,8 +991,7 @@ int run_loglik_grad(const bn_plan* plan, HyperView hv, const float* dt, const fl
                      dim3(kBlock), 0, st, plan->view, hv, dt, y, r, mask, cs(b.fagg), cs(b.ftcarry), go);
   hipLaunchKernelGGL((k_grad_chunk<K1, K2, 2>), dim3(lane_grid(p).x, (unsigned)NH), dim3(kBlock), 0, st, plan->view, hv, dt, y, r, mask, cs(b.fagg), cs(b.ftcarry), go);
   constexpr int NT = GradDims<K1, K2>::NF <= 128 ? 128 : 256;
-  int32_t max_nc = 1;
-  for (int32_t v : p.series_nchunks) max_nc = std::max(max_nc, v);
+  const int32_t max_nc = p.max_chunks;
   int32_t span = 1;  // chunks between consecutive elements of the current level
   while ((max_nc + span - 1) / span > kGradGroup) {
     const int32_t ne = (max_nc + span - 1) / span;

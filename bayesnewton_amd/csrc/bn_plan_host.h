@@ -15,6 +15,7 @@ static constexpr int kTile = 128;  // chunks per level-1 tile, and tiles per ser
 struct PlanHost {
   int32_t n_series = 0, n_chunks = 0, n_chunks_pad = 0, n_tiles = 0, chunk_len = 0, gshift = 6;
   int64_t n_slots = 0, n_steps = 0;
+  int32_t max_chunks = 0;   // of one series
   bool needs_scan = false;  // some series spans more than one chunk
   std::vector<int32_t> chunk_series, chunk_len_, chunk_tile, tile_first, tile_count, tile_series;
   std::vector<int32_t> series_first_tile, series_ntiles, series_first_chunk, series_nchunks;
@@ -120,13 +121,14 @@ inline bool build_plan(const int64_t* offsets, int32_t n_series, int32_t chunk_l
   // Empty series inside a batch are fine (no chunk, log-likelihood 0); a batch
   // with no step at all would launch empty grids, so it is refused here.
   if (p.n_chunks == 0) { err = "offsets describe no steps (every series is empty)"; return false; }
+  p.max_chunks = *std::max_element(p.series_nchunks.begin(), p.series_nchunks.end());
   set_lane_groups(p);
   p.n_steps = offsets[n_series];
   return true;
 }
 
 // The counts of one series' plan (its tables are closed forms of the chunk's number and are
-// written by a kernel); refuses what build_plan refuses.
+// written by a kernel: the host's stay empty); refuses what build_plan refuses.
 inline bool single_plan(int64_t n, int32_t chunk_len, PlanHost& p, std::string& err) {
   if (chunk_len < 1 || chunk_len > (1 << 24)) { err = "chunk_len must be in [1, 2^24]"; return false; }
   if (n < 0) { err = "offsets must be non-decreasing"; return false; }
@@ -139,7 +141,7 @@ inline bool single_plan(int64_t n, int32_t chunk_len, PlanHost& p, std::string& 
   p = PlanHost();
   p.n_series = 1;
   p.chunk_len = chunk_len;
-  p.n_chunks = (int32_t)nc;
+  p.n_chunks = p.max_chunks = (int32_t)nc;
   p.n_tiles = (int32_t)((nc + kTile - 1) / kTile);
   p.needs_scan = nc > 1;
   p.n_steps = n;

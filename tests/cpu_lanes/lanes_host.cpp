@@ -417,6 +417,18 @@ int main() {
       }
       check(wok, "wave_maxlen is the longest chunk of each 64 (chunk_len " + std::to_string(cl) + ")");
     }
+    // one series' plan without host tables has the counts of the plan with them
+    for (int64_t n : {1, 7, 64, 65, 128, 129, 513, 4097, 20000})
+      for (int32_t cl : {2, 3, 8, 64, 5000}) {
+        const int64_t one[2] = {0, n};
+        PlanHost a, b;
+        const bool ok = build_plan(one, 1, cl, a, err) && single_plan(n, cl, b, err);
+        check(ok && a.n_series == b.n_series && a.n_chunks == b.n_chunks && a.n_chunks_pad == b.n_chunks_pad &&
+                  a.n_tiles == b.n_tiles && a.chunk_len == b.chunk_len && a.gshift == b.gshift &&
+                  a.n_slots == b.n_slots && a.n_steps == b.n_steps && a.needs_scan == b.needs_scan &&
+                  a.max_chunks == a.series_nchunks[0] && b.max_chunks == a.max_chunks,
+              "counts of one series' plan (" + std::to_string(n) + " steps, chunk_len " + std::to_string(cl) + ")");
+      }
     // many short series pack eight tiles to a group, long ones one
     {
       std::vector<int64_t> o2(41, 0);

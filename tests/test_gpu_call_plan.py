@@ -41,6 +41,28 @@ def test_tables_equal_the_kept_plan(n, chunk):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,chunk", [(1, 1), (16, 1), (17, 1), (1000, 3), (4097, 2)])
+def test_gradient_composes_in_the_kept_plans_order(n, chunk):
+    """16 elements a level, whoever made the plan: the same bits."""
+    from bayesnewton_amd import kernels as K
+    dev = torch.device("cuda", torch.cuda.current_device())
+    rng = np.random.default_rng(n)
+    rows = [torch.as_tensor(a.astype(np.float32), device=dev)
+            for a in (rng.uniform(0.05, 0.5, n), rng.standard_normal(n), rng.uniform(0.05, 0.2, n))]
+    k, out = K.Matern32(variance=1.0, lengthscale=2.0), []
+    desc, (ls, var), L = k.desc(), k.hypers(dev), nat.lib()
+    for plan in (SeriesPlan(np.array([0, n], dtype=np.int64), chunk_len=chunk), SeriesPlan.for_call(n, chunk, dev)):
+        dt, y, r = (plan.gather(a, pad=1.0) for a in rows)
+        res = torch.zeros(3, dtype=torch.float64, device=dev)
+        gws = torch.empty(int(L.bn_grad_workspace_bytes(plan.handle, ctypes.byref(desc))), dtype=torch.uint8, device=dev)
+        nat.check(L.bn_filter_loglik_grad(plan.handle, ctypes.byref(desc), nat.ptr(ls), nat.ptr(var), 0, nat.ptr(dt),
+                                          nat.ptr(y), nat.ptr(r), None, nat.ptr(res), nat.ptr(res[1:]),
+                                          nat.ptr(plan.workspace(desc)), nat.ptr(gws), nat.stream_ptr()))
+        out.append(res.cpu())
+    assert torch.equal(*out) and bool(torch.isfinite(out[0]).all())
+
+
+@pytest.mark.gpu
 def test_calls_on_other_streams():
     from bayesnewton_amd import kernels as K, ops
     rng = np.random.default_rng(3)
