@@ -77,6 +77,30 @@ def test_filter_and_smoother_match_oracle(temporal, M, N, hetero, iters, warm):
         assert _rel(dc.cpu().numpy(), odc) < STATE_TOL
 
 
+@pytest.mark.parametrize("temporal", ["m12", "m32"])
+@pytest.mark.parametrize("M", [2, 15, 16, 17, 31, 32, 33, 36, 47, 48, 49, 63])
+def test_inducing_points_around_tiles(M, temporal):
+    """The Riccati and smoother iterations hold their matrices in 16-wide tiles, one to four a
+    side: every number of tiles, both state sizes, per-step and tied noise."""
+    from bayesnewton_amd import ops
+    gk, ok = _kernels(temporal, M, seed=M)
+    dt, y, R, Rt = _problem(M, M, 9)
+    dts = np.r_[dt[1:], 0.0]
+    for hetero, iters in ((True, 4), (False, 3)):
+        kw = dict(heteroscedastic=hetero, noise_cov_tied=Rt, dare_iters=iters)
+        ell, (fm, (Pd, cov)) = ops.kalman_filter_infinite_horizon(dt, gk, y, R, **kw)
+        oell, (ofm, (oPd, ocov)) = OP.kalman_filter_infinite_horizon(dt, ok, y, R, **kw)
+        assert abs(float(ell) - oell) <= LL_TOL * abs(oell)
+        for a, b in ((fm, ofm), (Pd, oPd), (cov, ocov)):
+            assert _rel(a.cpu().numpy(), b) < STATE_TOL
+        got = ops.rauch_tung_striebel_smoother_infinite_horizon(dts, gk, ofm, (oPd, ocov), return_full=True,
+                                                                dare_iters=iters)
+        want = OP.rauch_tung_striebel_smoother_infinite_horizon(dts, ok, ofm, (oPd, ocov), return_full=True,
+                                                                dare_iters=iters)
+        for a, b in zip(got, want):
+            assert a.shape == b.shape and _rel(a.cpu().numpy(), b) < STATE_TOL
+
+
 def _grid(g):
     gz = np.linspace(0, 1, g)
     a, b = np.meshgrid(gz, gz)
@@ -129,3 +153,25 @@ def test_infinite_horizon_model_matches_oracle(kind, lik, g, T, nr):
     Xf, Xs = gm.dare_solutions
     assert _rel(Xf.cpu().numpy(), om.dare_init_filter) < 1e-6
     assert _rel(Xs.cpu().numpy(), om.dare_init_smoother) < 1e-6
+
+
+def test_either_projection_gives_the_same_posterior():
+    """The model inverts L L' explicitly, on the projection whose sums do not keep one order.  Where
+    neighbouring inducing points are strongly correlated (64 of them, spatial lengthscale 0.8: the
+    condition of B' diag(nat2) B is about 1e6) that and the ordered projection may differ by the
+    rounding unit times a small part of the condition: 1e-10, a tenth of what the mean-field form
+    shows there."""
+    from bayesnewton_amd import kernels as K, likelihoods as L, spacetime as S
+    t, r, y = _st_data(8, 12, 256, "poisson")
+    out = []
+    for whitened in (True, False):
+        class Model(S.SpaceTimeVariationalInfiniteHorizonGP):
+            _whitened = whitened
+        k = K.SpatioTemporalKernel(K.Matern32(variance=1.0, lengthscale=10.0), K.Matern32(variance=1.0, lengthscale=0.8),
+                                   z=_grid(8))
+        m = Model.from_runs(k, L.Poisson(binsize=2.0), [t], [r], [y])
+        for _ in range(3):
+            m.inference(lr=0.3)
+        out.append([a.cpu().numpy() for a in (m.posterior_mean, m.posterior_variance, m.energy_per_run())])
+    for a, b in zip(*out):
+        assert _rel(a, b) < 1e-10

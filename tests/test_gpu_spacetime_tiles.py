@@ -87,3 +87,54 @@ def test_many_runs_in_blocks_of_steps():
         out.append((m.posterior_mean[-2:].cpu().numpy(), m.posterior_variance[-2:].cpu().numpy()))
     for x, w in zip(*out):
         assert np.max(np.abs(x - w)) <= 1e-10 * np.max(np.abs(w))
+
+
+def test_blocks_of_several_chunks():
+    """One run of 2,700 steps at M = 64 goes back in two blocks of steps, two such runs in three,
+    every block in several chunks: the ends of blocks and chunks lie elsewhere, and only the
+    order of the covariance sums differs, 1e-10.  The first steps see all of them."""
+    from bayesnewton_amd import kernels as K, likelihoods as L, spacetime as S
+    g = np.linspace(0.0, 1.0, 8)
+    z = np.stack([a.ravel() for a in np.meshgrid(g, g)], 1)
+    rng = np.random.default_rng(6)
+    T, nr = 2700, 70
+    t = np.cumsum(rng.integers(1, 3, T)).astype(np.float64)
+    r = rng.uniform(size=(T, nr, 2)).astype(np.float32).astype(np.float64)
+    y = np.sin(4 * r[..., 0] + 0.05 * t[:, None]) + 0.3 * rng.standard_normal((T, nr))
+    out = []
+    for n in (1, 2):
+        kern = K.SpatioTemporalKernel(K.Matern32(variance=1.0, lengthscale=300.0),
+                                      K.Matern32(variance=1.0, lengthscale=0.25), z=z)
+        m = S.SpaceTimeVariationalGP.from_runs(kern, L.Gaussian(variance=0.09), [t] * n, [r] * n, [y] * n)
+        m.inference(lr=1.0, return_terms=False)
+        out.append([a.reshape(n, T, -1)[-1].cpu().numpy() for a in (m.posterior_mean, m.posterior_variance)])
+    for a, b in zip(*out):
+        for s in (slice(0, 60), slice(60, 120), slice(1200, 1500), slice(2500, 2700)):
+            assert np.max(np.abs(a[s] - b[s])) <= 1e-10 * np.max(np.abs(b[s]))
+
+
+@pytest.mark.parametrize("M", [9, 33])
+@pytest.mark.parametrize("noise", [1e-2, 1e-4, 1e-6])
+def test_equal_times_and_precise_observations(M, noise):
+    """Steps of length zero: the predicted covariance is the filtered one, as small as the noise
+    where the sites determine the field, and the gain is the identity.  The oracle agrees with
+    the dense posterior to 1e-15 / noise; the library has the same terms: 1e-8."""
+    from bayesnewton_amd import kernels as K, likelihoods as L, models as GM
+    g = np.linspace(0.0, 1.0, 8)
+    z = np.stack([a.ravel() for a in np.meshgrid(g, g)], 1)[:M]
+    rng = np.random.default_rng(3)
+    t = np.array([0.0, 0.0, 1.0, 1.0, 1.0, 2.0, 5.0, 5.0, 6.0])
+    T, nr = len(t), 4 * M + 3
+    r = rng.uniform(size=(T, nr, 2)).astype(np.float32).astype(np.float64)
+    f = np.sin(0.3 * t)[:, None] + np.cos(3.0 * r[..., 0]) * np.sin(2.0 * r[..., 1])
+    y = (f + np.sqrt(noise) * rng.standard_normal((T, nr))).astype(np.float32).astype(np.float64)
+    gk = K.SpatioTemporalKernel(K.Matern32(variance=1.2, lengthscale=6.0), K.Matern32(variance=0.9, lengthscale=0.25), z=z)
+    ok = OK.SpatioTemporalKernel(OK.Matern32(1.2, 6.0), OK.Matern32(0.9, 0.25), z, sparse=True, conditional="Full")
+    gm = GM.MarkovVariationalGP(gk, L.Gaussian(variance=noise), t, y, R=r)
+    om = OM.MarkovGP(ok, OL.Gaussian(noise), t[:, None], y, R=r, inference="VI")
+    for m in (gm, om):
+        m.inference(lr=1.0)
+    for got, want in ((gm.posterior_mean, om.posterior_mean), (gm.posterior_variance, om.posterior_variance)):
+        got, want = got.cpu().numpy(), np.asarray(want)
+        assert np.max(np.abs(got - want)) <= 1e-8 * np.max(np.abs(want))
+    assert abs(float(gm.energy()) - om.energy()) <= 1e-8 * abs(om.energy())
