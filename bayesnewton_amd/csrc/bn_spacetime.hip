@@ -13,8 +13,8 @@
 //                     pseudo observation in whitened form: W = B' diag(nat2) B + 1e-12 I = L L',
 //                     z = L^-1 B' nat1 (basemodels.py:676-687 without forming W^-1), on register
 //                     tiles.  k_st_sites_ordered: the same with every sum in one fixed order,
-//                     for the mean-field filter and the EP update, which invert L L' explicitly
-//                     and so amplify a last place of it.
+//                     for the mean-field filter and the EP update, whose results multiply a
+//                     last place of L L' by its condition.
 //   k_st_transitions  A_t, Q_t of every step.
 //   k_st_filter       block per run, loop over T: predict, measurement update in whitened form
 //                     with Mm = I + L' Sh L = Lm Lm', W = U Lm^-T, P = P- - W W'.
@@ -425,8 +425,10 @@ static_assert(2 * kRC * kLC >= kMaxM * kMaxM, "the two chunk buffers hold an M x
 // condition of W (1e6 and more on a grid of 64 inducing points), so W is summed over the
 // locations in their order and factored pivot by pivot, whatever the number of wavefronts.
 // k_st_sites is faster (1.09 -> 0.45 ms at 4 runs of 500 steps, M = 64, R = 256) but rounds
-// differently in the last place, which moved mean-field posteriors by 1e-9 to 5e-9 (dense and
-// infinite-horizon ones by 1e-14 to 4e-13).
+// differently in the last place, which moved mean-field posteriors by 1e-9 to 5e-9.  Dense ones
+// moved by 1e-14, infinite-horizon ones, which invert L L' too, by 2e-14 to 4e-13 (conditions of
+// 3e3 to 7e5); against 80-bit arithmetic their errors are the same on both kernels, 7e-15 at a
+// condition of 2e3, 3e-10 at 1e7, 1e-4 at 1e13.
 // KIND: the likelihood as a compile-time constant (0: the projection, which has none);
 // with only its branch compiled, the site step spills a fraction of what it does with
 // every likelihood's code in the kernel.
@@ -553,9 +555,11 @@ __device__ inline double row_sums4(const double (&x)[4], int l) {
 
 // A L^-T for a row tile A, into X (row stride ld) and returned: the product with the explicit
 // inverse I of the diagonal block, then one step of refinement with the block's factor L (row
-// stride kSLd).  Without it L L' would miss W by the condition of the diagonal blocks (16
-// neighbouring inducing points) times the rounding unit, which the mean-field form's explicit
-// inverse of L L' amplifies.
+// stride kSLd).  Without it L L' misses W by the condition of the diagonal blocks (16
+// neighbouring inducing points) times the rounding unit.  That matters where W is singular but
+// for its 1e-12: with 8 locations for 64 inducing points the remaining columns then lost their
+// positive pivots and the factor became NaN.  With four locations an inducing point L L', the
+// posteriors and the time (32 runs of 100 steps, 6.7 ms) are the same without it.
 __device__ inline tile4 solve_tile(double* X, int ld, const double* I, const double* L, tile4 A, int l) {
   double a[4];
   tile_store(X, ld, 0, 0, A, l);
@@ -686,10 +690,8 @@ __global__ __launch_bounds__(kT, 2) void k_st_sites(StDims dm, LikParams lik, GH
       const double mf = row_sums4(mq, l), vf = cd + row_sums4(vq, l);
       if (!in_batch || !mine) {
       } else if (UPDATE) {
-        // EP: (pm, pP) is the cavity of the inducing states, so (mf, vf) is the cavity at the data
-        SiteResult sr = METHOD == M_EP ? ep_site_from_cavity(lik, gh, yv, mf, vf, power, mask_pseudo != 0,
-                                                             ensure_psd != 0)
-                                       : site_step<METHOD>(lik, gh, yv, mf, vf, n1, n2, 1.0, ensure_psd != 0);
+        static_assert(!UPDATE || METHOD != M_EP, "the EP update goes through k_st_sites_ordered");
+        const SiteResult sr = site_step<METHOD>(lik, gh, yv, mf, vf, n1, n2, 1.0, ensure_psd != 0);
         acc0 += fabs(sr.nat1 - n1);
         acc1 += fabs(sr.nat2 - n2);
         n1 = (1.0 - lr) * n1 + lr * sr.nat1;
@@ -2045,9 +2047,13 @@ int gain_block_steps(const StDims& dm) {
   return (int)tb;
 }
 
-// Chunks per run of a block of nb steps: the number with the shortest chain, 2 ceil(nb / c) + c - 1
-// steps (compose, join, walk) against nb for one chunk, as long as the two workgroups a chunk
-// takes in the compose step run side by side for all runs.
+// Chunks per run of a block of nb steps.  Four launches follow each other: k_st_chain (one
+// product a step) and COMPOSE (two) over the steps of a chunk, JOIN over the chunks, WALK over
+// the steps again; 2 ceil(nb / c) + c - 1 steps of the walk stand for them, against nb for one
+// chunk.  Chunks are taken up to half as many as there are units, in all runs together: one run
+// of 1000 steps in 45 chunks 3.3 ms for the pass (90 ms in one), 32 runs of 100 steps in 4.
+// Whether more pay for 32 to 128 runs, where each launch then leaves units idle, has not been
+// measured.
 int smoother_chunks(const StDims& dm, int nb) {
   int best = 1, cost = nb;
   for (int c = 2; c <= nb && 2 * (int64_t)c * dm.K <= kUnits; ++c) {
