@@ -1855,7 +1855,8 @@ enum { ST_WALK = 0, ST_COMPOSE = 1, ST_JOIN = 2, ST_STEADY = 3 };
 // P_s = R + T G' (tiles j <= r; G in LDS, T through a staging tile): 51 k cycles of FP64 matrix
 // instructions a SIMD at D = 128, which bound it; the next step's G is on its way meanwhile.
 // 28 us a step, 35 with the outputs (89 us with both products through LDS panels of 8 columns);
-// one run of 1000 steps in 45 chunks: 3.3 ms for the whole pass, 90 ms walked as one chain.
+// one run of 1000 steps in 45 chunks: 3.3 ms for the whole pass (89 ms for those products walked
+// as one chain).
 template <int KT, int MB, int MODE>
 __global__ __launch_bounds__(64 * KT * MB, 2) void k_st_smoother(StDims dm, StSmootherIO io) {
   using S = StTiles<KT, MB>;
@@ -2049,11 +2050,11 @@ int gain_block_steps(const StDims& dm) {
 
 // Chunks per run of a block of nb steps.  Four launches follow each other: k_st_chain (one
 // product a step) and COMPOSE (two) over the steps of a chunk, JOIN over the chunks, WALK over
-// the steps again; 2 ceil(nb / c) + c - 1 steps of the walk stand for them, against nb for one
-// chunk.  Chunks are taken up to half as many as there are units, in all runs together: one run
-// of 1000 steps in 45 chunks 3.3 ms for the pass (90 ms in one), 32 runs of 100 steps in 4.
-// Whether more pay for 32 to 128 runs, where each launch then leaves units idle, has not been
-// measured.
+// the steps again.  2 ceil(nb / c) + c - 1 steps of the walk stand for them, against nb for one
+// chunk: at D = 128, 999 steps in 45 chunks, CHAIN and COMPOSE take 18 and 33 us a step, JOIN
+// 28 us a chunk, WALK 35 us a step, 3.2 ms in all (as one walk, 35 ms by that rate).  Chunks are taken up to
+// half as many as there are units, in all runs together; whether more pay for 32 to 128 runs,
+// where each launch then leaves units idle, has not been measured.
 int smoother_chunks(const StDims& dm, int nb) {
   int best = 1, cost = nb;
   for (int c = 2; c <= nb && 2 * (int64_t)c * dm.K <= kUnits; ++c) {
