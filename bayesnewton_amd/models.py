@@ -497,8 +497,7 @@ class MarkovGaussianProcess:
             longer = default_chunk_len(P.lengths)
             if D > 3 and 2 * P.chunk_len < longer and D * (D + 3) // 2 * P.n_chunks > GRAD_LANES:
                 G = SeriesPlan(self.offsets, chunk_len=longer, device=self.device)
-                missing = torch.isnan(torch.as_tensor(self.Y[:, 0], device=self.device))
-                self._grad_fixed = G.gather(P.scatter(self._dt)), G.gather_mask(missing)
+                self._grad_fixed = G.gather(P.scatter(self._dt)), G.gather_mask(torch.isnan(P.scatter(self._y)))
                 torch.cuda.current_stream().synchronize()  # later calls may come on other streams
                 self._grad_plan = G
             else:
